@@ -493,25 +493,41 @@ __global__ void __launch_bounds__(256) conv_update1_kernel(const ConvUpdateParam
 }
 
 // ---- Time-contiguous fast path ------------------------------------------------
-// For x, out, dout and dx with unit time stride, rows aligned to 4 elements and
-// seqlen a multiple of VT: each thread owns VT consecutive steps of one
-// (batch, channel) row (VT = 16 where seqlen allows, else 8) with 16-byte
-// (fp32) or 8-byte (16-bit) vector loads and stores; the W-1 inputs before its first step (and,
+// For x, out, dout and dx with unit time stride: each thread owns VT
+// consecutive steps of one (batch, channel) row with 16-byte (fp32) or 8-byte
+// (16-bit) vector loads and stores; the W-1 inputs before its first step (and,
 // in the backward, the W-1 steps after its last) are re-read from the
 // neighbouring thread's vector, which the cache serves. A workgroup covers
 // `rpw` rows of `tpr` threads each (short rows) or one 256 * VT-step segment of
-// a row (long rows), so a row segment never straddles a wave.
+// a row (long rows). Two forms:
+//   - aligned rows (RAG false): rows start on 4-element boundaries, seqlen is a
+//     multiple of VT and a row is whole waves, so the row and everything
+//     derived from it stay in the scalar unit;
+//   - any rows (RAG true): rows start anywhere (the vectors then carry only
+//     their element's alignment, which gfx950 takes), the last thread of a row
+//     moves what is left of it one element at a time, and tpr goes down to 4, so
+//     that rows of a few steps still fill their waves. Packed sequences (SEQ)
+//     run here too: a thread holds its steps' ids beside their inputs.
+// HBM bounds both. At batch 4, dim 1536, seqlen 1021 (float32, width 4, silu)
+// forward and backward take 10.6 and 17.6 us; the chunked kernels, whose lanes
+// load one element at a time 32 bytes apart, took 36.4 and 70.1 us.
 
-template <typename T>
+// A vector of 16-byte (fp32) or 8-byte (16-bit) width aligned to its element.
+typedef uint32_t u32x4_e4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u32x2_e2 __attribute__((ext_vector_type(2), aligned(2)));
+
+template <typename T, bool RAG = false>
 __device__ __forceinline__ void ld4(const void* base, int64_t idx, float* v) {
   if constexpr (sizeof(T) == 4) {
-    const float4 q = *reinterpret_cast<const float4*>(static_cast<const float*>(base) + idx);
-    v[0] = q.x;
-    v[1] = q.y;
-    v[2] = q.z;
-    v[3] = q.w;
+    using V = std::conditional_t<RAG, u32x4_e4, uint4>;
+    const V q = *reinterpret_cast<const V*>(static_cast<const float*>(base) + idx);
+    v[0] = __builtin_bit_cast(float, static_cast<uint32_t>(q.x));
+    v[1] = __builtin_bit_cast(float, static_cast<uint32_t>(q.y));
+    v[2] = __builtin_bit_cast(float, static_cast<uint32_t>(q.z));
+    v[3] = __builtin_bit_cast(float, static_cast<uint32_t>(q.w));
   } else {
-    const uint2 q = *reinterpret_cast<const uint2*>(static_cast<const T*>(base) + idx);
+    using V = std::conditional_t<RAG, u32x2_e2, uint2>;
+    const V q = *reinterpret_cast<const V*>(static_cast<const T*>(base) + idx);
     const uint32_t h[4] = {q.x & 0xffffu, q.x >> 16, q.y & 0xffffu, q.y >> 16};
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -521,18 +537,84 @@ __device__ __forceinline__ void ld4(const void* base, int64_t idx, float* v) {
   }
 }
 
-template <typename T>
+template <typename T, bool RAG = false>
 __device__ __forceinline__ void st4(void* base, int64_t idx, const float* v) {
   if constexpr (sizeof(T) == 4) {
-    *reinterpret_cast<float4*>(static_cast<float*>(base) + idx) = make_float4(v[0], v[1], v[2], v[3]);
-  } else if constexpr (std::is_same_v<T, bf16>) {
-    *reinterpret_cast<uint2*>(static_cast<T*>(base) + idx) =
-        make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+    if constexpr (RAG) {
+      const u32x4_e4 q = {__builtin_bit_cast(uint32_t, v[0]), __builtin_bit_cast(uint32_t, v[1]),
+                          __builtin_bit_cast(uint32_t, v[2]), __builtin_bit_cast(uint32_t, v[3])};
+      *reinterpret_cast<u32x4_e4*>(static_cast<float*>(base) + idx) = q;
+    } else {
+      *reinterpret_cast<float4*>(static_cast<float*>(base) + idx) = make_float4(v[0], v[1], v[2], v[3]);
+    }
   } else {
-    uint32_t h[4];
+    uint32_t lo, hi;
+    if constexpr (std::is_same_v<T, bf16>) {
+      lo = pack_bf16x2(v[0], v[1]);
+      hi = pack_bf16x2(v[2], v[3]);
+    } else {
+      uint32_t h[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) h[i] = __builtin_bit_cast(uint16_t, from_f32<T>(v[i]));
-    *reinterpret_cast<uint2*>(static_cast<T*>(base) + idx) = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
+      for (int i = 0; i < 4; ++i) h[i] = __builtin_bit_cast(uint16_t, from_f32<T>(v[i]));
+      lo = h[0] | (h[1] << 16);
+      hi = h[2] | (h[3] << 16);
+    }
+    if constexpr (RAG) {
+      const u32x2_e2 q = {lo, hi};
+      *reinterpret_cast<u32x2_e2*>(static_cast<T*>(base) + idx) = q;
+    } else {
+      *reinterpret_cast<uint2*>(static_cast<T*>(base) + idx) = make_uint2(lo, hi);
+    }
+  }
+}
+
+// v[0 .. N) = elements idx .. idx + N of base, those from `left` on zero (RAG;
+// without it all N exist). N is a multiple of 4.
+template <typename T, int N, bool RAG>
+__device__ __forceinline__ void ld_steps(const void* base, int64_t idx, int64_t left, float* v) {
+  if (!RAG || left >= N) {
+#pragma unroll
+    for (int q = 0; q < N; q += 4) ld4<T, RAG>(base, idx + q, v + q);
+  } else {
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] = i < left ? ld<T>(base, idx + i) : 0.f;
+  }
+}
+
+// The first `left` of v[0 .. N) (all of them without RAG) to base + idx.
+template <typename T, int N, bool RAG>
+__device__ __forceinline__ void st_steps(void* base, int64_t idx, int64_t left, const float* v) {
+  if (!RAG || left >= N) {
+#pragma unroll
+    for (int q = 0; q < N; q += 4) st4<T, RAG>(base, idx + q, v + q);
+  } else {
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+      if (i < left) st<T>(base, idx + i, v[i]);
+  }
+}
+
+// Sequence ids of steps s0 .. s0 + N of row b (SEQ), positions clamped to the
+// sequence: what lies outside reads zero inputs, or carries a zero gradient,
+// whatever its id.
+template <int N>
+__device__ __forceinline__ void conv_ids(const ConvParams& p, int64_t b, int64_t s0, int32_t (&id)[N]) {
+  const int32_t* ids = p.seq_idx + b * p.seqlen;
+  if (s0 >= 0 && s0 + N <= p.seqlen) {
+#pragma unroll
+    for (int i = 0; i < N; i += 4) {
+      const u32x4_e4 q = *reinterpret_cast<const u32x4_e4*>(ids + s0 + i);
+      id[i] = static_cast<int32_t>(q.x);
+      id[i + 1] = static_cast<int32_t>(q.y);
+      id[i + 2] = static_cast<int32_t>(q.z);
+      id[i + 3] = static_cast<int32_t>(q.w);
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const int64_t s = s0 + i;
+      id[i] = ids[s < 0 ? 0 : (s >= p.seqlen ? p.seqlen - 1 : s)];
+    }
   }
 }
 
@@ -549,18 +631,18 @@ struct ConvTile {
   bool active;    // the thread has steps to do
 };
 
-template <int VT>
+template <int VT, bool RAG>
 __device__ __forceinline__ ConvTile conv_tile(const ConvParams& p, int tid) {
   ConvTile g;
-  // A row segment is whole waves (tpr >= 64), so the row is wave-uniform and
-  // its (batch, channel) split stays in the scalar unit.
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int lt = tid & (p.tpr - 1), sub = (wave * 64) / p.tpr;
+  const int lt = tid & (p.tpr - 1);
   int64_t row;
   if (p.nseg > 1) {
     row = blockIdx.x / p.nseg;
     g.seg = blockIdx.x % p.nseg;
   } else {
+    // Without RAG a row segment is whole waves (tpr >= 64), so the row is
+    // wave-uniform and its (batch, channel) split stays in the scalar unit.
+    const int sub = RAG ? tid >> __builtin_ctz(p.tpr) : (__builtin_amdgcn_readfirstlane(tid >> 6) * 64) / p.tpr;
     row = static_cast<int64_t>(blockIdx.x) * p.rpw + sub;
     g.seg = 0;
   }
@@ -568,17 +650,24 @@ __device__ __forceinline__ ConvTile conv_tile(const ConvParams& p, int tid) {
   const int64_t rows = p.batch * p.dim;
   g.active = row < rows && g.t0 < p.seqlen;
   if (row >= rows) row = rows - 1;
-  g.c.b = row / p.dim;
-  g.c.d = row % p.dim;
+  if constexpr (RAG) {  // rows < 2^31: one 32-bit division per lane
+    const uint32_t r = static_cast<uint32_t>(row), dim = static_cast<uint32_t>(p.dim);
+    g.c.b = r / dim;
+    g.c.d = r % dim;
+  } else {
+    g.c.b = row / p.dim;
+    g.c.d = row % p.dim;
+  }
   g.c.r = 0;
   return g;
 }
 
-template <typename T, int W, int VT>
+template <typename T, int W, int VT, bool RAG, bool SEQ>
 __global__ void __launch_bounds__(256) conv_fwd_vt_kernel(const ConvParams p) {
-  const ConvTile g = conv_tile<VT>(p, threadIdx.x);
+  const ConvTile g = conv_tile<VT, RAG>(p, threadIdx.x);
   if (!g.active) return;
   const ConvRow& c = g.c;
+  const int64_t left = p.seqlen - g.t0;  // steps from this thread's first on
   float w[W];
 #pragma unroll
   for (int k = 0; k < W; ++k) w[k] = p.w[c.d * W + k];
@@ -586,24 +675,27 @@ __global__ void __launch_bounds__(256) conv_fwd_vt_kernel(const ConvParams p) {
   const int64_t xrow = c.b * p.sx[0] + c.d * p.sx[1];
   float xv[4 + VT];  // X[t0 - 4 .. t0 + VT)
   if (g.t0 > 0) {
-    ld4<T>(p.x, xrow + g.t0 - 4, xv);
+    ld4<T, RAG>(p.x, xrow + g.t0 - 4, xv);
   } else {
 #pragma unroll
     for (int i = 0; i < 4; ++i) xv[i] = conv_x<T>(p, c, i - 4);
   }
-#pragma unroll
-  for (int q = 0; q < VT; q += 4) ld4<T>(p.x, xrow + g.t0 + q, xv + 4 + q);
+  ld_steps<T, VT, RAG>(p.x, xrow + g.t0, left, xv + 4);
+  int32_t id[SEQ ? 4 + VT : 1];
+  if constexpr (SEQ) conv_ids(p, c.b, g.t0 - 4, id);
   float o[VT];
 #pragma unroll
   for (int i = 0; i < VT; ++i) {
     float acc = bias;
 #pragma unroll
-    for (int k = 0; k < W; ++k) acc = fmaf(w[k], xv[4 + i - (W - 1) + k], acc);
+    for (int k = 0; k < W; ++k) {
+      float xk = xv[4 + i - (W - 1) + k];
+      if constexpr (SEQ) xk = id[4 + i - (W - 1) + k] == id[4 + i] ? xk : 0.f;
+      acc = fmaf(w[k], xk, acc);
+    }
     o[i] = p.silu ? acc * sigmoid(acc) : acc;
   }
-  const int64_t orow = c.b * p.sout[0] + c.d * p.sout[1];
-#pragma unroll
-  for (int q = 0; q < VT; q += 4) st4<T>(p.out, orow + g.t0 + q, o + q);
+  st_steps<T, VT, RAG>(p.out, c.b * p.sout[0] + c.d * p.sout[1] + g.t0, left, o);
 }
 
 // Sum over the 64 lanes of a wave, in a fixed order, result in every lane.
@@ -613,12 +705,13 @@ __device__ __forceinline__ float wave_sum(float x) {
   return swap_sum<16>(x, x);
 }
 
-template <typename T, int W, int VT>
+template <typename T, int W, int VT, bool RAG, bool SEQ>
 __global__ void __launch_bounds__(256) conv_bwd_vt_kernel(const ConvParams p) {
-  __shared__ float s_part[4][W + 1];
-  const ConvTile g = conv_tile<VT>(p, threadIdx.x);
+  __shared__ float s_part[RAG ? 256 : 4][W + 1];
+  const ConvTile g = conv_tile<VT, RAG>(p, threadIdx.x);
   const ConvRow& c = g.c;
   const int64_t L = p.seqlen;
+  const int64_t left = L - g.t0;  // steps from this thread's first on
   float dwk[W + 1];  // dweight[0..W), dbias
 #pragma unroll
   for (int k = 0; k <= W; ++k) dwk[k] = 0.f;
@@ -631,17 +724,16 @@ __global__ void __launch_bounds__(256) conv_bwd_vt_kernel(const ConvParams p) {
 #pragma unroll
   for (int i = 0; i < VT + 4; ++i) go[i] = 0.f;
   if (g.active) {
-#pragma unroll
-    for (int q = 0; q < VT; q += 4) {
-      ld4<T>(p.x, xrow + g.t0 + q, xv + 4 + q);
-      ld4<T>(p.dout, orow + g.t0 + q, go + q);
-    }
+    ld_steps<T, VT, RAG>(p.x, xrow + g.t0, left, xv + 4);
+    ld_steps<T, VT, RAG>(p.dout, orow + g.t0, left, go);
   }
   // The halos are the neighbouring lanes' own steps: a wave's lanes hold
   // consecutive VT-step pieces of one row, so lane l's four steps before t0
   // are lane l - 1's last four and its four after are lane l + 1's first
   // four (every lane runs the shifts; inactive lanes hold zeros). Only the
-  // wave's end lanes read them from memory.
+  // wave's end lanes read them from memory. Where a wave holds several rows
+  // (RAG), a row's first lane takes its initial states below instead, and what
+  // its last lane receives lies past the sequence and is masked.
   const int lane = threadIdx.x & 63;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -654,30 +746,37 @@ __global__ void __launch_bounds__(256) conv_bwd_vt_kernel(const ConvParams p) {
 #pragma unroll
     for (int k = 0; k < W; ++k) w[k] = p.w[c.d * W + k];
     const float bias = p.bias ? p.bias[c.d] : 0.f;
-    const bool tail = g.t0 + VT < L;  // the next VT steps exist
+    const bool tail = left > VT;  // steps exist after this thread's
     if (g.t0 == 0) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) xv[i] = conv_x<T>(p, c, i - 4);
     } else if (lane == 0) {
-      ld4<T>(p.x, xrow + g.t0 - 4, xv);
+      ld4<T, RAG>(p.x, xrow + g.t0 - 4, xv);
     }
     if (tail && lane == 63) {
-      ld4<T>(p.x, xrow + g.t0 + VT, xv + 4 + VT);
-      ld4<T>(p.dout, orow + g.t0 + VT, go + VT);
+      ld_steps<T, 4, RAG>(p.x, xrow + g.t0 + VT, left - VT, xv + 4 + VT);
+      ld_steps<T, 4, RAG>(p.dout, orow + g.t0 + VT, left - VT, go + VT);
     }
+    int32_t id[SEQ ? 4 + VT + 4 : 1];  // sequence ids of the xv positions
+    if constexpr (SEQ) conv_ids(p, c.b, g.t0 - 4, id);
+    // Tap mask: the input at xv index a feeds the output at xv index o.
+    auto same = [&](int a, int o) { if constexpr (SEQ) return id[a] == id[o]; else return true; };
     // dpre[t0 + i] for i < VT + W - 1 (zero past the sequence end).
     float dp[VT + W - 1];
 #pragma unroll
     for (int i = 0; i < VT + W - 1; ++i) {
       float pre = bias;
 #pragma unroll
-      for (int k = 0; k < W; ++k) pre = fmaf(w[k], xv[4 + i - (W - 1) + k], pre);
+      for (int k = 0; k < W; ++k) {
+        const int a = 4 + i - (W - 1) + k;
+        pre = fmaf(w[k], same(a, 4 + i) ? xv[a] : 0.f, pre);
+      }
       float v = go[i];
       if (p.silu) {
         const float sg = sigmoid(pre);
         v *= sg * (1.f + pre * (1.f - sg));
       }
-      dp[i] = (i < VT || tail) ? v : 0.f;
+      dp[i] = (RAG ? i < left : i < VT || tail) ? v : 0.f;
     }
     float dx[VT];
     const int64_t fin0 = L - (W - 1);
@@ -685,17 +784,19 @@ __global__ void __launch_bounds__(256) conv_bwd_vt_kernel(const ConvParams p) {
     for (int i = 0; i < VT; ++i) {
       dwk[W] += dp[i];
 #pragma unroll
-      for (int k = 0; k < W; ++k) dwk[k] = fmaf(dp[i], xv[4 + i - (W - 1) + k], dwk[k]);
+      for (int k = 0; k < W; ++k) {
+        const int a = 4 + i - (W - 1) + k;
+        dwk[k] = fmaf(same(a, 4 + i) ? dp[i] : 0.f, xv[a], dwk[k]);
+      }
       float acc = 0.f;
 #pragma unroll
-      for (int k = 0; k < W; ++k) acc = fmaf(w[k], dp[i + (W - 1) - k], acc);
-      if (p.dfinal != nullptr && g.t0 + i >= fin0)
+      for (int k = 0; k < W; ++k)
+        acc = fmaf(w[k], same(4 + i, 4 + i + (W - 1) - k) ? dp[i + (W - 1) - k] : 0.f, acc);
+      if (p.dfinal != nullptr && g.t0 + i >= fin0 && (!RAG || i < left))
         acc += ld<T>(p.dfinal, (c.b * p.dim + c.d) * (W - 1) + (g.t0 + i - fin0));
       dx[i] = acc;
     }
-    const int64_t xr = c.b * p.sdx[0] + c.d * p.sdx[1];
-#pragma unroll
-    for (int q = 0; q < VT; q += 4) st4<T>(p.dx, xr + g.t0 + q, dx + q);
+    st_steps<T, VT, RAG>(p.dx, c.b * p.sdx[0] + c.d * p.sdx[1] + g.t0, left, dx);
     if (g.t0 == 0 && p.dinit != nullptr) {
       // dX[s] for s in [-(W-1), 0): the initial-state columns.
 #pragma unroll
@@ -708,19 +809,27 @@ __global__ void __launch_bounds__(256) conv_bwd_vt_kernel(const ConvParams p) {
       }
     }
   }
-  // Per-segment sums of dweight/dbias: wave sums, then the segment's waves in order.
-  const int wave = threadIdx.x >> 6;
+  // Per-segment sums of dweight/dbias. Whole waves: wave sums, then the
+  // segment's waves in order. Rows of less than a wave: every thread parks its
+  // terms and one thread per (row, tap) adds them in order.
+  const bool whole = !RAG || p.tpr >= 64;
+  if (whole) {
+    const int wave = threadIdx.x >> 6;
 #pragma unroll
-  for (int k = 0; k <= W; ++k) {
-    const float v = wave_sum(dwk[k]);
-    if ((threadIdx.x & 63) == 0) s_part[wave][k] = v;
+    for (int k = 0; k <= W; ++k) {
+      const float v = wave_sum(dwk[k]);
+      if ((threadIdx.x & 63) == 0) s_part[wave][k] = v;
+    }
+  } else {
+#pragma unroll
+    for (int k = 0; k <= W; ++k) s_part[threadIdx.x][k] = dwk[k];
   }
   __syncthreads();
-  const int wps = p.tpr / 64;  // waves per segment
-  if (threadIdx.x < p.rpw * (W + 1)) {
-    const int sg = threadIdx.x / (W + 1), k = threadIdx.x % (W + 1);
+  const int per = whole ? p.tpr / 64 : p.tpr;  // partial sums per segment
+  for (int e = threadIdx.x; e < p.rpw * (W + 1); e += 256) {
+    const int sg = e / (W + 1), k = e % (W + 1);
     float acc = 0.f;
-    for (int q = 0; q < wps; ++q) acc += s_part[sg * wps + q][k];
+    for (int q = 0; q < per; ++q) acc += s_part[sg * per + q][k];
     const int64_t row = p.nseg > 1 ? static_cast<int64_t>(blockIdx.x) / p.nseg
                                    : static_cast<int64_t>(blockIdx.x) * p.rpw + sg;
     if (row < p.batch * p.dim) {
@@ -1054,20 +1163,27 @@ static hipError_t launch_cl_dtype(const ConvParams& p, int dtype, bool bwd, hipS
   }
 }
 
+template <typename T, int W, int VT>
+static void launch_vt_width(const ConvParams& p, bool bwd, dim3 grid, hipStream_t st) {
+  const dim3 wg(256);
+  auto go = [&](auto rag, auto seq) {
+    if (bwd) hipLaunchKernelGGL((conv_bwd_vt_kernel<T, W, VT, rag.value, seq.value>), grid, wg, 0, st, p);
+    else hipLaunchKernelGGL((conv_fwd_vt_kernel<T, W, VT, rag.value, seq.value>), grid, wg, 0, st, p);
+  };
+  if (p.seq_idx != nullptr) go(std::true_type{}, std::true_type{});
+  else if (p.vt_any) go(std::true_type{}, std::false_type{});
+  else go(std::false_type{}, std::false_type{});
+}
+
 template <typename T>
 static hipError_t launch_vt(const ConvParams& p, bool bwd, hipStream_t st) {
-  const unsigned grid = static_cast<unsigned>(
-      p.nseg > 1 ? p.batch * p.dim * p.nseg : (p.batch * p.dim + p.rpw - 1) / p.rpw);
+  const dim3 grid(static_cast<unsigned>(
+      p.nseg > 1 ? p.batch * p.dim * p.nseg : (p.batch * p.dim + p.rpw - 1) / p.rpw));
   switch (p.width) {
-#define MCPU_CONV_VT(WW)                                                                             \
-  case WW:                                                                                           \
-    if (p.vt == 16) {                                                                                \
-      if (bwd) hipLaunchKernelGGL((conv_bwd_vt_kernel<T, WW, 16>), dim3(grid), dim3(256), 0, st, p);  \
-      else hipLaunchKernelGGL((conv_fwd_vt_kernel<T, WW, 16>), dim3(grid), dim3(256), 0, st, p);      \
-    } else {                                                                                         \
-      if (bwd) hipLaunchKernelGGL((conv_bwd_vt_kernel<T, WW, 8>), dim3(grid), dim3(256), 0, st, p);   \
-      else hipLaunchKernelGGL((conv_fwd_vt_kernel<T, WW, 8>), dim3(grid), dim3(256), 0, st, p);       \
-    }                                                                                                \
+#define MCPU_CONV_VT(WW)                                           \
+  case WW:                                                         \
+    if (sizeof(T) == 2 && p.vt == 16) launch_vt_width<T, WW, 16>(p, bwd, grid, st); \
+    else launch_vt_width<T, WW, 8>(p, bwd, grid, st);              \
     break;
     MCPU_CONV_VT(2)
     MCPU_CONV_VT(3)

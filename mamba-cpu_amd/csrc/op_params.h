@@ -36,9 +36,10 @@ struct ConvParams {
   const int32_t* seq_idx;  // (batch, seqlen) packed-sequence ids, or null
   int channels_last;  // thread index decomposed channel-fastest
   // Time-contiguous fast path (conv_*_vt_kernel): vt = steps per thread (8 or
-  // 16), 0 when the path does not apply.
-  int vt;
-  int tpr;            // threads per row segment: 64, 128 or 256
+  // 16), 0 when the path does not apply; vt_any: the form for rows of any
+  // length and alignment.
+  int vt, vt_any;
+  int tpr;            // threads per row segment: a power of two from 4 (vt_any) or 64 to 256
   int rpw;            // row segments per workgroup: 256 / tpr
   int64_t nseg;       // segments per row (rows longer than 2048 steps)
   // Channel-contiguous fast path (conv_*_cl_kernel): cl = 1 when it applies;

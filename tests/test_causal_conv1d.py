@@ -476,3 +476,43 @@ def test_wide_width_update_matches_oracle(seqlen):
         want, want_state = O.causal_conv1d_update(x, want_state, w, bias, "silu")
         close(out, want, 1e-5, 1e-5, f"out step {step}")
         close(state, want_state, 0, 0, f"state step {step}")
+
+
+@pytest.mark.parametrize("seqlen", [8, 9, 15, 16, 31, 33, 127, 129, 256, 511, 1021, 2049, 4099])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("kind", ["plain", "states", "packed"])
+def test_time_contiguous_rows_of_any_length(seqlen, dtype, kind):
+    """Rows that start and end off the vectors' boundaries (one to many
+    threads, waves and segments per row; 5 x 13 rows leave a workgroup partly
+    empty), in a buffer whose base is one element off, widths 2 to 5, with
+    initial and final states or packed sequences: forward and every gradient.
+    Bounds: float32 as above; 16-bit results carry one rounding, 2^-8 (bf16)
+    or 2^-11 (f16) of the value, of float32 arithmetic on the same inputs."""
+    width = 2 + seqlen % 4
+    torch.manual_seed(seqlen)
+    b, d = 5, 13
+    flat = torch.randn(b * d * seqlen + 1, device=DEV).to(dtype)
+    x = flat[1:].view(b, d, seqlen).requires_grad_()
+    w, bias = (torch.randn(d, width, device=DEV) * 0.5).requires_grad_(), torch.randn(d, device=DEV).requires_grad_()
+    g = torch.randn(b, d, seqlen, device=DEV).to(dtype)
+    kw = {}
+    if kind == "packed":
+        kw["seq_idx"] = torch.sort(torch.randint(0, 4, (b, seqlen), device=DEV, dtype=torch.int32), dim=1).values
+    init = gf = None
+    if kind == "states":
+        init = torch.randn(b, d, width - 1, device=DEV).to(dtype).requires_grad_()
+        gf = torch.randn(b, d, width - 1, device=DEV).to(dtype)
+        out, fin = causal_conv1d_fn(x, w, bias, initial_states=init, return_final_states=True, activation="silu")
+        grads = torch.autograd.grad([out, fin], [x, w, bias, init], [g, gf])
+    else:
+        out = causal_conv1d_fn(x, w, bias, activation="silu", **kw)
+        grads = torch.autograd.grad(out, [x, w, bias], g)
+    kw = {k: v.cpu().numpy() for k, v in kw.items()}
+    want, _ = O.causal_conv1d_fwd(x, w, bias, activation="silu", initial_states=init, **kw)
+    wg = O.causal_conv1d_bwd(x, w, bias, activation="silu", initial_states=init, dout=g, dfinal_states=gf, **kw)
+    tol = {torch.float32: 1e-5, torch.bfloat16: 2.0**-8, torch.float16: 2.0**-11}[dtype]
+    close(out, want, tol, 1e-5 if dtype == torch.float32 else 1e-3)
+    gtol = max(tol, 1e-4)
+    for name, got, ref in zip(("dx", "dw", "dbias", "dinit"), grads, wg):
+        scale = 1.0 if name in ("dx", "dinit") else max(1.0, float(np.abs(ref).max()))
+        close(got / scale, ref / scale, gtol, 1e-4 if dtype == torch.float32 else 1e-3, name)
