@@ -277,7 +277,7 @@ extern "C" int mcpu_selective_state_update(const mcpu_state_update_args* a, void
     return fail(MCPU_ERR_UNSUPPORTED, "selective_state_update: dstate must be in [1, 256]");
   if (a->ngroups < 1 || (a->nheads > 0 && a->nheads % a->ngroups != 0))
     return fail(MCPU_ERR_INVALID, "selective_state_update: nheads must be divisible by ngroups");
-  if (!valid_dtype(a->dtype) || !valid_dtype(a->state_dtype))
+  if (!valid_dtype(a->dtype) || !valid_dtype(a->state_dtype) || (a->bc_dtype != MCPU_F32 && a->bc_dtype != a->dtype))
     return fail(MCPU_ERR_INVALID, "selective_state_update: bad dtype");
   if (a->nheads * a->headdim > 0xffff0000ll)
     return fail(MCPU_ERR_UNSUPPORTED, "selective_state_update: nheads * headdim too large");
@@ -301,6 +301,7 @@ extern "C" int mcpu_selective_state_update(const mcpu_state_update_args* a, void
   p.headdim = a->headdim;
   p.dstate = a->dstate;
   p.ngroups = a->ngroups;
+  p.bc_dtype = a->bc_dtype;
   for (int i = 0; i < 3; ++i) {
     p.sst[i] = a->state_stride[i];
     p.sx[i] = a->x_stride[i];

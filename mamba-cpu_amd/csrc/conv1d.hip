@@ -512,59 +512,32 @@ __global__ void __launch_bounds__(256) conv_update1_kernel(const ConvUpdateParam
 // forward and backward take 10.6 and 17.6 us; the chunked kernels, whose lanes
 // load one element at a time 32 bytes apart, took 36.4 and 70.1 us.
 
-// A vector of 16-byte (fp32) or 8-byte (16-bit) width aligned to its element.
-typedef uint32_t u32x4_e4 __attribute__((ext_vector_type(4), aligned(4)));
-typedef uint32_t u32x2_e2 __attribute__((ext_vector_type(2), aligned(2)));
-
 template <typename T, bool RAG = false>
 __device__ __forceinline__ void ld4(const void* base, int64_t idx, float* v) {
-  if constexpr (sizeof(T) == 4) {
-    using V = std::conditional_t<RAG, u32x4_e4, uint4>;
-    const V q = *reinterpret_cast<const V*>(static_cast<const float*>(base) + idx);
-    v[0] = __builtin_bit_cast(float, static_cast<uint32_t>(q.x));
-    v[1] = __builtin_bit_cast(float, static_cast<uint32_t>(q.y));
-    v[2] = __builtin_bit_cast(float, static_cast<uint32_t>(q.z));
-    v[3] = __builtin_bit_cast(float, static_cast<uint32_t>(q.w));
+  if constexpr (RAG) {
+    ld4_elem<T>(base, idx, v);
+  } else if constexpr (sizeof(T) == 4) {
+    const float4 q = *reinterpret_cast<const float4*>(static_cast<const float*>(base) + idx);
+    v[0] = q.x;
+    v[1] = q.y;
+    v[2] = q.z;
+    v[3] = q.w;
   } else {
-    using V = std::conditional_t<RAG, u32x2_e2, uint2>;
-    const V q = *reinterpret_cast<const V*>(static_cast<const T*>(base) + idx);
-    const uint32_t h[4] = {q.x & 0xffffu, q.x >> 16, q.y & 0xffffu, q.y >> 16};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      if constexpr (std::is_same_v<T, bf16>) v[i] = to_f32(bf16{static_cast<uint16_t>(h[i])});
-      else v[i] = to_f32(__builtin_bit_cast(f16, static_cast<uint16_t>(h[i])));
-    }
+    const uint2 q = *reinterpret_cast<const uint2*>(static_cast<const T*>(base) + idx);
+    widen4<T>(q.x, q.y, v);
   }
 }
 
 template <typename T, bool RAG = false>
 __device__ __forceinline__ void st4(void* base, int64_t idx, const float* v) {
-  if constexpr (sizeof(T) == 4) {
-    if constexpr (RAG) {
-      const u32x4_e4 q = {__builtin_bit_cast(uint32_t, v[0]), __builtin_bit_cast(uint32_t, v[1]),
-                          __builtin_bit_cast(uint32_t, v[2]), __builtin_bit_cast(uint32_t, v[3])};
-      *reinterpret_cast<u32x4_e4*>(static_cast<float*>(base) + idx) = q;
-    } else {
-      *reinterpret_cast<float4*>(static_cast<float*>(base) + idx) = make_float4(v[0], v[1], v[2], v[3]);
-    }
+  if constexpr (RAG) {
+    st4_elem<T>(base, idx, v);
+  } else if constexpr (sizeof(T) == 4) {
+    *reinterpret_cast<float4*>(static_cast<float*>(base) + idx) = make_float4(v[0], v[1], v[2], v[3]);
   } else {
     uint32_t lo, hi;
-    if constexpr (std::is_same_v<T, bf16>) {
-      lo = pack_bf16x2(v[0], v[1]);
-      hi = pack_bf16x2(v[2], v[3]);
-    } else {
-      uint32_t h[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) h[i] = __builtin_bit_cast(uint16_t, from_f32<T>(v[i]));
-      lo = h[0] | (h[1] << 16);
-      hi = h[2] | (h[3] << 16);
-    }
-    if constexpr (RAG) {
-      const u32x2_e2 q = {lo, hi};
-      *reinterpret_cast<u32x2_e2*>(static_cast<T*>(base) + idx) = q;
-    } else {
-      *reinterpret_cast<uint2*>(static_cast<T*>(base) + idx) = make_uint2(lo, hi);
-    }
+    narrow4<T>(v, lo, hi);
+    *reinterpret_cast<uint2*>(static_cast<T*>(base) + idx) = make_uint2(lo, hi);
   }
 }
 

@@ -49,6 +49,56 @@ template <typename T> __device__ __forceinline__ void st(void* base, int64_t idx
   static_cast<T*>(base)[idx] = from_f32<T>(v);
 }
 
+// ---- four consecutive elements ------------------------------------------------------
+// 16-bit types: the elements of two dwords widened, and rounded back.
+template <typename T> __device__ __forceinline__ void widen4(uint32_t lo, uint32_t hi, float* v) {
+  const uint32_t h[4] = {lo & 0xffffu, lo >> 16, hi & 0xffffu, hi >> 16};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) v[i] = to_f32(__builtin_bit_cast(T, static_cast<uint16_t>(h[i])));
+}
+template <typename T> __device__ __forceinline__ void narrow4(const float* v, uint32_t& lo, uint32_t& hi) {
+  if constexpr (std::is_same_v<T, bf16>) {
+    lo = pack_bf16x2(v[0], v[1]);
+    hi = pack_bf16x2(v[2], v[3]);
+  } else {
+    uint32_t h[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) h[i] = __builtin_bit_cast(uint16_t, from_f32<T>(v[i]));
+    lo = h[0] | (h[1] << 16);
+    hi = h[2] | (h[3] << 16);
+  }
+}
+
+// A 16-byte (float32) or 8-byte (16-bit) vector aligned to its element only:
+// gfx950 moves it in one instruction at any element's address.
+typedef uint32_t u32x4_e4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u32x2_e2 __attribute__((ext_vector_type(2), aligned(2)));
+
+template <typename T> __device__ __forceinline__ void ld4_elem(const void* base, int64_t idx, float* v) {
+  if constexpr (sizeof(T) == 4) {
+    const u32x4_e4 q = *reinterpret_cast<const u32x4_e4*>(static_cast<const float*>(base) + idx);
+    v[0] = __builtin_bit_cast(float, static_cast<uint32_t>(q.x));
+    v[1] = __builtin_bit_cast(float, static_cast<uint32_t>(q.y));
+    v[2] = __builtin_bit_cast(float, static_cast<uint32_t>(q.z));
+    v[3] = __builtin_bit_cast(float, static_cast<uint32_t>(q.w));
+  } else {
+    const u32x2_e2 q = *reinterpret_cast<const u32x2_e2*>(static_cast<const T*>(base) + idx);
+    widen4<T>(q.x, q.y, v);
+  }
+}
+template <typename T> __device__ __forceinline__ void st4_elem(void* base, int64_t idx, const float* v) {
+  if constexpr (sizeof(T) == 4) {
+    const u32x4_e4 q = {__builtin_bit_cast(uint32_t, v[0]), __builtin_bit_cast(uint32_t, v[1]),
+                        __builtin_bit_cast(uint32_t, v[2]), __builtin_bit_cast(uint32_t, v[3])};
+    *reinterpret_cast<u32x4_e4*>(static_cast<float*>(base) + idx) = q;
+  } else {
+    uint32_t lo, hi;
+    narrow4<T>(v, lo, hi);
+    const u32x2_e2 q = {lo, hi};
+    *reinterpret_cast<u32x2_e2*>(static_cast<T*>(base) + idx) = q;
+  }
+}
+
 // ---- buffer loads ---------------------------------------------------------------
 // Loads through a raw buffer descriptor built from a wave-uniform base pointer
 // (scalar registers) and a 32-bit per-lane byte offset: the address

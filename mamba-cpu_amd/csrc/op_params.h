@@ -68,12 +68,13 @@ struct StateUpdateParams {
   const void* x;
   const void* dt;
   const float* A;
-  const float* B;
-  const float* C;
+  const void* B;
+  const void* C;
   const float* D;
   const void* z;
   const float* dt_bias;
   void* out;
+  int bc_dtype;              // storage type of B and C: float32 or x's
   int64_t batch, nheads, headdim, dstate, ngroups;
   int64_t sst[3], sx[3], sdt[3], sz[3], sB[2], sC[2];
   int64_t sA[3], sD[2], sbias[2];  // A over (head, headdim, dstate); D, dt_bias over (head, headdim)

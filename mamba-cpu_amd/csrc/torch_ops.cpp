@@ -972,8 +972,10 @@ Tensor selective_state_update(Tensor& state, const Tensor& x, const Tensor& dt, 
   const bool x_ok = heads ? (x.size(1) == h && x.size(2) == p) : x.size(1) == p;
   TORCH_CHECK_VALUE(x_ok && dt.sizes() == x.sizes() && (!has(z) || z->sizes() == x.sizes()), name,
                     " expects x, dt and z shaped like the state without dstate");
-  auto unit_last = [](const Tensor& t) {
-    const Tensor f = t.to(at::kFloat);
+  // B and C that share x's storage type are read as stored, others as float32.
+  const bool bc_stored = B_in.scalar_type() == x.scalar_type() && C_in.scalar_type() == x.scalar_type();
+  auto unit_last = [&](const Tensor& t) {
+    const Tensor f = bc_stored ? t : t.to(at::kFloat);
     return (f.stride(-1) == 1 || f.size(-1) == 1) ? f : f.contiguous();
   };
   // float32 parameters are read through their own strides (the Mamba-2 step
@@ -1004,8 +1006,9 @@ Tensor selective_state_update(Tensor& state, const Tensor& x, const Tensor& dt, 
   a.x = x.data_ptr();
   a.dt = dt.data_ptr();
   a.A = static_cast<const float*>(A.data_ptr());
-  a.B = static_cast<const float*>(B.data_ptr());
-  a.C = static_cast<const float*>(C.data_ptr());
+  a.B = B.data_ptr();
+  a.C = C.data_ptr();
+  a.bc_dtype = dtype_tag(B.scalar_type());
   a.D = fptr(D);
   a.z = ptr(z);
   a.dt_bias = fptr(dt_bias);

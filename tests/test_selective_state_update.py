@@ -139,3 +139,28 @@ def test_rejects_malformed_state_batch_indices():
                                torch.zeros(4, 2, device=DEV), torch.zeros(1, 2, device=DEV),
                                torch.zeros(1, 2, device=DEV),
                                state_batch_indices=torch.zeros(2, dtype=torch.int32, device=DEV))
+
+
+@pytest.mark.parametrize("n", [8, 16, 24, 32, 48, 64, 96, 100, 128, 200, 256])
+@pytest.mark.parametrize("sdt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("bcdt", [torch.float32, torch.bfloat16, torch.float16])
+def test_state_sizes_types_and_unaligned_views(n, sdt, bcdt):
+    """Every lane layout (vectors at 16, 32, 64, 128 and 256 states, one state
+    per lane otherwise) with B and C as stored, on views that start one element
+    into their buffers, a ragged number of rows, and A both full and expanded
+    from per-head values. Bounds: float32 as above (out sums up to 256 terms:
+    twice that); 16-bit values carry one rounding, at most 2^-8 of the value."""
+    torch.manual_seed(n)
+    b, h, p = 3, 2, 19
+    state = torch.randn(b * h * p * n + 1, device=DEV).to(sdt)[1:].view(b, h, p, n)
+    xdt = torch.float32 if sdt == torch.float32 else bcdt  # with a 16-bit state, B and C of x's type
+    x, dt, z = (f(b, h, p, device=DEV).to(xdt) for f in (torch.randn, torch.rand, torch.randn))
+    bc = torch.randn(b, 2 * n + 1, device=DEV).to(bcdt)
+    B, C = bc[:, 1:n + 1].unsqueeze(1), bc[:, n + 1:].unsqueeze(1)
+    D, dtb = torch.randn(h, p, device=DEV), torch.rand(h, p, device=DEV) * 0.1
+    for A in (-torch.rand(h, p, n, device=DEV) - 0.5, (-torch.rand(h, device=DEV))[:, None, None].expand(h, p, n)):
+        want, want_state = O.selective_state_update(state, x, dt, A, B, C, D, z, dtb, True)
+        out = selective_state_update(state, x, dt, A, B, C, D, z, dtb, True)
+        close(out, want, 2e-5 if xdt == torch.float32 else 2.0**-8, 2e-5, "out")
+        tol = 1e-5 if sdt == torch.float32 else 2.0**-8
+        close(state, want_state, tol, 1e-5, "state")
