@@ -48,22 +48,23 @@ int check_ssd(const mcpu_ssd_args* a) {
   return MCPU_OK;
 }
 
-// Heads per workgroup of the chunk kernels. Their LDS holds one workgroup
-// per CU, so a launch takes ceil(workgroups / CUs) rounds, each as long as one
-// workgroup: a part shared by its heads (staging B and C, forming C B^T) plus
-// a part per head, the shared part about 0.4 of a head's in both directions.
-// The divisor of the heads per group, up to kSsdMaxHeadBlock, with the least
-// rounds x (0.4 + heads) is chosen; against timings of both directions at
-// batch 1-8, 24-80 heads, seqlen 256-4096 this picks the fastest block or one
-// within 3 % of it.
-int head_block(const mcpu_ssd_args* a) {
+// Heads per workgroup of the chunk kernels. Their LDS holds one workgroup of
+// the backward's per CU and two of the forward's, so a launch takes
+// ceil(workgroups / slots) rounds, each as long as one workgroup: a part shared
+// by its heads (staging B and C, forming C B^T) plus a part per head, the shared
+// part about 0.4 of a head's in both directions. The divisor of the heads per
+// group, up to kSsdMaxHeadBlock, with the least rounds x (0.4 + heads) is
+// chosen; against timings of both directions at batch 1-8, 24-80 heads, seqlen
+// 256-4096 this picks the fastest block or one within 3 % of it.
+int head_block(const mcpu_ssd_args* a, bool bwd) {
   const int64_t hpg = a->nheads / a->ngroups;
   const int64_t chunks = a->batch * ((a->seqlen + kSsdQ - 1) / kSsdQ);
+  const int64_t slots = bwd ? kSsdCUs : 2 * kSsdCUs;
   int hb = 1;
   int64_t best = -1;
   for (int d = 1; d <= kSsdMaxHeadBlock; ++d) {
     if (hpg % d != 0) continue;
-    const int64_t rounds = (chunks * (a->nheads / d) + kSsdCUs - 1) / kSsdCUs;
+    const int64_t rounds = (chunks * (a->nheads / d) + slots - 1) / slots;
     const int64_t cost = rounds * (4 + 10 * d);
     if (best < 0 || cost < best) {
       best = cost;
@@ -108,7 +109,7 @@ SsdParams make_ssd(const mcpu_ssd_args* a, bool bwd = false) {
   p.in_order = in_order(a, bwd) ? 1 : 0;
   p.nslices = p.in_order ? (a->dstate + kSsdPassCols - 1) / kSsdPassCols
                          : (a->headdim * a->dstate + kSsdSlice - 1) / kSsdSlice;
-  p.hb = a->head_block != 0 ? a->head_block : head_block(a);
+  p.hb = a->head_block != 0 ? a->head_block : head_block(a, bwd);
   p.nhb = static_cast<int>(a->nheads / p.hb);
   p.softplus = a->dt_softplus != 0;
   p.dt_lo = a->dt_limit_lo;

@@ -28,12 +28,11 @@
 #include "mcpu_common.h"
 #include "scan_common.h"
 #include "ssd_params.h"
+#include "ssd_pieces.h"
 
 namespace mcpu {
 
 namespace {
-
-typedef float v4f __attribute__((ext_vector_type(4)));
 
 constexpr int Q = kSsdQ;
 constexpr int QP = Q + 4;          // padded row lengths of the LDS tiles (16-byte multiples)
@@ -212,6 +211,80 @@ __device__ __forceinline__ void tile_store_scaled(float* s, int ld, const raw4<T
   }
 }
 
+// How TPB threads move a tile of NC columns (64 or 128), of which the first
+// ncols exist, four elements at a time: NC / 4 threads to a row, so a thread
+// keeps its column and steps down the rows. EXACT: ncols = NC.
+template <int TPB, int NC, bool EXACT> struct TileMap {
+  static constexpr int step = TPB / (NC / 4);
+  int row, col;
+  bool on;   // the thread's column exists
+  __device__ __forceinline__ explicit TileMap(int ncols) {
+    row = static_cast<int>(threadIdx.x) / (NC / 4);
+    col = (static_cast<int>(threadIdx.x) % (NC / 4)) * 4;
+    on = EXACT || col < ncols;
+  }
+};
+
+// A lane's offset, kept apart from the uniform pointer it is added to: out of a
+// loop the compiler would carry their 64-bit sum per lane, one for each tensor
+// and entry, and spill.
+__device__ __forceinline__ uint32_t lane_offset(uint32_t off) {
+  asm volatile("" : "+v"(off));
+  return off;
+}
+
+// Entry k of a thread: row m.row + k m.step of src, row stride rs elements, with
+// nvalid rows. Every load is unconditional (what does not exist loads an
+// element that does, and map_park zeroes it), so that a tile's loads issue
+// together. Offsets from the uniform src are 32 bits: 64 rows of at most 65535
+// heads.
+template <typename Tx, int V, int TPB, int NC, bool EXACT>
+__device__ __forceinline__ void map_load(raw4<Tx> (&x)[V], const TileMap<TPB, NC, EXACT>& m, const Tx* src,
+                                         int64_t rs, int nvalid) {
+  static_assert(V * TPB * 4 == 64 * NC, "a thread's entries cover 64 rows");
+  const int col = m.on ? m.col : 0;
+#pragma unroll
+  for (int k = 0; k < V; ++k) {
+    const int r = m.row + k * m.step < nvalid ? m.row + k * m.step : nvalid - 1;
+    x[k] = ld_raw<Tx>(src + lane_offset(r * static_cast<uint32_t>(rs) + col));
+  }
+}
+
+// Those entries as bf16 pieces (ssd_pieces.h) in LDS tile s; rows from nvalid
+// on, and columns that do not exist, zero.
+template <typename Tx, int V, int TPB, int NC, bool EXACT>
+__device__ __forceinline__ void map_park(uint16_t* s, int ld, int plane, const TileMap<TPB, NC, EXACT>& m,
+                                         const raw4<Tx> (&x)[V], int nvalid) {
+  constexpr int NP = kPieces<Tx>;
+  uint16_t* at = s + m.row * ld + m.col;
+#pragma unroll
+  for (int k = 0; k < V; ++k) {
+    const raw4<Tx> v = m.on && m.row + k * m.step < nvalid ? x[k] : raw_zero<Tx>();
+    uint16_t* to = at + k * m.step * ld;
+    if constexpr (std::is_same_v<Tx, bf16>) {
+      *reinterpret_cast<uint2*>(to) = v;
+    } else {
+      const float4 f = widen<Tx>(v);
+      const float fv[4] = {f.x, f.y, f.z, f.w};
+      uint2 o[NP];
+      split4<NP>(fv, o);
+#pragma unroll
+      for (int i = 0; i < NP; ++i) *reinterpret_cast<uint2*>(to + i * plane) = o[i];
+    }
+  }
+}
+
+// Four elements of a row of pieces, summed.
+template <int NP> __device__ __forceinline__ float4 pieces4(const uint16_t* at, int plane) {
+  float4 f = widen<bf16>(*reinterpret_cast<const uint2*>(at));
+#pragma unroll
+  for (int i = 1; i < NP; ++i) {
+    const float4 g = widen<bf16>(*reinterpret_cast<const uint2*>(at + i * plane));
+    f = make_float4(f.x + g.x, f.y + g.y, f.z + g.z, f.w + g.w);
+  }
+  return f;
+}
+
 // tile_load then tile_store.
 template <typename Tx, int V, int TPB = kThreads>
 __device__ __forceinline__ void stage(float* s, int ld, const Tx* src, int64_t rs, int nrows, int nvalid, int ncols,
@@ -297,10 +370,11 @@ struct DyTiles {
 // each addition keeps its rounding error (Knuth's TwoSum) in lo, so a
 // difference (hi_t - hi_s) + (lo_t - lo_s) is accurate relative to itself
 // rather than to the size of the running sums.
-__device__ __forceinline__ void wave_prefix_sum2(float v, float& hi, float& lo) {
+// v comes as the pair v + vlo.
+__device__ __forceinline__ void wave_prefix_sum2(float v, float& hi, float& lo, float vlo = 0.f) {
   const int lane = threadIdx.x & 63;
   hi = v;
-  lo = 0.f;
+  lo = vlo;
 #pragma unroll
   for (int d = 1; d < 64; d <<= 1) {
     const float oh = __shfl_up(hi, d, 64), ol = __shfl_up(lo, d, 64);
@@ -328,6 +402,22 @@ __device__ __forceinline__ float wave_suffix_sum(float v) {
     if (lane + d < 64) v += o;
   }
   return v;
+}
+
+// a + b as a float pair: the sum, its rounding error added to lo (TwoSum).
+__device__ __forceinline__ float add2(float a, float b, float& lo) {
+  const float sum = a + b, bv = sum - a;
+  lo += (a - (sum - bv)) + (b - bv);
+  return sum;
+}
+
+// The same of pairs v + lo (wave_prefix_sum2), rounded once: the terms nearly
+// cancel over a chunk.
+__device__ __forceinline__ float wave_suffix_sum2(float v, float vlo) {
+  const int from = 63 - (threadIdx.x & 63);
+  float hi, lo;
+  wave_prefix_sum2(__shfl(v, from, 64), hi, lo, __shfl(vlo, from, 64));
+  return __shfl(hi + lo, 63 - (threadIdx.x & 63), 64);
 }
 
 // Sum over the 64 lanes of a wave, in a fixed order, in every lane.
@@ -621,149 +711,206 @@ __global__ void __launch_bounds__(kThreads, 3) ssd_state_scan_kernel(const SsdPa
 
 // F3: the chunk's outputs, Y = (C B^T o M) (dt x) + diag(exp(cs)) C H^T + D x,
 // out = Y silu(z) (and Y itself into ysave when the backward needs it).
-// Grid (nchunks, nhb, batch), 8 waves: wave w computes rows t in
-// [16 (w % 4), 16 (w % 4) + 16) and half w / 4 of the column tiles (C B^T:
-// tiles 2h, 2h + 1; Y: the first or second half of the headdim tiles), so each
-// SIMD runs two waves. C B^T is formed once for the block's heads.
-template <typename Tx, bool HAS_Z, bool SEQ>
-__global__ void __launch_bounds__(kThreads3, 2) ssd_chunk_scan_kernel(const SsdParams p) {
-  constexpr int TPB = kThreads3;
-  constexpr int VX = vec_x<TPB>(), VN = vec_n<TPB>();
-  __shared__ __align__(16) float s_C[Q][NP];
-  __shared__ __align__(16) float s_BH[Q][NP];     // B (Q x N), then each head's entering state H (P x N)
-  __shared__ __align__(16) float s_G[Q][QP];      // (C B^T o M)[t][s] dt_s, then Y
-  __shared__ __align__(16) float s_X[Q][XP];      // x
-  __shared__ float s_cs[Q], s_csl[Q], s_dt[Q];
-  __shared__ __align__(4) uint8_t s_first[Q];     // first step of each step's sequence run in the chunk
+// Grid (nchunks, nhb, batch), 8 waves: wave w computes rows t of strip w % 4
+// (16 rows), its half w / 4 taking steps s of [32 half, 32 half + 32) and states
+// of [64 half, 64 half + 64); the halves' Y are added where it is stored. Every
+// product runs on the bf16 matrix cores in pieces (ssd_pieces.h). A wave keeps
+// its part of C and of (C B^T)^T (rows s, columns t) in registers for the
+// block's heads, so G = C B^T o M dt is formed and split in the registers that
+// G x reads it from, and only x and H go through LDS, as pieces, staged once per
+// head. Tiles above the diagonal (s > t) are never formed.
+// What bounds it is memory: x, z and H in, out and y out. At
+// batch 4, seqlen 2048, 80 heads, bf16 with z it takes 137 us (4.9 TB/s) against
+// 308 us on the float32 matrix cores; batch 4, seqlen 1000, 24 heads, float32:
+// 32 against 48 us.
+// MN: 64 or 128, at least dstate. EXACT: headdim is 64 and dstate MN (128 in
+// every Mamba-2 model); otherwise tiles are filled up with zeros.
+template <typename Tx, bool HAS_Z, bool SEQ, int MN, bool EXACT>
+__global__ void __launch_bounds__(kThreads3, 4) ssd_chunk_scan_kernel(const SsdParams p) {
+  constexpr int TPB = kThreads3, NT = kSsdMaxP / 16;
+  constexpr int NX = kPieces<Tx>, NK = MN / 64;   // k-steps of a half over the states
+  constexpr int VX = vec_x<TPB>(), VN = Q * MN / 4 / TPB;
+  __shared__ __align__(16) uint16_t s_H[3 * kPlaneN];   // B (Q x N), then each head's entering state H (P x N), then Y
+  __shared__ __align__(16) uint16_t s_X[NX * kPlaneP];  // x
+  __shared__ __align__(16) float s_cs[Q], s_csl[Q], s_dt[Q], s_D[kSsdMaxP];
+  __shared__ uint8_t s_first[Q];                        // first step of each step's sequence run in the chunk
+  float* s_Y = reinterpret_cast<float*>(s_H);           // per half (Q x P), rows of XP floats
+  static_assert(2 * Q * XP * 4 <= sizeof(s_H), "Y fits over H");
+  // x and z load once the products are done where three pieces of C leave no
+  // registers for them before (spills: a reload waits for every load in flight).
+  constexpr bool kLate = NX == 3;
   const int64_t c = blockIdx.x, b = blockIdx.z;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int ws = wave & 3, hf = wave >> 2;        // row strip, column half
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int ws = wave & 3, hf = wave >> 2;        // row strip, half
   const int r = lane & 15, q = lane >> 4;
-  const int64_t L = p.seqlen, H = p.nheads, P = p.headdim, N = p.dstate, G = p.ngroups;
+  const int64_t L = p.seqlen, H = p.nheads, G = p.ngroups;
+  const int64_t P = EXACT ? kSsdMaxP : p.headdim, N = EXACT ? MN : p.dstate;
   const int64_t h0 = static_cast<int64_t>(blockIdx.y) * p.hb;
   const int64_t g = h0 / (H / G);
   const int64_t t0 = c * Q;
   const int nvalid = chunk_steps(p, t0);
   const int np = static_cast<int>(P / 16);
-  const int pa = (np + 1) / 2;
-  const int p0 = hf ? pa : 0, npw = hf ? np - pa : pa;   // this wave's headdim tiles
+  const TileMap<TPB, kSsdMaxP, EXACT> mp(static_cast<int>(P));
+  const TileMap<TPB, MN, EXACT> mn(static_cast<int>(N));
+  // C, rows t = 16 ws + r: operand fragments over this half's states
+  const int64_t bcoff = ((b * L + t0) * G + g) * N;
+  auto c_frag = [&](int k) {
+    const int t = 16 * ws + r, n = 32 * k + 8 * q;
+    return frag_mem<Tx>(static_cast<const Tx*>(p.C) + bcoff + t * G * N + n, t < nvalid && n < N);
+  };
+  Frag<NX> cf[NK];
+#pragma unroll
+  for (int k = 0; k < NK; ++k) cf[k] = c_frag(NK * hf + k);
   {
-    const int64_t off = ((b * L + t0) * G + g) * N;
-    stage<Tx, VN, TPB>(&s_C[0][0], NP, static_cast<const Tx*>(p.C) + off, G * N, Q, nvalid, static_cast<int>(N));
-    stage<Tx, VN, TPB>(&s_BH[0][0], NP, static_cast<const Tx*>(p.B) + off, G * N, Q, nvalid, static_cast<int>(N));
+    raw4<Tx> rb[VN];
+    map_load<Tx>(rb, mn, static_cast<const Tx*>(p.B) + bcoff, G * N, nvalid);
+    map_park<Tx>(s_H, kLdN, kPlaneN, mn, rb, nvalid);
   }
   if (SEQ && wave == 0) s_first[lane] = static_cast<uint8_t>(run_first<SEQ>(p, b, t0, lane));
   // the entering state reaches the chunk's first run
   const bool enter = seq_of<SEQ>(p, b, t0) == seq_of<SEQ>(p, b, t0 - 1);
-  __syncthreads();
-  // runs of this thread's rows t = 16 ws + 4 q + e: M[t][s] needs first_t <= s <= t
-  const uint32_t firsts = SEQ ? *reinterpret_cast<const uint32_t*>(&s_first[16 * ws + 4 * q]) : 0u;
-  v4f cb[2];
-  zero(cb);
-  mma(cb, 2, &s_C[16 * ws][0], NP, 1, &s_BH[32 * hf][0], 1, NP, static_cast<int>(N));
   // The next head's x tile, entering state and decays load into registers
   // while this head's products run.
   raw4<Tx> rx[VX], zc[VX];
-  float4 rh[VN], rD[VX];
-  float rcs = 0.f, rcsl = 0.f, rdt = 0.f;
-  // The headdim column of this thread's output entries (fixed over heads).
-  int ocol[VX];
-  {
-    const float inv = 1.0f / static_cast<float>(np * 4);
-#pragma unroll
-    for (int k = 0; k < VX; ++k) {
-      const int v = tid + k * TPB;
-      const int t = tile_row(v, inv);
-      ocol[k] = v < Q * np * 4 ? (v - t * np * 4) << 2 : 0;
-    }
-  }
+  float4 rh[VN];
+  float rcs = 0.f, rcsl = 0.f, rdt = 0.f, rD = 0.f;
   auto fetch = [&](int64_t h) {
     const int64_t row = chunk_row(p, b, h, c);
     if (tid < Q) {
-      rcs = p.cs[row + tid];
-      rcsl = p.cs_lo[row + tid];
-      rdt = p.step[row + tid];
+      const uint32_t at = lane_offset(tid);
+      rcs = (p.cs + row)[at];
+      rcsl = (p.cs_lo + row)[at];
+      rdt = (p.step + row)[at];
+      if (p.D && tid < P) rD = (p.D + h * P)[at];
     }
-    tile_load<Tx, VX, TPB>(rx, static_cast<const Tx*>(p.x) + ((b * L + t0) * H + h) * P, H * P, Q, nvalid,
-                           static_cast<int>(P));
-    tile_load<float, VN, TPB>(rh, p.states + state_block(p, b, c, h), N, static_cast<int>(P), static_cast<int>(P),
-                              static_cast<int>(N));
-#pragma unroll
-    for (int k = 0; k < VX; ++k)
-      rD[k] = p.D ? *reinterpret_cast<const float4*>(p.D + h * P + ocol[k]) : make_float4(0.f, 0.f, 0.f, 0.f);
+    map_load<float>(rh, mn, p.states + state_block(p, b, c, h), N, static_cast<int>(P));
+  };
+  auto fetch_x = [&](int64_t h) {
+    map_load<Tx>(rx, mp, static_cast<const Tx*>(p.x) + ((b * L + t0) * H + h) * P, H * P, nvalid);
   };
   fetch(h0);
-  for (int i = 0; i < p.hb; ++i) {
-    const int64_t h = h0 + i;
-    const int64_t xoff = ((b * L + t0) * H + h) * P;
-    float4 dcol[VX];  // this head's D at the output columns (rD moves on to the next head below)
+  fetch_x(h0);
+  __syncthreads();
+  // runs of this lane's step t = 16 ws + r (M[t][s] needs first_t <= s <= t)
+  // and of the rows t = 16 ws + 4 q + e it outputs
+  const int first_t = SEQ ? s_first[16 * ws + r] : 0;
+  bool from[4];
 #pragma unroll
-    for (int k = 0; k < VX; ++k) dcol[k] = rD[k];
-    __syncthreads();  // every wave is done with s_BH, s_G, s_X and s_cs
+  for (int e = 0; e < 4; ++e) from[e] = enter && (!SEQ || s_first[16 * ws + 4 * q + e] == 0);
+  // (C B^T)^T: rows s of tiles 2 hf and 2 hf + 1, columns t of this strip
+  v4f cb[2];
+  zero(cb);
+  for (int k = 0; k < 2 * NK; ++k) {
+    const Frag<NX> ck = c_frag(k);
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+      if (2 * hf + u <= ws)
+        cb[u] = mma32(frag_row<NX>(s_H + 16 * (2 * hf + u) * kLdN + 32 * k, kLdN, kPlaneN), ck, cb[u]);
+  }
+  for (int i = 0; i < p.hb; ++i) {
+    int64_t h = h0 + i;
+    asm volatile("" : "+s"(h));
+    const int64_t xoff = ((b * L + t0) * H + h) * P;
+    __syncthreads();  // every wave is done with s_H (B, Y), s_X and s_cs
     if (tid < Q) {
       s_cs[tid] = rcs;
       s_csl[tid] = rcsl;
       s_dt[tid] = rdt;
+      s_D[tid] = rD;
     }
-    tile_store<Tx, VX, TPB>(&s_X[0][0], XP, rx, Q, static_cast<int>(P));
-    tile_store<float, VN, TPB>(&s_BH[0][0], NP, rh, static_cast<int>(P), static_cast<int>(N));
+    map_park<Tx>(s_X, kLdP, kPlaneP, mp, rx, nvalid);
+    map_park<float>(s_H, kLdN, kPlaneN, mn, rh, static_cast<int>(P));
     __syncthreads();
-    if (HAS_Z)
-      tile_load<Tx, VX, TPB>(zc, static_cast<const Tx*>(p.z) + xoff, H * P, Q, nvalid, static_cast<int>(P));
-    if (i + 1 < p.hb) fetch(h + 1);
+    if (HAS_Z && !kLate) map_load<Tx>(zc, mp, static_cast<const Tx*>(p.z) + xoff, H * P, nvalid);
+    if (i + 1 < p.hb) {
+      fetch(h + 1);
+      if (!kLate) fetch_x(h + 1);
+    }
+    v4f y[NT];
+    zero(y);
+    // C H^T over this half's states
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int k = 0; k < NK; ++k)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int t = 16 * ws + 4 * q + e, s = 32 * hf + 16 * j + r;
-        const int ft = (firsts >> (8 * e)) & 0xff;
-        s_G[t][s] = (s <= t && s >= ft) ? cb[j][e] * seg_exp(s_cs, s_csl, t, s) * s_dt[s] : 0.f;
+      for (int j = 0; j < NT; ++j) {
+        if (EXACT || j < np)
+          y[j] = mma32(cf[k], frag_row<3>(s_H + 16 * j * kLdN + 32 * (NK * hf + k), kLdN, kPlaneN), y[j]);
+        if (NX == 3) __builtin_amdgcn_sched_barrier(0);  // one operand at a time: registers
       }
-    __syncthreads();
-    v4f y1[2], y2[2];
-    zero(y1);
-    zero(y2);
-    mma(y1, npw, &s_G[16 * ws][0], QP, 1, &s_X[0][16 * p0], XP, 1, Q);
-    mma(y2, npw, &s_C[16 * ws][0], NP, 1, &s_BH[16 * p0][0], 1, NP, static_cast<int>(N));
-    __syncthreads();  // every wave is done reading s_G
-    // Y (float32) into s_G, then out = (Y + D x) silu(z) four elements at a time.
+    float ecs[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const int t = 16 * ws + 4 * q + e;
-      const bool from = enter && ((firsts >> (8 * e)) & 0xff) == 0;
-      const float ecs = from ? fast_exp(s_cs[t] + s_csl[t]) : 0.f;
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-        if (j < npw) s_G[t][16 * (p0 + j) + r] = fmaf(ecs, y2[j][e], y1[j][e]);
+      const int te = 16 * ws + 4 * q + e;
+      ecs[e] = from[e] ? fast_exp(s_cs[te] + s_csl[te]) : 0.f;
     }
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) y[j][e] *= ecs[e];
+    // G x over this half's steps s
+    if (2 * hf <= ws) {
+      const int t = 16 * ws + r;
+      const float cst = s_cs[t], cslt = s_csl[t];
+      v4f gt[2];
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const int s0 = 32 * hf + 16 * u + 4 * q;
+        const float4 c4 = *reinterpret_cast<const float4*>(&s_cs[s0]);
+        const float4 l4 = *reinterpret_cast<const float4*>(&s_csl[s0]);
+        const float4 d4 = *reinterpret_cast<const float4*>(&s_dt[s0]);
+        const float cv[4] = {c4.x, c4.y, c4.z, c4.w}, lv[4] = {l4.x, l4.y, l4.z, l4.w},
+                    dv[4] = {d4.x, d4.y, d4.z, d4.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int sx = s0 + e;
+          const float m = cb[u][e] * fast_exp((cst - cv[e]) + (cslt - lv[e])) * dv[e];
+          gt[u][e] = (sx <= t && sx >= first_t) ? m : 0.f;
+        }
+      }
+      const Frag<3> ga = frag_acc<3>(gt[0], gt[1]);
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        if (EXACT || j < np) y[j] = mma32(ga, frag_col<NX>(s_X + 32 * hf * kLdP + 16 * j, kLdP, kPlaneP), y[j]);
+        if (NX == 3) __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    if constexpr (kLate) {
+      __builtin_amdgcn_sched_barrier(0);
+      if (HAS_Z) map_load<Tx>(zc, mp, static_cast<const Tx*>(p.z) + xoff, H * P, nvalid);
+      if (i + 1 < p.hb) fetch_x(h + 1);
+    }
+    __syncthreads();  // every wave is done reading s_H
+    // Y (float32) over H, then out = (Y + D x) silu(z) four elements at a time.
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+        if (EXACT || j < np) s_Y[(Q * hf + 16 * ws + 4 * q + e) * XP + 16 * j + r] = y[j][e];
     __syncthreads();
     {
-      const int nv = np * 4;
-      const float inv = 1.0f / static_cast<float>(nv);
 #pragma unroll
       for (int k = 0; k < VX; ++k) {
-        const int v = tid + k * TPB;
-        if (v >= Q * nv) continue;
-        const int t = tile_row(v, inv);
-        if (t >= nvalid) continue;
-        const int pp = (v - t * nv) << 2;
-        const int64_t at = xoff + t * H * P + pp;
-        float y[4] = {s_G[t][pp], s_G[t][pp + 1], s_G[t][pp + 2], s_G[t][pp + 3]};
+        const int to = mp.row + k * mp.step, pp = mp.col;
+        if (!mp.on || to >= nvalid) continue;
+        const uint32_t at = lane_offset(to * static_cast<uint32_t>(H * P) + pp);
+        const float4 ya = *reinterpret_cast<const float4*>(&s_Y[to * XP + pp]);
+        const float4 yb = *reinterpret_cast<const float4*>(&s_Y[(Q + to) * XP + pp]);
+        float o[4] = {ya.x + yb.x, ya.y + yb.y, ya.z + yb.z, ya.w + yb.w};
         if (p.D) {
-          const float4 d = dcol[k];
-          y[0] = fmaf(d.x, s_X[t][pp], y[0]);
-          y[1] = fmaf(d.y, s_X[t][pp + 1], y[1]);
-          y[2] = fmaf(d.z, s_X[t][pp + 2], y[2]);
-          y[3] = fmaf(d.w, s_X[t][pp + 3], y[3]);
+          const float4 d = *reinterpret_cast<const float4*>(&s_D[pp]), x4 = pieces4<NX>(s_X + to * kLdP + pp, kPlaneP);
+          o[0] = fmaf(d.x, x4.x, o[0]);
+          o[1] = fmaf(d.y, x4.y, o[1]);
+          o[2] = fmaf(d.z, x4.z, o[2]);
+          o[3] = fmaf(d.w, x4.w, o[3]);
         }
         if (HAS_Z) {
-          if (p.ysave) st4<Tx>(static_cast<Tx*>(p.ysave) + at, make_float4(y[0], y[1], y[2], y[3]));
+          if (p.ysave) st4<Tx>(static_cast<Tx*>(p.ysave) + xoff + at, make_float4(o[0], o[1], o[2], o[3]));
           const float4 z4 = widen<Tx>(zc[k]);
           const float zx[4] = {z4.x, z4.y, z4.z, z4.w};
 #pragma unroll
-          for (int u = 0; u < 4; ++u) y[u] *= zx[u] * sigmoid(zx[u]);
+          for (int u = 0; u < 4; ++u) o[u] *= zx[u] * sigmoid(zx[u]);
         }
-        st4<Tx>(static_cast<Tx*>(p.out) + at, make_float4(y[0], y[1], y[2], y[3]));
+        st4<Tx>(static_cast<Tx*>(p.out) + xoff + at, make_float4(o[0], o[1], o[2], o[3]));
       }
     }
   }
@@ -1317,6 +1464,432 @@ __global__ void __launch_bounds__(kThreads3, 2) ssd_bwd_chunk_kernel(const SsdPa
   }
 }
 
+// K3 for bf16 storage, headdim 64 and dstate 128 (every Mamba-2 model): the same
+// gradients with every product on the bf16 matrix cores in pieces
+// (ssd_pieces.h): x, B and C are one piece as stored; dY, G, dCB, dH^out and H
+// three. Waves 0-3 ("s") own 16 rows s each of d(dt x) and dB, waves 4-7 ("t")
+// 16 rows t of dC:
+//   - an s-wave forms C B^T and dG as (rows t, columns s), a t-wave as (rows s,
+//     columns t), each over its own 16 columns, so what it makes of them (G, dCB)
+//     is the operand of its next products where it stands, in registers, and
+//     neither goes through LDS; tiles above the diagonal are never formed;
+//   - products over rows of an LDS tile read it transposed (frag_col), so each
+//     tile is stored once.
+// dX = d(dt x), and its part W from the state, then pass through LDS once, where
+// all threads take c = <x, dX>, b = dt <x, W> (the sum over states of B (dt x)
+// dH^out) and dx, and one wave closes the chunk's decay gradients.
+// What bounds it: the LDS holds one workgroup per CU, so its phases (park, chunk
+// products, two state groups, output) run one after the other with two waves per
+// SIMD. Batch 4, seqlen 2048, 80 heads with z: 438 us against 971 us for the
+// float32 products below, whose matrix cores alone take 640.
+constexpr int kLdT = kSsdMaxN + 16;   // rows of B and C here, read mostly transposed: eight rows on 64 banks
+
+struct BwdChunkLds {
+  __align__(16) uint16_t C[Q * kLdT], B[Q * kLdT];
+  __align__(16) uint16_t X[kPlaneP], dY[3 * kPlaneP];
+  __align__(16) uint16_t st[6 * kPlaneP];   // dH^out, then H, of a 64-state group; then dX and W
+  __align__(16) float cs[Q], csl[Q], dt[Q], w[Q], ecs[Q];
+  float row[Q], col[Q], a[Q], b[Q], c[Q];
+  float dD[8][kSsdMaxP];
+  uint8_t first[Q], last[Q];                // ends of each step's sequence run in the chunk
+};
+
+// The waves of one kind, s (SW) or t: the head loop. Both kinds meet at the same
+// barriers, in the same order.
+template <bool HAS_Z, bool SEQ, bool SW>
+__device__ __forceinline__ void bwd_chunk_waves(const SsdParams& p, BwdChunkLds& lds) {
+  constexpr int TPB = kThreads3, P = kSsdMaxP, N = kSsdMaxN;
+  constexpr int VX = vec_x<TPB>();
+  constexpr bool sw = SW;
+  uint16_t (&s_X)[kPlaneP] = lds.X;
+  uint16_t (&s_dY)[3 * kPlaneP] = lds.dY;
+  float (&s_cs)[Q] = lds.cs;
+  float (&s_csl)[Q] = lds.csl;
+  float (&s_dt)[Q] = lds.dt;
+  float (&s_w)[Q] = lds.w;
+  float (&s_ecs)[Q] = lds.ecs;
+  uint16_t* const s_dH = lds.st;
+  uint16_t* const s_H = lds.st + 3 * kPlaneP;
+  float* const s_dX = reinterpret_cast<float*>(lds.st);    // rows of XP floats
+  float* const s_W = s_dX + Q * XP;
+  static_assert(2 * Q * XP * 4 <= sizeof(lds.st), "dX and W fit over the states");
+  const int64_t c = blockIdx.x, b = blockIdx.z;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int own = 16 * (wave & 3);                       // its strip's first row
+  const int r = lane & 15, q = lane >> 4;
+  const int64_t L = p.seqlen, H = p.nheads;
+  const int64_t h0 = static_cast<int64_t>(blockIdx.y) * p.hb;
+  const int64_t t0 = c * Q;
+  const int nvalid = chunk_steps(p, t0);
+  const TileMap<TPB, P, true> mp(P);
+  // The strip's own matrix and the other: B and C for an s-wave, C and B for a t-wave.
+  const uint16_t* const s_own = (sw ? lds.B : lds.C) + own * kLdT;
+  const uint16_t* const s_oth = sw ? lds.C : lds.B;
+  // C at this t-wave's dC elements, (rows t = own + 4 q + e, states 16 j + r), in pairs over j
+  uint32_t cd[4][4];
+  // Wave 4 (a t-wave: those have registers to spare) keeps the chunk's per-step
+  // values, lane t step t, and closes their gradients; wave 5 sums dD.
+  const bool keeper = !SW && wave == 4;
+  // Packed sequences: step `lane` reaches the chunk's end state (w) and reads the
+  // entering state (exp(cs)) only within one sequence.
+  bool reach = true, from = true;
+  if (keeper) {
+    if (SEQ) {
+      const bool starts = lane == 0 || seq_of<SEQ>(p, b, t0 + lane) != seq_of<SEQ>(p, b, t0 + lane - 1);
+      const unsigned long long begin = __ballot(starts);
+      const unsigned long long later = lane == 63 ? 0ull : begin & (~0ull << (lane + 1));
+      lds.first[lane] = static_cast<uint8_t>(run_first<SEQ>(p, b, t0, lane));
+      lds.last[lane] = static_cast<uint8_t>(later ? __builtin_ctzll(later) - 1 : Q - 1);
+    }
+    const int32_t id = seq_of<SEQ>(p, b, t0 + lane);
+    reach = id == seq_of<SEQ>(p, b, t0 + nvalid - 1);
+    from = id == seq_of<SEQ>(p, b, t0 - 1);
+  }
+  // The next head's tiles and decays, and the next states, load into registers
+  // while the current products run.
+  raw4<bf16> rx[VX], rgo[VX], rz[VX], ry[VX];
+  float4 su[VX], sv[VX];
+  float rcs = 0.f, rcsl = 0.f, rdt = 0.f, rpre = 0.f, rdl = 0.f;
+  auto fetch = [&](int64_t h) {
+    const int64_t row = chunk_row(p, b, h, c);
+    const int64_t xoff = ((b * L + t0) * H + h) * P;
+    if (keeper) {
+      const uint32_t at = lane_offset(lane);
+      rcs = (p.cs + row)[at];
+      rcsl = (p.cs_lo + row)[at];
+      rdt = (p.step + row)[at];
+      rpre = (p.dt + (b * L + t0) * H + h)[lane_offset((lane < nvalid ? lane : 0) * static_cast<uint32_t>(H))];
+      rdl = lane < p.nslices ? (p.dcsL + (row / Q) * p.nslices)[at] : 0.f;
+    }
+    map_load<bf16>(rx, mp, static_cast<const bf16*>(p.x) + xoff, H * P, nvalid);
+    map_load<bf16>(rgo, mp, static_cast<const bf16*>(p.dout) + xoff, H * P, nvalid);
+    if (HAS_Z) {
+      map_load<bf16>(rz, mp, static_cast<const bf16*>(p.z) + xoff, H * P, nvalid);
+      map_load<bf16>(ry, mp, static_cast<const bf16*>(p.ysave) + xoff, H * P, nvalid);
+    }
+  };
+  auto fetch_states = [&](int64_t h, int grp) {
+    const int64_t sb = state_block(p, b, c, h) + 64 * grp;
+    map_load<float>(su, mp, p.dstates + sb, N, P);
+    map_load<float>(sv, mp, p.states + sb, N, P);
+  };
+  auto park_states = [&]() {
+    map_park<float>(s_dH, kLdP, kPlaneP, mp, su, P);
+    map_park<float>(s_H, kLdP, kPlaneP, mp, sv, P);
+  };
+  fetch(h0);
+  fetch_states(h0, 0);
+  __syncthreads();
+  // The run bound of this lane's own step: t <= last_s for an s-wave's column s
+  // (with t >= s), s >= first_t for a t-wave's column t (with s <= t).
+  const int step_own = own + r;
+  const int bound = SEQ ? (sw ? lds.last[step_own] : lds.first[step_own]) : (sw ? Q - 1 : 0);
+  // C B^T: rows = the other's steps (tile u), columns = own steps
+  v4f cb[4];
+  zero(cb);
+#pragma unroll
+  for (int k = 0; k < N / 32; ++k) {
+    const Frag<1> o = frag_row<1>(s_own + 32 * k, kLdT, 0);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) cb[u] = mma32(frag_row<1>(s_oth + 16 * u * kLdT + 32 * k, kLdT, 0), o, cb[u]);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  if (!sw)
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const uint16_t* at = s_own + (4 * q + e) * kLdT + 32 * j + r;
+        cd[e][j] = static_cast<uint32_t>(at[0]) | (static_cast<uint32_t>(at[16]) << 16);
+      }
+  v4f acc[8];   // dB (s-wave) or dC (t-wave): rows own + 4 q + e, states 16 j + r
+  zero(acc);
+  for (int i = 0; i < p.hb; ++i) {
+    int64_t h = h0 + i;
+    asm volatile("" : "+s"(h));
+    const int64_t xoff = ((b * L + t0) * H + h) * P;
+    __syncthreads();  // every wave is done with the previous head's tiles
+    const float pre = rpre, dl = rdl;   // the keeper: this head's raw steps and dL/dcs_L shares
+    if (keeper) {
+      const float csL = __shfl(rcs, Q - 1, 64), cslL = __shfl(rcsl, Q - 1, 64);
+      s_cs[lane] = rcs;
+      s_csl[lane] = rcsl;
+      s_dt[lane] = rdt;
+      s_w[lane] = reach ? fast_exp((csL - rcs) + (cslL - rcsl)) : 0.f;
+      s_ecs[lane] = from ? fast_exp(rcs + rcsl) : 0.f;
+    }
+    map_park<bf16>(s_X, kLdP, kPlaneP, mp, rx, nvalid);
+    {  // dY = dout silu(z), dz
+#pragma unroll
+      for (int k = 0; k < VX; ++k) {
+        const int t = mp.row + k * mp.step;
+        const bool in = t < nvalid;
+        const float4 g4 = widen<bf16>(in ? rgo[k] : raw_zero<bf16>());
+        float dy[4] = {g4.x, g4.y, g4.z, g4.w};
+        if (HAS_Z) {
+          const float4 z4 = widen<bf16>(rz[k]), y4 = widen<bf16>(ry[k]);
+          const float zx[4] = {z4.x, z4.y, z4.z, z4.w}, yv[4] = {y4.x, y4.y, y4.z, y4.w};
+          float dz[4];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            const float sg = sigmoid(zx[u]);
+            dz[u] = dy[u] * yv[u] * sg * (1.f + zx[u] * (1.f - sg));
+            dy[u] = in ? dy[u] * zx[u] * sg : 0.f;
+          }
+          if (in)
+            st4<bf16>(static_cast<bf16*>(p.dz) + xoff + lane_offset(t * static_cast<uint32_t>(H * P) + mp.col),
+                      make_float4(dz[0], dz[1], dz[2], dz[3]));
+        }
+        uint2 o[3];
+        split4<3>(dy, o);
+#pragma unroll
+        for (int u = 0; u < 3; ++u) *reinterpret_cast<uint2*>(s_dY + u * kPlaneP + t * kLdP + mp.col) = o[u];
+      }
+    }
+    park_states();
+    __syncthreads();
+    fetch_states(h, 1);
+    // This wave's own x (s) or dY (t) rows, terms over p in frag_col's order.
+    Frag<1> xo[2];
+    Frag<3> yo[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      if (sw) xo[k] = frag_row_as_col<1>(s_X + own * kLdP + 32 * k, kLdP, kPlaneP);
+      else yo[k] = frag_row_as_col<3>(s_dY + own * kLdP + 32 * k, kLdP, kPlaneP);
+    }
+    v4f dxa[4], dxs[4];   // s-wave: d(dt x) from the chunk, and from the state before w
+    zero(dxa);
+    zero(dxs);
+    // dG of each pair of tiles (32 of the other's steps), then G, dCB = dt_s dG
+    // o M and R = dCB o C B^T, whose sum over the pair's rows is this lane's
+    // column sum (s-wave) or row sum (t-wave) of R.
+    float rpart[4] = {0.f, 0.f, 0.f, 0.f};   // per tile: short chains of additions
+    {
+      const float cso = s_cs[step_own], cslo = s_csl[step_own], dto = s_dt[step_own];
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt) {
+        if (sw ? 32 * kt + 31 < own : 32 * kt > own) continue;   // above the diagonal
+        v4f gv[2], dv[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          const int row0 = 32 * kt + 16 * u;
+          v4f dg = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int k = 0; k < 2; ++k) {
+            if (sw) dg = mma32(frag_row_as_col<3>(s_dY + row0 * kLdP + 32 * k, kLdP, kPlaneP), xo[k], dg);
+            else dg = mma32(frag_row_as_col<1>(s_X + row0 * kLdP + 32 * k, kLdP, kPlaneP), yo[k], dg);
+          }
+          const int o0 = row0 + 4 * q;
+          const float4 c4 = *reinterpret_cast<const float4*>(&s_cs[o0]);
+          const float4 l4 = *reinterpret_cast<const float4*>(&s_csl[o0]);
+          const float4 d4 = *reinterpret_cast<const float4*>(&s_dt[o0]);
+          const float cv[4] = {c4.x, c4.y, c4.z, c4.w}, lv[4] = {l4.x, l4.y, l4.z, l4.w},
+                      tv[4] = {d4.x, d4.y, d4.z, d4.w};
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int o = o0 + e;
+            const float dc = sw ? (cv[e] - cso) + (lv[e] - cslo) : (cso - cv[e]) + (cslo - lv[e]);
+            const bool in = sw ? (o >= step_own && o <= bound) : (o <= step_own && o >= bound);
+            const float m = in ? fast_exp(dc) : 0.f;
+            gv[u][e] = cb[2 * kt + u][e] * m;
+            dv[u][e] = dg[e] * (sw ? dto : tv[e]) * m;
+            rpart[2 * kt + u] = fmaf(dv[u][e], cb[2 * kt + u][e], rpart[2 * kt + u]);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        const Frag<3> df = frag_acc<3>(dv[0], dv[1]);
+        if (sw) {  // d(dt x)[s][p] += sum_t G[t][s] dY[t][p]
+          const Frag<3> gf = frag_acc<3>(gv[0], gv[1]);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            dxa[j] = mma32(gf, frag_col<3>(s_dY + 32 * kt * kLdP + 16 * j, kLdP, kPlaneP), dxa[j]);
+            if (j & 1) __builtin_amdgcn_sched_barrier(0);  // two operands at a time: registers
+          }
+        }
+        // dB[s][n] += sum_t dCB[t][s] C[t][n], or dC[t][n] += sum_s dCB[t][s] B[s][n]
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          acc[j] = mma32(df, frag_col<1>(s_oth + 32 * kt * kLdT + 16 * j, kLdT, 0), acc[j]);
+          if (j & 1) __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      float rsum = (rpart[0] + rpart[1]) + (rpart[2] + rpart[3]);
+      rsum = swap_sum<32>(rsum, rsum);
+      rsum = swap_sum<16>(rsum, rsum);
+      if (q == 0) (sw ? lds.col : lds.row)[step_own] = rsum;
+    }
+    if (i + 1 < p.hb) fetch(h + 1);   // here, not above: the chunk products need the registers
+    // State terms, over 64-state groups of dH^out and H.
+    const float4 f4 = *reinterpret_cast<const float4*>(sw ? &s_w[own + 4 * q] : &s_ecs[own + 4 * q]);
+    const float4 t4 = *reinterpret_cast<const float4*>(&s_dt[own + 4 * q]);
+    const float fr[4] = {f4.x, f4.y, f4.z, f4.w};   // w_s or exp(cs_t) of the rows own + 4 q + e
+    const float dtr[4] = {t4.x, t4.y, t4.z, t4.w};
+    float a_grp[4][4] = {};                         // t-wave: sum_n C[t][n] exp(cs_t) (dY H)[t][n], 32 states each
+#pragma unroll
+    for (int grp = 0; grp < 2; ++grp) {
+      if (grp == 1) {
+        __syncthreads();  // every wave is done reading s_dH / s_H
+        park_states();
+        __syncthreads();
+        if (i + 1 < p.hb) fetch_states(h + 1, 0);
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        v4f tv = {0.f, 0.f, 0.f, 0.f};
+        if (sw) {
+          // (x dH)[s][n], and (B dH^T)[s][p] of headdim tile j
+#pragma unroll
+          for (int k = 0; k < 2; ++k) {
+            tv = mma32(xo[k], frag_col<3>(s_dH + 32 * k * kLdP + 16 * j, kLdP, kPlaneP), tv);
+            dxs[j] = mma32(frag_row<1>(s_own + 64 * grp + 32 * k, kLdT, 0),
+                           frag_row<3>(s_dH + 16 * j * kLdP + 32 * k, kLdP, kPlaneP), dxs[j]);
+          }
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[4 * grp + j][e] = fmaf(fr[e] * dtr[e], tv[e], acc[4 * grp + j][e]);
+        } else {
+          // (dY H)[t][n]
+#pragma unroll
+          for (int k = 0; k < 2; ++k)
+            tv = mma32(yo[k], frag_col<3>(s_H + 32 * k * kLdP + 16 * j, kLdP, kPlaneP), tv);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float ys = fr[e] * tv[e];
+            acc[4 * grp + j][e] += ys;
+            const uint32_t cw = cd[e][2 * grp + (j >> 1)];
+            a_grp[2 * grp + (j >> 1)][e] =
+                fmaf(__builtin_bit_cast(float, j & 1 ? cw & 0xffff0000u : cw << 16), ys, a_grp[2 * grp + (j >> 1)][e]);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    if (!sw) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float a = row_allreduce16((a_grp[0][e] + a_grp[1][e]) + (a_grp[2][e] + a_grp[3][e]));
+        if (r == e) lds.a[own + 4 * q + e] = a;
+      }
+    }
+    __syncthreads();  // every wave is done reading s_dH / s_H
+    if (sw)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int at = (own + 4 * q + e) * XP + 16 * j + r;
+          const float wv = fr[e] * dxs[j][e];
+          s_W[at] = wv;
+          s_dX[at] = dxa[j][e] + wv;
+        }
+    __syncthreads();
+    // dx = dt dX + D dY; c = <x, dX>, b = dt <x, W> per row; dD over the rows
+    {
+      float dD[4] = {0.f, 0.f, 0.f, 0.f};
+      const float4 D4 = p.D ? *reinterpret_cast<const float4*>(p.D + h * P + mp.col) : make_float4(0.f, 0.f, 0.f, 0.f);
+      const float Dv[4] = {D4.x, D4.y, D4.z, D4.w};
+#pragma unroll
+      for (int k = 0; k < VX; ++k) {
+        const int s = mp.row + k * mp.step;
+        const float4 X4 = *reinterpret_cast<const float4*>(&s_dX[s * XP + mp.col]);
+        const float4 W4 = *reinterpret_cast<const float4*>(&s_W[s * XP + mp.col]);
+        const float4 x4 = pieces4<1>(s_X + s * kLdP + mp.col, kPlaneP);
+        const float4 y4 = pieces4<3>(s_dY + s * kLdP + mp.col, kPlaneP);
+        const float dt = s_dt[s];
+        const float Xv[4] = {X4.x, X4.y, X4.z, X4.w}, Wv[4] = {W4.x, W4.y, W4.z, W4.w},
+                    xv[4] = {x4.x, x4.y, x4.z, x4.w}, yv[4] = {y4.x, y4.y, y4.z, y4.w};
+        float cr = fmaf(Xv[0], xv[0], Xv[1] * xv[1]) + fmaf(Xv[2], xv[2], Xv[3] * xv[3]);
+        float br = fmaf(Wv[0], xv[0], Wv[1] * xv[1]) + fmaf(Wv[2], xv[2], Wv[3] * xv[3]);
+        float o[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          dD[u] = fmaf(yv[u], xv[u], dD[u]);
+          o[u] = fmaf(Dv[u], yv[u], Xv[u] * dt);
+        }
+        cr = row_allreduce16(cr);
+        br = row_allreduce16(br);
+        if (r == 0) {
+          lds.c[s] = cr;
+          lds.b[s] = br * dt;
+        }
+        if (s < nvalid)
+          st4<bf16>(static_cast<bf16*>(p.dx) + xoff + lane_offset(s * static_cast<uint32_t>(H * P) + mp.col),
+                    make_float4(o[0], o[1], o[2], o[3]));
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        dD[u] = swap_sum<32>(dD[u], dD[u]);
+        dD[u] = swap_sum<16>(dD[u], dD[u]);
+      }
+      if (q == 0) *reinterpret_cast<float4*>(&lds.dD[wave][4 * r]) = make_float4(dD[0], dD[1], dD[2], dD[3]);
+    }
+    __syncthreads();
+    const int64_t prt = (b * p.nchunks + c) * H + h;
+    if (keeper) {
+      // dcs = row sums - column sums of R + the state terms; the last step also
+      // takes the cs_L terms (the states' dependence on w, and the passing's
+      // shares); da = suffix sums over the chunk; dstep = c + da A, then through
+      // softplus / clamp / bias
+      const float bv = lds.b[lane];
+      float lo = 0.f;
+      float v = add2(add2(lds.row[lane], -lds.col[lane], lo), add2(lds.a[lane], -bv, lo), lo);
+      const float last = wave_total(bv) + wave_total(dl);
+      if (lane == Q - 1) v = add2(v, last, lo);
+      const float da = wave_suffix_sum2(v, lo);
+      float ddt_raw = 0.f, dA_term = 0.f;
+      if (lane < nvalid) {
+        float gfac;
+        step_of(p, pre + (p.dt_bias ? p.dt_bias[h] : 0.f), &gfac);
+        ddt_raw = fmaf(da, p.A[h], lds.c[lane]) * gfac;
+        dA_term = da * s_dt[lane];
+        p.ddt[(b * L + t0 + lane) * H + h] = ddt_raw;
+      }
+      const float wa = wave_total(dA_term), wb = wave_total(ddt_raw);
+      if (lane == 0) {
+        p.dA_part[prt] = wa;
+        p.dbias_part[prt] = wb;
+      }
+    } else if (!SW && wave == 5) {
+      float v = 0.f;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v += lds.dD[k][lane];
+      p.dD_part[prt * P + lane] = v;
+    }
+  }
+  // the block's dB and dC partial sums
+  float* const part = sw ? p.dB_part : p.dC_part;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int t = own + 4 * q + e;
+    if (t >= nvalid) continue;
+    const int64_t at = ((b * L + t0 + t) * p.nhb + blockIdx.y) * N;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) part[at + 16 * j + r] = acc[j][e];
+  }
+}
+
+template <bool HAS_Z, bool SEQ>
+__global__ void __launch_bounds__(kThreads3, 2) ssd_bwd_chunk_bf16_kernel(const SsdParams p) {
+  constexpr int TPB = kThreads3, N = kSsdMaxN;
+  __shared__ BwdChunkLds lds;
+  const int64_t c = blockIdx.x, b = blockIdx.z;
+  const int64_t L = p.seqlen, G = p.ngroups;
+  const int64_t g = static_cast<int64_t>(blockIdx.y) * p.hb / (p.nheads / G);
+  const int64_t t0 = c * Q;
+  const int nvalid = chunk_steps(p, t0);
+  {
+    const TileMap<TPB, N, true> mn(N);
+    constexpr int VN = vec_n<TPB>();
+    const int64_t off = ((b * L + t0) * G + g) * N;
+    raw4<bf16> rb[VN], rc[VN];
+    map_load<bf16>(rb, mn, static_cast<const bf16*>(p.B) + off, G * N, nvalid);
+    map_load<bf16>(rc, mn, static_cast<const bf16*>(p.C) + off, G * N, nvalid);
+    map_park<bf16>(lds.B, kLdT, 0, mn, rb, nvalid);
+    map_park<bf16>(lds.C, kLdT, 0, mn, rc, nvalid);
+  }
+  if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) < 4) bwd_chunk_waves<HAS_Z, SEQ, true>(p, lds);
+  else bwd_chunk_waves<HAS_Z, SEQ, false>(p, lds);
+}
+
 // Per-sequence final states of packed sequences in batch row 0 (mamba_ssm's
 // varlen states): entry i is the state after step e = cu[i + 1] - 1. From the
 // chunk c holding e, h_e = exp(cs_e) H_c (when step e is in the entering
@@ -1412,8 +1985,15 @@ hipError_t fwd_t(const SsdParams& p, hipStream_t st) {
     hipLaunchKernelGGL(ssd_state_pass_kernel<SEQ>, slices, dim3(kThreads), 0, st, p);
   }
   if (hipError_t e = hipGetLastError()) return e;
-  if (p.z) hipLaunchKernelGGL((ssd_chunk_scan_kernel<Tx, true, SEQ>), chunks, dim3(kThreads3), 0, st, p);
-  else hipLaunchKernelGGL((ssd_chunk_scan_kernel<Tx, false, SEQ>), chunks, dim3(kThreads3), 0, st, p);
+  auto scan = [&](auto mn, auto exact) {
+    if (p.z)
+      hipLaunchKernelGGL((ssd_chunk_scan_kernel<Tx, true, SEQ, mn.value, exact.value>), chunks, dim3(kThreads3), 0, st, p);
+    else
+      hipLaunchKernelGGL((ssd_chunk_scan_kernel<Tx, false, SEQ, mn.value, exact.value>), chunks, dim3(kThreads3), 0, st, p);
+  };
+  if (p.headdim == kSsdMaxP && p.dstate == 128) scan(std::integral_constant<int, 128>{}, std::true_type{});
+  else if (p.dstate > 64) scan(std::integral_constant<int, 128>{}, std::false_type{});
+  else scan(std::integral_constant<int, 64>{}, std::false_type{});
   return hipGetLastError();
 }
 
@@ -1437,6 +2017,13 @@ hipError_t bwd_t(const SsdParams& p, hipStream_t st) {
     hipLaunchKernelGGL(ssd_bwd_pass_kernel<SEQ>, slices, dim3(kThreads), 0, st, p);
   }
   if (hipError_t e = hipGetLastError()) return e;
+  if constexpr (std::is_same_v<Tx, bf16>) {
+    if (p.headdim == kSsdMaxP && p.dstate == kSsdMaxN) {
+      if (p.z) hipLaunchKernelGGL((ssd_bwd_chunk_bf16_kernel<true, SEQ>), chunks, dim3(kThreads3), 0, st, p);
+      else hipLaunchKernelGGL((ssd_bwd_chunk_bf16_kernel<false, SEQ>), chunks, dim3(kThreads3), 0, st, p);
+      return hipGetLastError();
+    }
+  }
   if (p.z) hipLaunchKernelGGL((ssd_bwd_chunk_kernel<Tx, true, SEQ>), chunks, dim3(kThreads3), 0, st, p);
   else hipLaunchKernelGGL((ssd_bwd_chunk_kernel<Tx, false, SEQ>), chunks, dim3(kThreads3), 0, st, p);
   return hipGetLastError();

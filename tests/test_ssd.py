@@ -295,3 +295,28 @@ def test_opcheck_ssd_ops():
     out, fin, saved, ysave = torch.ops.mamba_cpu.ssd_fwd(*args)
     bargs = (torch.randn_like(out), torch.randn_like(fin)) + args[:12] + (saved, ysave)
     torch.library.opcheck(torch.ops.mamba_cpu.ssd_bwd.default, bargs)
+
+
+@pytest.mark.parametrize("seqlen", [1, 17, 63, 64, 65, 128, 200])
+@pytest.mark.parametrize("headdim,dstate", [(64, 128), (64, 64), (16, 16), (48, 80), (32, 112)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_tile_edges_of_every_product_form(seqlen, headdim, dstate, dtype):
+    """The products in bf16 pieces (one to three per operand, by storage type)
+    with chunks and tiles cut at every edge: lengths around the 64-step chunk and
+    its 32-step halves, the exact 64 x 128 shape and ones padded in headdim,
+    dstate or both, single and packed sequences. The pieces carry float32's 24
+    bits, so without z (whose saved y is rounded to the storage type) the float32
+    results of 16-bit inputs meet the float32 bounds too."""
+    rng = np.random.default_rng(seqlen)
+    for seq in (None, np.sort(rng.integers(0, 3, (2, seqlen)), axis=1).astype(np.int32)):
+        c = case(2, seqlen, 4, headdim, 2, dstate, seed=seqlen + headdim, z=dtype == torch.float32, init=True,
+                 dtype=dtype)
+        got = run_ops(c, seq=seq)
+        check_ops(c, got, low=dtype != torch.float32, seq=seq)
+        if dtype != torch.float32:
+            _, fin, g, W, V = got
+            kw = dict(dt_softplus=True, seq_idx=seq)
+            assert_close_report(fin, S.ssd_fwd(**c, **kw)[1], 1e-4, 1e-5, "final_states")
+            wg = dict(zip(NAMES, S.ssd_bwd(**c, **kw, dout=W.float(), dfinal_states=V)))
+            for name, i, atol in (("dt", 1, 1e-4), ("A", 2, 1e-3), ("D", 5, 1e-3), ("dt_bias", 7, 1e-3)):
+                assert_close_report(g[i], wg[name], 1e-3, atol, f"d{name}")
