@@ -74,16 +74,16 @@ int head_block(const mcpu_ssd_args* a, bool bwd) {
   return hb;
 }
 
-// Whether the chunk states are carried by the in-order kernels, one
-// workgroup per (batch, head, 64-state column block) walking every chunk, or
-// by the two-launch form, parallel over chunks. The in-order forward is the
-// faster from about 256 such workgroups, the in-order backward from about
-// 160 (measured at 48-640 of them); the two directions choose on their own
-// (the saved buffer is the same for both forms).
-bool in_order(const mcpu_ssd_args* a, bool bwd) {
+// Whether the chunk states are carried by the walking kernels, one workgroup
+// per (batch, head, 64-state column block) in chunk order, or by the two-launch
+// form, parallel over chunks. In both directions walking is the faster from
+// about 150 such workgroups (timed at 48-320 of them, 5-64 chunks, bf16 and
+// float32: at 144, 152 against 153 us forward and 318 against 317 backward; at
+// 160, 56 against 61 and 84 against 89; at 96, 47 against 41 and 67 against 62).
+bool in_order(const mcpu_ssd_args* a) {
   if (a->chunk_pass != 0) return a->chunk_pass == 2;
   const int64_t cols = (a->dstate + kSsdPassCols - 1) / kSsdPassCols;
-  return a->batch * a->nheads * cols >= (bwd ? 160 : 256);
+  return a->batch * a->nheads * cols >= 150;
 }
 
 SsdParams make_ssd(const mcpu_ssd_args* a, bool bwd = false) {
@@ -106,7 +106,7 @@ SsdParams make_ssd(const mcpu_ssd_args* a, bool bwd = false) {
   p.ngroups = a->ngroups;
   p.dstate = a->dstate;
   p.nchunks = (a->seqlen + kSsdQ - 1) / kSsdQ;
-  p.in_order = in_order(a, bwd) ? 1 : 0;
+  p.in_order = in_order(a) ? 1 : 0;
   p.nslices = p.in_order ? (a->dstate + kSsdPassCols - 1) / kSsdPassCols
                          : (a->headdim * a->dstate + kSsdSlice - 1) / kSsdSlice;
   p.hb = a->head_block != 0 ? a->head_block : head_block(a, bwd);

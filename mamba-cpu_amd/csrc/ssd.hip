@@ -1,7 +1,8 @@
 // Mamba-2 SSD scan (mamba_ssm's mamba_chunk_scan_combined) on gfx950, in
-// 64-step chunks with the chunk-local contractions on the matrix cores
-// (v_mfma_f32_16x16x4_f32, float32 in and out; the storage type is widened
-// when a tile is staged in LDS).
+// 64-step chunks with the chunk-local contractions on the matrix cores: in bf16
+// pieces at float32 accuracy (ssd_pieces.h), or, in the chunk gradients of
+// storage and shapes other than bf16 64 x 128 and the per-sequence states, on
+// v_mfma_f32_16x16x4_f32 with the storage type widened when a tile is staged.
 //
 // Per batch row b and head h (group g), with a_t = dt_t A and, inside a
 // chunk, cs_t = a_0 + ... + a_t (so cs <= 0 and decays are exp of differences):
@@ -21,9 +22,11 @@
 //         per-chunk partials of dA, dD, ddt_bias
 //     a fixed-order reduce sums dB/dC over the head blocks of a group and the
 //     partials.
-// The chunk kernels (F1, F3, K1, K3) give a workgroup one chunk of `hb` heads
-// of one group: B, C and C B^T are staged and formed once and each head reuses
-// them; K3 keeps dB and dC of the block's heads in matrix-core accumulators.
+// F1 and F2, and K1 and K2, run as one launch each (F12, K12) where enough
+// workgroups walk the chunks in order (ssd_state_kernel).
+// The chunk kernels (F3, K3) give a workgroup one chunk of `hb` heads of one
+// group: B, C and C B^T are staged and formed once and each head reuses them;
+// K3 keeps dB and dC of the block's heads in matrix-core accumulators.
 // Chunks past the sequence end are padded with dt = 0 (no decay, no input).
 #include "mcpu_common.h"
 #include "scan_common.h"
@@ -195,22 +198,6 @@ __device__ __forceinline__ void tile_store(float* s, int ld, const raw4<Tx> (&x)
   }
 }
 
-// The same with entry k times sc[k].
-template <typename Tx, int V, int TPB = kThreads>
-__device__ __forceinline__ void tile_store_scaled(float* s, int ld, const raw4<Tx> (&x)[V], int nrows, int ncols,
-                                                  const float (&sc)[V]) {
-  const int nv = ncols >> 2, total = nrows * nv;
-  const float inv = 1.0f / static_cast<float>(nv);
-#pragma unroll
-  for (int k = 0; k < V; ++k) {
-    const int v = threadIdx.x + k * TPB;
-    if (v < total) {
-      const int r = tile_row(v, inv);
-      *reinterpret_cast<float4*>(s + r * ld + ((v - r * nv) << 2)) = scale4(widen<Tx>(x[k]), sc[k]);
-    }
-  }
-}
-
 // How TPB threads move a tile of NC columns (64 or 128), of which the first
 // ncols exist, four elements at a time: NC / 4 threads to a row, so a thread
 // keeps its column and steps down the rows. EXACT: ncols = NC.
@@ -310,10 +297,10 @@ struct DyTiles {
     }
   }
 
-  // LDS tile of dY = dout silu(z) (dout without z), times scale[r] when
-  // given; dz = dout y silu'(z) written to rows below nvalid when write_dz.
+  // LDS tile of dY = dout silu(z) (dout without z); dz = dout y silu'(z)
+  // written to rows below nvalid when write_dz.
   __device__ __forceinline__ void store(float* s, int ld, const SsdParams& p, int64_t off, int64_t rs, int nvalid,
-                                        int ncols, bool write_dz, const float* scale = nullptr) const {
+                                        int ncols, bool write_dz) const {
     const int nv = ncols >> 2, total = Q * nv;
     const float inv = 1.0f / static_cast<float>(nv);
 #pragma unroll
@@ -325,20 +312,7 @@ struct DyTiles {
       float4 dz = make_float4(0.f, 0.f, 0.f, 0.f);
       const float4 dy = dy_of(k, write_dz ? &dz : nullptr);
       if (HAS_Z && write_dz && r < nvalid) st4<Tx>(static_cast<Tx*>(p.dz) + off + r * rs + c, dz);
-      *reinterpret_cast<float4*>(s + r * ld + c) = scale ? scale4(dy, scale[r]) : dy;
-    }
-  }
-
-  // The same LDS tile (no dz) with float4 number k scaled by sc[k].
-  __device__ __forceinline__ void store_scaled(float* s, int ld, int ncols, const float (&sc)[V]) const {
-    const int nv = ncols >> 2, total = Q * nv;
-    const float inv = 1.0f / static_cast<float>(nv);
-#pragma unroll
-    for (int k = 0; k < V; ++k) {
-      const int v = threadIdx.x + k * TPB;
-      if (v >= total) continue;
-      const int r = tile_row(v, inv);
-      *reinterpret_cast<float4*>(s + r * ld + ((v - r * nv) << 2)) = scale4(dy_of(k, nullptr), sc[k]);
+      *reinterpret_cast<float4*>(s + r * ld + c) = dy;
     }
   }
 
@@ -499,59 +473,6 @@ __device__ __forceinline__ bool carries(const SsdParams& p, int64_t b, int64_t c
 
 }  // namespace
 
-// F1: steps and running decays of each head's chunk (saved for F3 and the
-// backward), and the chunk-end state S(p, n) = sum_s exp(cs_L - cs_s) dt_s
-// x_s(p) B_s(n). Grid (nchunks, nhb, batch); wave w computes state rows p in
-// [16 w, 16 w + 16).
-template <typename Tx, bool SEQ>
-__global__ void __launch_bounds__(kThreads) ssd_chunk_state_kernel(const SsdParams p) {
-  __shared__ __align__(16) float s_B[Q][NP];
-  __shared__ __align__(16) float s_x[Q][XP];
-  __shared__ float s_sc[Q];
-  const int64_t c = blockIdx.x, b = blockIdx.z;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int r = lane & 15, q = lane >> 4;
-  const int64_t L = p.seqlen, H = p.nheads, P = p.headdim, N = p.dstate, G = p.ngroups;
-  const int64_t h0 = static_cast<int64_t>(blockIdx.y) * p.hb;
-  const int64_t g = h0 / (H / G);
-  const int64_t t0 = c * Q;
-  const int nvalid = chunk_steps(p, t0);
-  stage<Tx, kVecN>(&s_B[0][0], NP, static_cast<const Tx*>(p.B) + ((b * L + t0) * G + g) * N, G * N, Q, nvalid,
-            static_cast<int>(N));
-  for (int i = 0; i < p.hb; ++i) {
-    const int64_t h = h0 + i;
-    if (wave == 0) {
-      const float st = ssd_step(p, b, t0 + lane, h, nullptr);
-      float cs, csl;
-      wave_prefix_sum2(st * p.A[h], cs, csl);
-      const int64_t row = chunk_row(p, b, h, c);
-      p.cs[row + lane] = cs;
-      p.cs_lo[row + lane] = csl;
-      p.step[row + lane] = st;
-      const float csL = __shfl(cs, Q - 1, 64), cslL = __shfl(csl, Q - 1, 64);
-      // steps of another sequence than the chunk's last do not reach its end state
-      const bool reach = seq_of<SEQ>(p, b, t0 + lane) == seq_of<SEQ>(p, b, t0 + nvalid - 1);
-      s_sc[lane] = reach ? st * fast_exp((csL - cs) + (cslL - csl)) : 0.f;
-    }
-    __syncthreads();
-    stage<Tx, kVecX>(&s_x[0][0], XP, static_cast<const Tx*>(p.x) + ((b * L + t0) * H + h) * P, H * P, Q, nvalid,
-              static_cast<int>(P), s_sc);
-    __syncthreads();
-    if (16 * wave < P) {
-      v4f acc[kSsdMaxN / 16];
-      zero(acc);
-      mma(acc, static_cast<int>(N / 16), &s_x[0][16 * wave], 1, XP, &s_B[0][0], NP, 1, Q);
-      float* dst = p.states + state_block(p, b, c, h);
-#pragma unroll
-      for (int j = 0; j < kSsdMaxN / 16; ++j)
-        if (j < N / 16)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) dst[(16 * wave + 4 * q + e) * N + 16 * j + r] = acc[j][e];
-    }
-    __syncthreads();
-  }
-}
-
 // F2: walks the chunks in order, replacing each chunk-end state by the state
 // entering the chunk, H_c = exp(cs_L(c-1)) H_{c-1} + S_{c-1} (H_0 = the
 // initial state or 0), and writes the final state. One thread per state
@@ -597,115 +518,199 @@ __global__ void __launch_bounds__(kThreads) ssd_chunk_decay_kernel(const SsdPara
   p.step[row + lane] = st;
 }
 
-// Rows of the float4 entries a thread holds of a (64 x ncols) tile
-// (tile_load's mapping), clamped to the tile.
-template <int V>
-__device__ __forceinline__ void tile_rows(int (&rows)[V], int ncols) {
-  const float inv = 1.0f / static_cast<float>(ncols >> 2);
+constexpr int kLdS = 64 + 4;          // rows of the state kernel's 64-column tiles
+constexpr int kPlaneS = Q * kLdS;
+
+// Entries of map_load's mapping, times sc[k], in three pieces.
+template <int V, int TPB, int NC, bool EXACT>
+__device__ __forceinline__ void park_scaled(uint16_t* s, const TileMap<TPB, NC, EXACT>& m, const float4 (&x)[V],
+                                            const float (&sc)[V]) {
+  uint16_t* at = s + m.row * kLdS + m.col;
 #pragma unroll
   for (int k = 0; k < V; ++k) {
-    const int r = tile_row(static_cast<int>(threadIdx.x) + k * kThreads, inv);
-    rows[k] = r < Q ? r : Q - 1;
+    const float fv[4] = {x[k].x * sc[k], x[k].y * sc[k], x[k].z * sc[k], x[k].w * sc[k]};
+    uint2 o[3];
+    split4<3>(fv, o);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) *reinterpret_cast<uint2*>(at + k * m.step * kLdS + i * kPlaneS) = o[i];
   }
 }
 
-// F1 and F2 in one launch: the workgroup of (b, h, column block) walks the
-// chunks in order, holding state columns [64 x, 64 x + 64) of every row in
-// matrix-core accumulators. Per chunk c it stores H_c (the state entering c)
-// and forms H_{c+1} = exp(cs_L) H_c + sum_s exp(cs_L - cs_s) dt_s x_s B_s^T by
-// starting the products from the scaled H_c, so chunk-end states never reach
-// memory. The chunks' steps and running decays come from
-// ssd_chunk_decay_kernel; each thread loads those of its own x rows with the
-// next chunk's x and B while the current chunk's products run.
-// Grid (column blocks, nheads, batch); wave w owns state rows [16 w, 16 w + 16).
-// Three waves per SIMD, as the backward's.
-template <typename Tx, bool SEQ>
-__global__ void __launch_bounds__(kThreads, 3) ssd_state_scan_kernel(const SsdParams p) {
-  constexpr int VX = vec_x();
-  constexpr int VB = Q * kSsdPassCols / 4 / kThreads;
-  constexpr int BP = kSsdPassCols + 4;
-  __shared__ __align__(16) float s_x[Q][XP];    // dt_s exp(cs_L - cs_s) x_s
-  __shared__ __align__(16) float s_B[Q][BP];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+// The states' products, in both directions and both forms. Per chunk c, for 64
+// state columns of one head,
+//   forward   U_c = sum_s exp(cs_L - cs_s) dt_s x_s B_s^T
+//   backward  U_c = sum_t exp(cs_t) dY_t C_t^T
+// as (rows p, columns n) in matrix-core accumulators, both operands in pieces
+// and read transposed from the LDS tiles they are staged in.
+//   WALK (F12, K12): the workgroup of (b, h, column block) walks the chunks in
+//     the direction's order with the state X in the accumulators: it stores X
+//     (the state entering the chunk, or the gradient of the one leaving it), then
+//     X <- exp(cs_L) X + U_c, so that U never reaches memory. Grid (column
+//     blocks, nheads, batch).
+//   otherwise (F1, K1): the workgroup of (chunk, column block) stores U_c for
+//     the passing kernel; forward, it also forms and saves the chunk's steps and
+//     running decays. Grid (nchunks x column blocks, nheads, batch).
+// EXACT: headdim 64, dstate 128; otherwise tiles are filled up with zeros. The
+// next chunk's tiles load while the current products run.
+// DCS (backward walk): also <X, exp(cs_L) H_c> over its columns to dcsL, which the
+// bf16 chunk-gradient kernel (EXACT, bf16) forms itself from tiles it reads anyway.
+// What bounds it is memory: x (or dout and z) once per column block, X out.
+// Batch 4, seqlen 2048, 80 heads, bf16 with z: forward 138 us (3.7 TB/s), backward
+// 171 us (3.9 TB/s), against 195 and 254 us on float32 tiles, the latter with
+// H_c read for dcsL.
+template <typename Tx, bool HAS_Z, bool SEQ, bool BWD, bool WALK, bool EXACT>
+__global__ void __launch_bounds__(kThreads, 3) ssd_state_kernel(const SsdParams p) {
+  constexpr int TPB = kThreads, V = vec_x(), NX = kPieces<Tx>, NT = kSsdPassCols / 16;
+  constexpr bool DCS = BWD && WALK && !(EXACT && std::is_same_v<Tx, bf16>);
+  __shared__ __align__(16) uint16_t s_A[3 * kPlaneS];    // the scaled x or dY (steps x headdim)
+  __shared__ __align__(16) uint16_t s_B[NX * kPlaneS];   // B or C (steps x 64 states)
+  __shared__ float s_part[TPB / 64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, q = lane >> 4;
-  const int64_t L = p.seqlen, H = p.nheads, P = p.headdim, N = p.dstate, G = p.ngroups;
-  const int64_t n0 = static_cast<int64_t>(blockIdx.x) * kSsdPassCols;
+  const int64_t L = p.seqlen, H = p.nheads, G = p.ngroups;
+  const int64_t P = EXACT ? kSsdMaxP : p.headdim, N = EXACT ? kSsdMaxN : p.dstate;
+  const uint32_t ncb = static_cast<uint32_t>((N + kSsdPassCols - 1) / kSsdPassCols);
+  const int64_t blk = WALK ? blockIdx.x : blockIdx.x % ncb;
+  const int64_t n0 = blk * kSsdPassCols;
   const int64_t h = blockIdx.y, b = blockIdx.z;
   const int64_t g = h / (H / G);
   const int ncol = static_cast<int>(N - n0 < kSsdPassCols ? N - n0 : kSsdPassCols);
-  const int nt = ncol >> 4;
-  const bool act = 16 * wave < P;
+  const bool act = EXACT || 16 * wave < P;
+  const TileMap<TPB, kSsdMaxP, EXACT> ma(static_cast<int>(P));
+  const TileMap<TPB, kSsdPassCols, EXACT> mb(ncol);
   // Accumulator element (j, e) of this lane: state row 16 wave + 4 q + e,
   // column n0 + 16 j + r, at offset eo + e N + 16 j of a (headdim x dstate) block.
-  const int64_t eo = (16 * wave + 4 * q) * N + n0 + r;
-  v4f acc[kSsdPassCols / 16];
+  const uint32_t eo = static_cast<uint32_t>((16 * wave + 4 * q) * N + n0 + r);
+  auto on = [&](int j) { return EXACT || (act && 16 * j < ncol); };
+  v4f acc[NT];
+  zero(acc);
+  const float* init = BWD ? p.dfinal : p.init;
+  if (WALK && init != nullptr) {
+    const float* src = init + (b * H + h) * P * N;
 #pragma unroll
-  for (int j = 0; j < kSsdPassCols / 16; ++j)
+    for (int j = 0; j < NT; ++j)
 #pragma unroll
-    for (int e = 0; e < 4; ++e)
-      acc[j][e] = (act && j < nt && p.init) ? p.init[(b * H + h) * P * N + eo + e * N + 16 * j] : 0.f;
-
-  const Tx* xh = static_cast<const Tx*>(p.x) + b * L * H * P + h * P;
-  const Tx* Bg = static_cast<const Tx*>(p.B) + b * L * G * N + g * N + n0;
-  raw4<Tx> nx[VX], nB[VB];
-  int rows[VX];
-  tile_rows(rows, static_cast<int>(P));
-  float ncs[VX], nlo[VX], nst[VX], ncsL = 0.f, nloL = 0.f;
-  // packed sequences: the chunk's last run starts at step nlast (its steps
-  // reach the chunk's end state); H_c carries through the chunk
-  int nlast = 0;
-  bool ncarry = true;
+      for (int e = 0; e < 4; ++e)
+        if (on(j)) acc[j][e] = src[eo + e * N + 16 * j];
+  }
+  const Tx* const Ah = static_cast<const Tx*>(BWD ? p.dout : p.x) + b * L * H * P + h * P;
+  const Tx* const Zh = static_cast<const Tx*>(p.z) + b * L * H * P + h * P;
+  const Tx* const Bg = static_cast<const Tx*>(BWD ? p.C : p.B) + b * L * G * N + g * N + n0;
+  raw4<Tx> ra[V], rz[V], rb[V];
+  float ncs = 0.f, nlo = 0.f, nst = 0.f, nH[DCS ? NT : 1][4];
   auto fetch = [&](int64_t c) {
     const int64_t t0 = c * Q;
     const int nv = chunk_steps(p, t0);
-    tile_load<Tx, VX>(nx, xh + t0 * H * P, H * P, Q, nv, static_cast<int>(P));
-    tile_load<Tx, VB>(nB, Bg + t0 * G * N, G * N, Q, nv, ncol);
+    map_load<Tx>(ra, ma, Ah + t0 * H * P, H * P, nv);
+    if constexpr (BWD && HAS_Z) map_load<Tx>(rz, ma, Zh + t0 * H * P, H * P, nv);
+    map_load<Tx>(rb, mb, Bg + t0 * G * N, G * N, nv);
     const int64_t row = chunk_row(p, b, h, c);
-#pragma unroll
-    for (int k = 0; k < VX; ++k) {
-      ncs[k] = p.cs[row + rows[k]];
-      nlo[k] = p.cs_lo[row + rows[k]];
-      nst[k] = p.step[row + rows[k]];
+    if constexpr (BWD || WALK) {
+      const uint32_t at = lane_offset(lane);
+      ncs = (p.cs + row)[at];
+      nlo = (p.cs_lo + row)[at];
+      if (!BWD) nst = (p.step + row)[at];
+    } else {
+      nst = ssd_step(p, b, t0 + lane, h, nullptr);
+      wave_prefix_sum2(nst * p.A[h], ncs, nlo);
+      if (blk == 0 && wave == 0) {
+        p.cs[row + lane] = ncs;
+        p.cs_lo[row + lane] = nlo;
+        p.step[row + lane] = nst;
+      }
     }
-    ncsL = p.cs[row + Q - 1];
-    nloL = p.cs_lo[row + Q - 1];
-    if constexpr (SEQ) {  // the last run's first step, from a ballot over the chunk's steps
-      nlast = __ffsll(static_cast<long long>(
-                  __ballot(seq_of<SEQ>(p, b, t0 + lane) == seq_of<SEQ>(p, b, t0 + nv - 1)))) - 1;
-      ncarry = carries<SEQ>(p, b, c);
+    if constexpr (DCS) {
+      const float* hs = p.states + state_block(p, b, c, h);
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) nH[j][e] = on(j) ? hs[eo + e * N + 16 * j] : 0.f;
     }
   };
-  fetch(0);
-  for (int64_t c = 0; c < p.nchunks; ++c) {
-    const float decay = ncarry ? fast_exp(ncsL + nloL) : 0.f;
-    float sc[VX];  // dt_s exp(cs_L - cs_s) of this thread's rows s
+  float* const dcsl = DCS ? p.dcsL + (chunk_row(p, b, h, 0) / Q) * p.nslices + blk : nullptr;
+  int64_t pend = -1;        // chunk whose dcsL share awaits the cross-wave sum
+  float pend_decay = 0.f;
+  const int64_t only = WALK ? 0 : blockIdx.x / ncb;
+  const int64_t count = WALK ? p.nchunks : 1;
+  auto chunk_at = [&](int64_t i) { return WALK ? (BWD ? p.nchunks - 1 - i : i) : only; };
+  fetch(chunk_at(0));
+  for (int64_t i = 0; i < count; ++i) {
+    const int64_t c = chunk_at(i), t0 = c * Q;
+    const int nv = chunk_steps(p, t0);
+    // Lane t: step t's factor. Packed sequences: forward only the chunk's last
+    // run reaches its end, backward only the first reads the entering state.
+    const float csL = __shfl(ncs, Q - 1, 64), loL = __shfl(nlo, Q - 1, 64);
+    float f;
+    if constexpr (BWD) {
+      f = seq_of<SEQ>(p, b, t0 + lane) == seq_of<SEQ>(p, b, t0 - 1) ? fast_exp(ncs + nlo) : 0.f;
+    } else {
+      const bool reach = seq_of<SEQ>(p, b, t0 + lane) == seq_of<SEQ>(p, b, t0 + nv - 1);
+      f = reach ? nst * fast_exp((csL - ncs) + (loL - nlo)) : 0.f;
+    }
+    const float decay = WALK && carries<SEQ>(p, b, c) ? fast_exp(csL + loL) : 0.f;
+    float sc[V];
+    float4 av[V];
 #pragma unroll
-    for (int k = 0; k < VX; ++k) sc[k] = rows[k] >= nlast ? nst[k] * fast_exp((ncsL - ncs[k]) + (nloL - nlo[k])) : 0.f;
-    __syncthreads();  // the previous chunk's products are done with s_x and s_B
-    tile_store_scaled<Tx, VX>(&s_x[0][0], XP, nx, Q, static_cast<int>(P), sc);
-    tile_store<Tx, VB>(&s_B[0][0], BP, nB, Q, ncol);
-    if (c + 1 < p.nchunks) fetch(c + 1);
-    __syncthreads();
-    if (act) {
-      float* dst = p.states + state_block(p, b, c, h) + eo;
+    for (int k = 0; k < V; ++k) {
+      const int t = ma.row + k * ma.step;
+      const bool in = ma.on && t < nv;
+      sc[k] = __shfl(f, t, 64);
+      av[k] = widen<Tx>(in ? ra[k] : raw_zero<Tx>());
+      if constexpr (BWD && HAS_Z) {
+        const float4 z = widen<Tx>(in ? rz[k] : raw_zero<Tx>());
+        av[k] = make_float4(av[k].x * z.x * sigmoid(z.x), av[k].y * z.y * sigmoid(z.y),
+                            av[k].z * z.z * sigmoid(z.z), av[k].w * z.w * sigmoid(z.w));
+      }
+    }
+    float part = 0.f;
+    if (WALK && act) {
+      float* dst = (BWD ? p.dstates : p.states) + state_block(p, b, c, h);
 #pragma unroll
-      for (int j = 0; j < kSsdPassCols / 16; ++j)
-        if (j < nt)
+      for (int j = 0; j < NT; ++j)
+        if (on(j))
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            dst[e * N + 16 * j] = acc[j][e];
+            dst[lane_offset(eo) + e * N + 16 * j] = acc[j][e];
+            if constexpr (DCS) part = fmaf(acc[j][e], nH[j][e], part);
             acc[j][e] *= decay;
           }
-      mma(acc, nt, &s_x[0][16 * wave], 1, XP, &s_B[0][0], BP, 1, Q);
     }
+    if constexpr (DCS) part = wave_total(part);
+    __syncthreads();  // the previous chunk's products are done with s_A and s_B; its parts are in
+    if constexpr (DCS)
+      if (pend >= 0 && tid == 0)
+        dcsl[pend * p.nslices] = pend_decay * ((s_part[0] + s_part[1]) + (s_part[2] + s_part[3]));
+    park_scaled(s_A, ma, av, sc);
+    map_park<Tx>(s_B, kLdS, kPlaneS, mb, rb, nv);
+    if (i + 1 < count) fetch(chunk_at(i + 1));
+    __syncthreads();
+    if constexpr (DCS) {
+      if (lane == 0) s_part[wave] = part;
+      pend = c;
+      pend_decay = decay;
+    }
+    if (act)
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const Frag<3> a = frag_col<3>(s_A + 32 * k * kLdS + 16 * wave, kLdS, kPlaneS);
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+          if (on(j)) acc[j] = mma32(a, frag_col<NX>(s_B + 32 * k * kLdS + 16 * j, kLdS, kPlaneS), acc[j]);
+      }
   }
-  if (p.final_states && act) {
-    float* dst = p.final_states + (b * H + h) * P * N + eo;
+  if constexpr (DCS) {
+    __syncthreads();
+    if (pend >= 0 && tid == 0)
+      dcsl[pend * p.nslices] = pend_decay * ((s_part[0] + s_part[1]) + (s_part[2] + s_part[3]));
+  }
+  float* end = WALK ? (BWD ? p.dinit : p.final_states) : (BWD ? p.dstates : p.states);
+  if (end != nullptr && act) {
+    end += WALK ? (b * H + h) * P * N : state_block(p, b, only, h);
 #pragma unroll
-    for (int j = 0; j < kSsdPassCols / 16; ++j)
-      if (j < nt)
+    for (int j = 0; j < NT; ++j)
+      if (on(j))
 #pragma unroll
-        for (int e = 0; e < 4; ++e) dst[e * N + 16 * j] = acc[j][e];
+        for (int e = 0; e < 4; ++e) end[eo + e * N + 16 * j] = acc[j][e];
   }
 }
 
@@ -916,60 +921,13 @@ __global__ void __launch_bounds__(kThreads3, 4) ssd_chunk_scan_kernel(const SsdP
   }
 }
 
-// K1: the seed E_c[p][n] = sum_t exp(cs_t) dY[t][p] C[t][n] of dL/dH_c from
-// the chunk's own outputs, for each head of the block, into dstates. Grid
-// (nchunks, nhb, batch); wave w computes rows p in [16 w, 16 w + 16).
-template <typename Tx, bool HAS_Z, bool SEQ>
-__global__ void __launch_bounds__(kThreads) ssd_bwd_seed_kernel(const SsdParams p) {
-  __shared__ __align__(16) float s_C[Q][NP];
-  __shared__ __align__(16) float s_dY[Q][XP];     // exp(cs_t) dY[t][p]
-  __shared__ float s_ecs[Q];
-  const int64_t c = blockIdx.x, b = blockIdx.z;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int r = lane & 15, q = lane >> 4;
-  const int64_t L = p.seqlen, H = p.nheads, P = p.headdim, N = p.dstate, G = p.ngroups;
-  const int64_t h0 = static_cast<int64_t>(blockIdx.y) * p.hb;
-  const int64_t g = h0 / (H / G);
-  const int64_t t0 = c * Q;
-  const int nvalid = chunk_steps(p, t0);
-  stage<Tx, kVecN>(&s_C[0][0], NP, static_cast<const Tx*>(p.C) + ((b * L + t0) * G + g) * N, G * N, Q, nvalid,
-            static_cast<int>(N));
-  // packed sequences: step tid reads the entering state only within its sequence
-  const bool from = tid < Q && seq_of<SEQ>(p, b, t0 + tid) == seq_of<SEQ>(p, b, t0 - 1);
-  for (int i = 0; i < p.hb; ++i) {
-    const int64_t h = h0 + i;
-    const int64_t row = chunk_row(p, b, h, c);
-    __syncthreads();  // every wave is done with s_dY and s_ecs
-    if (tid < Q) s_ecs[tid] = from ? fast_exp(p.cs[row + tid] + p.cs_lo[row + tid]) : 0.f;
-    __syncthreads();
-    {
-      const int64_t off = ((b * L + t0) * H + h) * P;
-      DyTiles<Tx, HAS_Z> dyt;
-      dyt.load(p, off, H * P, nvalid, static_cast<int>(P), false);
-      dyt.store(&s_dY[0][0], XP, p, off, H * P, nvalid, static_cast<int>(P), false, s_ecs);
-    }
-    __syncthreads();
-    if (16 * wave < P) {
-      v4f ev[kSsdMaxN / 16];
-      zero(ev);
-      mma(ev, static_cast<int>(N / 16), &s_dY[0][16 * wave], 1, XP, &s_C[0][0], NP, 1, Q);
-      float* dst = p.dstates + state_block(p, b, c, h);
-#pragma unroll
-      for (int j = 0; j < kSsdMaxN / 16; ++j)
-        if (j < N / 16)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) dst[(16 * wave + 4 * q + e) * N + 16 * j + r] = ev[j][e];
-    }
-  }
-}
-
 // K2: walks the chunks from the last: dH^out_c (gradient of the state leaving
 // chunk c) replaces E_c in dstates, dH^in_c = exp(cs_L) dH^out_c + E_c
 // carries on, and <dH^out_c, exp(cs_L) H_c> (this slice's share of dL/dcs_L)
 // goes to dcsL. The gradient of the initial state is what is left after
 // chunk 0. Grid (nslices, nheads, batch). The next chunk's loads issue before
-// this chunk's store.
-template <bool SEQ>
+// this chunk's store. DCS: false where the chunk-gradient kernel forms dcsL.
+template <bool SEQ, bool DCS>
 __global__ void __launch_bounds__(kThreads) ssd_bwd_pass_kernel(const SsdParams p) {
   __shared__ float s_part[kThreads / 64];
   const int64_t PN = p.headdim * p.dstate, H = p.nheads;
@@ -984,137 +942,26 @@ __global__ void __launch_bounds__(kThreads) ssd_bwd_pass_kernel(const SsdParams 
   float* dcsl = p.dcsL + (chunk_row(p, b, h, 0) / Q) * p.nslices + blockIdx.x;
   const int64_t last = p.nchunks - 1;
   float ec = ok ? p.dstates[base + last * cstride] : 0.f;
-  float hin = ok ? p.states[base + last * cstride] : 0.f;
+  float hin = DCS && ok ? p.states[base + last * cstride] : 0.f;
   float dl = csl[last * Q];
   for (int64_t c = last; c >= 0; --c) {
     const float ecc = ec, hc = hin, d = carries<SEQ>(p, b, c) ? fast_exp(dl) : 0.f;
     if (c > 0) {
       ec = ok ? p.dstates[base + (c - 1) * cstride] : 0.f;
-      hin = ok ? p.states[base + (c - 1) * cstride] : 0.f;
+      if (DCS) hin = ok ? p.states[base + (c - 1) * cstride] : 0.f;
       dl = csl[(c - 1) * Q];
     }
     if (ok) p.dstates[base + c * cstride] = run;
-    const float part = wave_total(run * d * hc);
-    if (lane == 0) s_part[wave] = part;
-    __syncthreads();
-    if (threadIdx.x == 0) dcsl[c * p.nslices] = (s_part[0] + s_part[1]) + (s_part[2] + s_part[3]);
-    __syncthreads();
+    if constexpr (DCS) {
+      const float part = wave_total(run * d * hc);
+      if (lane == 0) s_part[wave] = part;
+      __syncthreads();
+      if (threadIdx.x == 0) dcsl[c * p.nslices] = (s_part[0] + s_part[1]) + (s_part[2] + s_part[3]);
+      __syncthreads();
+    }
     run = fmaf(d, run, ecc);
   }
   if (ok && p.dinit) p.dinit[(b * H + h) * PN + e] = run;
-}
-
-// K1 and K2 in one launch: the workgroup of (b, h, column block) walks the
-// chunks from the last, holding columns [64 x, 64 x + 64) of dL/d(state
-// leaving the chunk) in matrix-core accumulators. Per chunk c it stores
-// dH^out_c, adds <dH^out_c, exp(cs_L) H_c> over its columns to dcsL (slice x),
-// and forms dH^in_c = exp(cs_L) dH^out_c + (diag(exp(cs)) C)^T dY by starting
-// the products from the scaled dH^out_c, so the seeds never reach memory.
-// What is left after chunk 0 is the initial state's gradient. The next
-// chunk's dout, z, C, running decays and H load while the current chunk's
-// products run. Grid (column blocks, nheads, batch); wave w owns rows
-// [16 w, 16 w + 16). Three waves per SIMD: 640 workgroups (the Mamba-2 2.7B
-// layer at batch 4) run in one round.
-template <typename Tx, bool HAS_Z, bool SEQ>
-__global__ void __launch_bounds__(kThreads, 3) ssd_bwd_state_scan_kernel(const SsdParams p) {
-  constexpr int VB = Q * kSsdPassCols / 4 / kThreads;
-  constexpr int BP = kSsdPassCols + 4;
-  using Dy = DyTiles<Tx, HAS_Z>;
-  __shared__ __align__(16) float s_dY[Q][XP];   // exp(cs_t) dY[t][p]
-  __shared__ __align__(16) float s_C[Q][BP];
-  __shared__ float s_part[kThreads / 64];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int r = lane & 15, q = lane >> 4;
-  const int64_t L = p.seqlen, H = p.nheads, P = p.headdim, N = p.dstate, G = p.ngroups;
-  const int64_t n0 = static_cast<int64_t>(blockIdx.x) * kSsdPassCols;
-  const int64_t h = blockIdx.y, b = blockIdx.z;
-  const int64_t g = h / (H / G);
-  const int ncol = static_cast<int>(N - n0 < kSsdPassCols ? N - n0 : kSsdPassCols);
-  const int nt = ncol >> 4;
-  const bool act = 16 * wave < P;
-  const int64_t eo = (16 * wave + 4 * q) * N + n0 + r;
-  v4f acc[kSsdPassCols / 16];
-#pragma unroll
-  for (int j = 0; j < kSsdPassCols / 16; ++j)
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-      acc[j][e] = (act && j < nt && p.dfinal) ? p.dfinal[(b * H + h) * P * N + eo + e * N + 16 * j] : 0.f;
-
-  const Tx* Cg = static_cast<const Tx*>(p.C) + b * L * G * N + g * N + n0;
-  Dy dyt;
-  raw4<Tx> nC[VB];
-  float ncs = 0.f, nlo = 0.f, nH[kSsdPassCols / 16][4];
-  bool nfrom = true, ncarry = true;  // packed sequences: step lane reads H_c; H_c carries through the chunk
-  auto fetch = [&](int64_t c) {
-    const int64_t t0 = c * Q;
-    const int nv = chunk_steps(p, t0);
-    dyt.load(p, ((b * L + t0) * H + h) * P, H * P, nv, static_cast<int>(P), false);
-    tile_load<Tx, VB>(nC, Cg + t0 * G * N, G * N, Q, nv, ncol);
-    const int64_t row = chunk_row(p, b, h, c);
-    ncs = p.cs[row + lane];
-    nlo = p.cs_lo[row + lane];
-    nfrom = seq_of<SEQ>(p, b, t0 + lane) == seq_of<SEQ>(p, b, t0 - 1);
-    ncarry = carries<SEQ>(p, b, c);
-    const float* hs = p.states + state_block(p, b, c, h) + eo;
-#pragma unroll
-    for (int j = 0; j < kSsdPassCols / 16; ++j)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) nH[j][e] = (act && j < nt) ? hs[e * N + 16 * j] : 0.f;
-  };
-  float* dcsl = p.dcsL + (chunk_row(p, b, h, 0) / Q) * p.nslices + blockIdx.x;
-  int64_t pend = -1;        // chunk whose dcsL share awaits the cross-wave sum
-  float pend_decay = 0.f;
-  fetch(p.nchunks - 1);
-  for (int64_t c = p.nchunks - 1; c >= 0; --c) {
-    const float ecs_all = fast_exp(ncs + nlo);
-    const float decay = ncarry ? __shfl(ecs_all, Q - 1, 64) : 0.f;
-    const float ecs = nfrom ? ecs_all : 0.f;
-    // dH^out_c out, its share of dL/dcs_L, and the decayed carry, before the
-    // next chunk's H_c loads into the same registers.
-    float part = 0.f;
-    if (act) {
-      float* dst = p.dstates + state_block(p, b, c, h) + eo;
-#pragma unroll
-      for (int j = 0; j < kSsdPassCols / 16; ++j)
-        if (j < nt)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            dst[e * N + 16 * j] = acc[j][e];
-            part = fmaf(acc[j][e], nH[j][e], part);
-            acc[j][e] *= decay;
-          }
-    }
-    part = wave_total(part);
-    float sc[Dy::V];  // exp(cs_t) of this thread's dY rows t, from the lanes that own them
-    {
-      int rows[Dy::V];
-      tile_rows(rows, static_cast<int>(P));
-#pragma unroll
-      for (int k = 0; k < Dy::V; ++k) sc[k] = __shfl(ecs, rows[k], 64);
-    }
-    __syncthreads();  // the previous chunk's products are done with s_dY and s_C; its parts are in
-    if (pend >= 0 && tid == 0)
-      dcsl[pend * p.nslices] = pend_decay * ((s_part[0] + s_part[1]) + (s_part[2] + s_part[3]));
-    dyt.store_scaled(&s_dY[0][0], XP, static_cast<int>(P), sc);
-    tile_store<Tx, VB>(&s_C[0][0], BP, nC, Q, ncol);
-    if (c > 0) fetch(c - 1);
-    __syncthreads();
-    if (lane == 0) s_part[wave] = part;
-    pend = c;
-    pend_decay = decay;
-    if (act) mma(acc, nt, &s_dY[0][16 * wave], 1, XP, &s_C[0][0], BP, 1, Q);
-  }
-  __syncthreads();
-  if (pend >= 0 && tid == 0)
-    dcsl[pend * p.nslices] = pend_decay * ((s_part[0] + s_part[1]) + (s_part[2] + s_part[3]));
-  if (p.dinit && act) {
-    float* dst = p.dinit + (b * H + h) * P * N + eo;
-#pragma unroll
-    for (int j = 0; j < kSsdPassCols / 16; ++j)
-      if (j < nt)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) dst[e * N + 16 * j] = acc[j][e];
-  }
 }
 
 // K3: every gradient of a chunk, for each head of the block. Grid (nchunks,
@@ -1489,7 +1336,7 @@ struct BwdChunkLds {
   __align__(16) uint16_t X[kPlaneP], dY[3 * kPlaneP];
   __align__(16) uint16_t st[6 * kPlaneP];   // dH^out, then H, of a 64-state group; then dX and W
   __align__(16) float cs[Q], csl[Q], dt[Q], w[Q], ecs[Q];
-  float row[Q], col[Q], a[Q], b[Q], c[Q];
+  float row[Q], col[Q], a[Q], b[Q], c[Q], dh[8];
   float dD[8][kSsdMaxP];
   uint8_t first[Q], last[Q];                // ends of each step's sequence run in the chunk
 };
@@ -1549,7 +1396,7 @@ __device__ __forceinline__ void bwd_chunk_waves(const SsdParams& p, BwdChunkLds&
   // while the current products run.
   raw4<bf16> rx[VX], rgo[VX], rz[VX], ry[VX];
   float4 su[VX], sv[VX];
-  float rcs = 0.f, rcsl = 0.f, rdt = 0.f, rpre = 0.f, rdl = 0.f;
+  float rcs = 0.f, rcsl = 0.f, rdt = 0.f, rpre = 0.f;
   auto fetch = [&](int64_t h) {
     const int64_t row = chunk_row(p, b, h, c);
     const int64_t xoff = ((b * L + t0) * H + h) * P;
@@ -1559,7 +1406,6 @@ __device__ __forceinline__ void bwd_chunk_waves(const SsdParams& p, BwdChunkLds&
       rcsl = (p.cs_lo + row)[at];
       rdt = (p.step + row)[at];
       rpre = (p.dt + (b * L + t0) * H + h)[lane_offset((lane < nvalid ? lane : 0) * static_cast<uint32_t>(H))];
-      rdl = lane < p.nslices ? (p.dcsL + (row / Q) * p.nslices)[at] : 0.f;
     }
     map_load<bf16>(rx, mp, static_cast<const bf16*>(p.x) + xoff, H * P, nvalid);
     map_load<bf16>(rgo, mp, static_cast<const bf16*>(p.dout) + xoff, H * P, nvalid);
@@ -1573,7 +1419,13 @@ __device__ __forceinline__ void bwd_chunk_waves(const SsdParams& p, BwdChunkLds&
     map_load<float>(su, mp, p.dstates + sb, N, P);
     map_load<float>(sv, mp, p.states + sb, N, P);
   };
-  auto park_states = [&]() {
+  auto park_states = [&](float& dh) {
+    float v = 0.f;
+#pragma unroll
+    for (int k = 0; k < VX; ++k)
+      v += fmaf(su[k].x, sv[k].x, su[k].y * sv[k].y) + fmaf(su[k].z, sv[k].z, su[k].w * sv[k].w);
+    v = wave_total(v);
+    dh += __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
     map_park<float>(s_dH, kLdP, kPlaneP, mp, su, P);
     map_park<float>(s_H, kLdP, kPlaneP, mp, sv, P);
   };
@@ -1609,7 +1461,8 @@ __device__ __forceinline__ void bwd_chunk_waves(const SsdParams& p, BwdChunkLds&
     asm volatile("" : "+s"(h));
     const int64_t xoff = ((b * L + t0) * H + h) * P;
     __syncthreads();  // every wave is done with the previous head's tiles
-    const float pre = rpre, dl = rdl;   // the keeper: this head's raw steps and dL/dcs_L shares
+    const float pre = rpre;   // the keeper: this head's raw steps
+    float dh = 0.f;           // this wave's part of <dH^out, H_c>, uniform
     if (keeper) {
       const float csL = __shfl(rcs, Q - 1, 64), cslL = __shfl(rcsl, Q - 1, 64);
       s_cs[lane] = rcs;
@@ -1646,7 +1499,7 @@ __device__ __forceinline__ void bwd_chunk_waves(const SsdParams& p, BwdChunkLds&
         for (int u = 0; u < 3; ++u) *reinterpret_cast<uint2*>(s_dY + u * kPlaneP + t * kLdP + mp.col) = o[u];
       }
     }
-    park_states();
+    park_states(dh);
     __syncthreads();
     fetch_states(h, 1);
     // This wave's own x (s) or dY (t) rows, terms over p in frag_col's order.
@@ -1729,7 +1582,7 @@ __device__ __forceinline__ void bwd_chunk_waves(const SsdParams& p, BwdChunkLds&
     for (int grp = 0; grp < 2; ++grp) {
       if (grp == 1) {
         __syncthreads();  // every wave is done reading s_dH / s_H
-        park_states();
+        park_states(dh);
         __syncthreads();
         if (i + 1 < p.hb) fetch_states(h + 1, 0);
       }
@@ -1763,6 +1616,7 @@ __device__ __forceinline__ void bwd_chunk_waves(const SsdParams& p, BwdChunkLds&
         __builtin_amdgcn_sched_barrier(0);
       }
     }
+    if (lane == 0) lds.dh[wave] = dh;
     if (!sw) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
@@ -1826,13 +1680,15 @@ __device__ __forceinline__ void bwd_chunk_waves(const SsdParams& p, BwdChunkLds&
     const int64_t prt = (b * p.nchunks + c) * H + h;
     if (keeper) {
       // dcs = row sums - column sums of R + the state terms; the last step also
-      // takes the cs_L terms (the states' dependence on w, and the passing's
-      // shares); da = suffix sums over the chunk; dstep = c + da A, then through
+      // takes the cs_L terms (the states' dependence on w, and the entering
+      // state's decay through the chunk, exp(cs_L) <dH^out, H_c>); da = suffix sums over the chunk; dstep = c + da A, then through
       // softplus / clamp / bias
       const float bv = lds.b[lane];
       float lo = 0.f;
       float v = add2(add2(lds.row[lane], -lds.col[lane], lo), add2(lds.a[lane], -bv, lo), lo);
-      const float last = wave_total(bv) + wave_total(dl);
+      const float dhs = ((lds.dh[0] + lds.dh[1]) + (lds.dh[2] + lds.dh[3])) +
+                        ((lds.dh[4] + lds.dh[5]) + (lds.dh[6] + lds.dh[7]));
+      const float last = fmaf(s_ecs[Q - 1], dhs, wave_total(bv));
       if (lane == Q - 1) v = add2(v, last, lo);
       const float da = wave_suffix_sum2(v, lo);
       float ddt_raw = 0.f, dA_term = 0.f;
@@ -1960,38 +1816,55 @@ __global__ void __launch_bounds__(kThreads) ssd_varlen_state_kernel(const SsdPar
 
 namespace {
 
+bool exact_shape(const SsdParams& p) { return p.headdim == kSsdMaxP && p.dstate == kSsdMaxN; }
+
+// The states' products of one direction: walking the chunks (in order), or per
+// chunk, for every head (whatever the chunk kernels' head block).
+template <typename Tx, bool SEQ, bool BWD>
+hipError_t state_t(const SsdParams& p, hipStream_t st) {
+  const int64_t ncb = (p.dstate + kSsdPassCols - 1) / kSsdPassCols;
+  const dim3 grid(static_cast<unsigned>(p.in_order ? ncb : ncb * p.nchunks), static_cast<unsigned>(p.nheads),
+                  static_cast<unsigned>(p.batch));
+  auto go = [&](auto z, auto walk, auto exact) {
+    hipLaunchKernelGGL((ssd_state_kernel<Tx, z.value, SEQ, BWD, walk.value, exact.value>), grid, dim3(kThreads), 0,
+                       st, p);
+  };
+  auto form = [&](auto z, auto walk) {
+    if (exact_shape(p)) go(z, walk, std::true_type{});
+    else go(z, walk, std::false_type{});
+  };
+  auto gate = [&](auto z) {
+    if (p.in_order) form(z, std::true_type{});
+    else form(z, std::false_type{});
+  };
+  if (BWD && p.z) gate(std::integral_constant<bool, BWD>{});
+  else gate(std::false_type{});
+  return hipGetLastError();
+}
+
 template <typename Tx, bool SEQ>
 hipError_t fwd_t(const SsdParams& p, hipStream_t st) {
   const dim3 chunks(static_cast<unsigned>(p.nchunks), static_cast<unsigned>(p.nhb), static_cast<unsigned>(p.batch));
-  const dim3 slices(static_cast<unsigned>(p.nslices), static_cast<unsigned>(p.nheads),
-                    static_cast<unsigned>(p.batch));
   if (p.in_order) {
     const dim3 rows(static_cast<unsigned>((p.nchunks + kThreads / 64 - 1) / (kThreads / 64)),
                     static_cast<unsigned>(p.nheads), static_cast<unsigned>(p.batch));
     hipLaunchKernelGGL(ssd_chunk_decay_kernel, rows, dim3(kThreads), 0, st, p);
     if (hipError_t e = hipGetLastError()) return e;
-    hipLaunchKernelGGL((ssd_state_scan_kernel<Tx, SEQ>), slices, dim3(kThreads), 0, st, p);
-  } else {
-    // F1 with one head per workgroup whatever the chunk kernels' head block:
-    // each of its heads stages its own x and product, so more, smaller
-    // workgroups fill the GPU better (28 against 39 us at batch 4, seqlen
-    // 1024, 24 heads with blocks of 6); its outputs are per head.
-    SsdParams q = p;
-    q.hb = 1;
-    q.nhb = static_cast<int>(p.nheads);
-    const dim3 heads(static_cast<unsigned>(p.nchunks), static_cast<unsigned>(p.nheads), static_cast<unsigned>(p.batch));
-    hipLaunchKernelGGL((ssd_chunk_state_kernel<Tx, SEQ>), heads, dim3(kThreads), 0, st, q);
-    if (hipError_t e = hipGetLastError()) return e;
-    hipLaunchKernelGGL(ssd_state_pass_kernel<SEQ>, slices, dim3(kThreads), 0, st, p);
   }
-  if (hipError_t e = hipGetLastError()) return e;
+  if (hipError_t e = state_t<Tx, SEQ, false>(p, st)) return e;
+  if (!p.in_order) {
+    const dim3 slices(static_cast<unsigned>(p.nslices), static_cast<unsigned>(p.nheads),
+                      static_cast<unsigned>(p.batch));
+    hipLaunchKernelGGL(ssd_state_pass_kernel<SEQ>, slices, dim3(kThreads), 0, st, p);
+    if (hipError_t e = hipGetLastError()) return e;
+  }
   auto scan = [&](auto mn, auto exact) {
     if (p.z)
       hipLaunchKernelGGL((ssd_chunk_scan_kernel<Tx, true, SEQ, mn.value, exact.value>), chunks, dim3(kThreads3), 0, st, p);
     else
       hipLaunchKernelGGL((ssd_chunk_scan_kernel<Tx, false, SEQ, mn.value, exact.value>), chunks, dim3(kThreads3), 0, st, p);
   };
-  if (p.headdim == kSsdMaxP && p.dstate == 128) scan(std::integral_constant<int, 128>{}, std::true_type{});
+  if (exact_shape(p)) scan(std::integral_constant<int, 128>{}, std::true_type{});
   else if (p.dstate > 64) scan(std::integral_constant<int, 128>{}, std::false_type{});
   else scan(std::integral_constant<int, 64>{}, std::false_type{});
   return hipGetLastError();
@@ -2000,25 +1873,18 @@ hipError_t fwd_t(const SsdParams& p, hipStream_t st) {
 template <typename Tx, bool SEQ>
 hipError_t bwd_t(const SsdParams& p, hipStream_t st) {
   const dim3 chunks(static_cast<unsigned>(p.nchunks), static_cast<unsigned>(p.nhb), static_cast<unsigned>(p.batch));
-  const dim3 slices(static_cast<unsigned>(p.nslices), static_cast<unsigned>(p.nheads),
-                    static_cast<unsigned>(p.batch));
-  if (p.in_order) {
-    if (p.z) hipLaunchKernelGGL((ssd_bwd_state_scan_kernel<Tx, true, SEQ>), slices, dim3(kThreads), 0, st, p);
-    else hipLaunchKernelGGL((ssd_bwd_state_scan_kernel<Tx, false, SEQ>), slices, dim3(kThreads), 0, st, p);
-  } else {
-    // K1 with one head per workgroup, as F1 in the forward
-    SsdParams q = p;
-    q.hb = 1;
-    q.nhb = static_cast<int>(p.nheads);
-    const dim3 heads(static_cast<unsigned>(p.nchunks), static_cast<unsigned>(p.nheads), static_cast<unsigned>(p.batch));
-    if (p.z) hipLaunchKernelGGL((ssd_bwd_seed_kernel<Tx, true, SEQ>), heads, dim3(kThreads), 0, st, q);
-    else hipLaunchKernelGGL((ssd_bwd_seed_kernel<Tx, false, SEQ>), heads, dim3(kThreads), 0, st, q);
+  // The bf16 chunk-gradient kernel, which forms its own dcsL.
+  const bool pieces = std::is_same_v<Tx, bf16> && exact_shape(p);
+  if (hipError_t e = state_t<Tx, SEQ, true>(p, st)) return e;
+  if (!p.in_order) {
+    const dim3 slices(static_cast<unsigned>(p.nslices), static_cast<unsigned>(p.nheads),
+                      static_cast<unsigned>(p.batch));
+    if (pieces) hipLaunchKernelGGL((ssd_bwd_pass_kernel<SEQ, false>), slices, dim3(kThreads), 0, st, p);
+    else hipLaunchKernelGGL((ssd_bwd_pass_kernel<SEQ, true>), slices, dim3(kThreads), 0, st, p);
     if (hipError_t e = hipGetLastError()) return e;
-    hipLaunchKernelGGL(ssd_bwd_pass_kernel<SEQ>, slices, dim3(kThreads), 0, st, p);
   }
-  if (hipError_t e = hipGetLastError()) return e;
   if constexpr (std::is_same_v<Tx, bf16>) {
-    if (p.headdim == kSsdMaxP && p.dstate == kSsdMaxN) {
+    if (pieces) {
       if (p.z) hipLaunchKernelGGL((ssd_bwd_chunk_bf16_kernel<true, SEQ>), chunks, dim3(kThreads3), 0, st, p);
       else hipLaunchKernelGGL((ssd_bwd_chunk_bf16_kernel<false, SEQ>), chunks, dim3(kThreads3), 0, st, p);
       return hipGetLastError();
