@@ -237,6 +237,15 @@ __device__ __forceinline__ float row_allreduce16(float x) {
   return x;
 }
 
+// Sum over each aligned group of LANES (8 or 16) lanes, in every lane of it.
+template <int LANES> __device__ __forceinline__ float lanes_allreduce(float x) {
+  static_assert(LANES == 8 || LANES == 16, "half a row or a row");
+  if constexpr (LANES == 16) return row_allreduce16(x);
+  x += dpp<kQuadXor1>(x);
+  x += dpp<kQuadXor2>(x);
+  return x + dpp<kRowHalfMirror>(x);
+}
+
 // Reduce-scatter over a row: lane j of every row returns sum_{lanes of row} p[j].
 // The first two halvings split the row by DPP bank masks (a bank is 4 lanes):
 // one v_add_f32_dpp per half writes only the lanes that keep that half, so a

@@ -228,7 +228,7 @@ __device__ __forceinline__ uint32_t lane_offset(uint32_t off) {
 template <typename Tx, int V, int TPB, int NC, bool EXACT>
 __device__ __forceinline__ void map_load(raw4<Tx> (&x)[V], const TileMap<TPB, NC, EXACT>& m, const Tx* src,
                                          int64_t rs, int nvalid) {
-  static_assert(V * TPB * 4 == 64 * NC, "a thread's entries cover 64 rows");
+  static_assert(V * TPB * 4 <= 64 * NC, "a thread's entries stay within 64 rows");
   const int col = m.on ? m.col : 0;
 #pragma unroll
   for (int k = 0; k < V; ++k) {
@@ -1311,7 +1311,7 @@ __global__ void __launch_bounds__(kThreads3, 2) ssd_bwd_chunk_kernel(const SsdPa
   }
 }
 
-// K3 for bf16 storage, headdim 64 and dstate 128 (every Mamba-2 model): the same
+// K3 for bf16 storage, headdim P 32 or 64 and dstate N 64 or 128: the same
 // gradients with every product on the bf16 matrix cores in pieces
 // (ssd_pieces.h): x, B and C are one piece as stored; dY, G, dCB, dH^out and H
 // three. Waves 0-3 ("s") own 16 rows s each of d(dt x) and dB, waves 4-7 ("t")
@@ -1326,9 +1326,13 @@ __global__ void __launch_bounds__(kThreads3, 2) ssd_bwd_chunk_kernel(const SsdPa
 // all threads take c = <x, dX>, b = dt <x, W> (the sum over states of B (dt x)
 // dH^out) and dx, and one wave closes the chunk's decay gradients.
 // What bounds it: the LDS holds one workgroup per CU, so its phases (park, chunk
-// products, two state groups, output) run one after the other with two waves per
-// SIMD. Batch 4, seqlen 2048, 80 heads with z: 438 us against 971 us for the
-// float32 products below, whose matrix cores alone take 640.
+// products, state groups, output) run one after the other with two waves per
+// SIMD. The sizes are template arguments: with every loop bound known the
+// prefetched tiles stay in registers (run-time bounds spill them, and a reload
+// waits for every load in flight). Batch 4, seqlen 2048, 80 heads with z, forward
+// and backward, these products against the float32 ones below: P 64, N 128 K3
+// alone 445 against 971 us, 64 x 64 750 against 1073,
+// 32 x 128 745 against 1161, 32 x 64 577 against 833.
 constexpr int kLdT = kSsdMaxN + 16;   // rows of B and C here, read mostly transposed: eight rows on 64 banks
 
 struct BwdChunkLds {
@@ -1343,10 +1347,11 @@ struct BwdChunkLds {
 
 // The waves of one kind, s (SW) or t: the head loop. Both kinds meet at the same
 // barriers, in the same order.
-template <bool HAS_Z, bool SEQ, bool SW>
+template <bool HAS_Z, bool SEQ, int P, int N, bool SW>
 __device__ __forceinline__ void bwd_chunk_waves(const SsdParams& p, BwdChunkLds& lds) {
-  constexpr int TPB = kThreads3, P = kSsdMaxP, N = kSsdMaxN;
-  constexpr int VX = vec_x<TPB>();
+  constexpr int TPB = kThreads3, VX = Q * P / 4 / TPB;
+  constexpr int PT = P / 16, PK = P / 32;                  // headdim tiles, and products' terms over it
+  constexpr int NG = N / 64, VS = P * 64 / 4 / TPB;        // 64-state groups, and a thread's entries of one
   constexpr bool sw = SW;
   uint16_t (&s_X)[kPlaneP] = lds.X;
   uint16_t (&s_dY)[3 * kPlaneP] = lds.dY;
@@ -1369,11 +1374,12 @@ __device__ __forceinline__ void bwd_chunk_waves(const SsdParams& p, BwdChunkLds&
   const int64_t t0 = c * Q;
   const int nvalid = chunk_steps(p, t0);
   const TileMap<TPB, P, true> mp(P);
+  const TileMap<TPB, 64, true> ms(64);
   // The strip's own matrix and the other: B and C for an s-wave, C and B for a t-wave.
   const uint16_t* const s_own = (sw ? lds.B : lds.C) + own * kLdT;
   const uint16_t* const s_oth = sw ? lds.C : lds.B;
   // C at this t-wave's dC elements, (rows t = own + 4 q + e, states 16 j + r), in pairs over j
-  uint32_t cd[4][4];
+  uint32_t cd[4][N / 32];
   // Wave 4 (a t-wave: those have registers to spare) keeps the chunk's per-step
   // values, lane t step t, and closes their gradients; wave 5 sums dD.
   const bool keeper = !SW && wave == 4;
@@ -1395,7 +1401,7 @@ __device__ __forceinline__ void bwd_chunk_waves(const SsdParams& p, BwdChunkLds&
   // The next head's tiles and decays, and the next states, load into registers
   // while the current products run.
   raw4<bf16> rx[VX], rgo[VX], rz[VX], ry[VX];
-  float4 su[VX], sv[VX];
+  float4 su[VS], sv[VS];
   float rcs = 0.f, rcsl = 0.f, rdt = 0.f, rpre = 0.f;
   auto fetch = [&](int64_t h) {
     const int64_t row = chunk_row(p, b, h, c);
@@ -1416,18 +1422,18 @@ __device__ __forceinline__ void bwd_chunk_waves(const SsdParams& p, BwdChunkLds&
   };
   auto fetch_states = [&](int64_t h, int grp) {
     const int64_t sb = state_block(p, b, c, h) + 64 * grp;
-    map_load<float>(su, mp, p.dstates + sb, N, P);
-    map_load<float>(sv, mp, p.states + sb, N, P);
+    map_load<float>(su, ms, p.dstates + sb, N, P);
+    map_load<float>(sv, ms, p.states + sb, N, P);
   };
   auto park_states = [&](float& dh) {
     float v = 0.f;
 #pragma unroll
-    for (int k = 0; k < VX; ++k)
+    for (int k = 0; k < VS; ++k)
       v += fmaf(su[k].x, sv[k].x, su[k].y * sv[k].y) + fmaf(su[k].z, sv[k].z, su[k].w * sv[k].w);
     v = wave_total(v);
     dh += __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
-    map_park<float>(s_dH, kLdP, kPlaneP, mp, su, P);
-    map_park<float>(s_H, kLdP, kPlaneP, mp, sv, P);
+    map_park<float>(s_dH, kLdP, kPlaneP, ms, su, P);
+    map_park<float>(s_H, kLdP, kPlaneP, ms, sv, P);
   };
   fetch(h0);
   fetch_states(h0, 0);
@@ -1450,11 +1456,11 @@ __device__ __forceinline__ void bwd_chunk_waves(const SsdParams& p, BwdChunkLds&
 #pragma unroll
     for (int e = 0; e < 4; ++e)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
+      for (int j = 0; j < N / 32; ++j) {
         const uint16_t* at = s_own + (4 * q + e) * kLdT + 32 * j + r;
         cd[e][j] = static_cast<uint32_t>(at[0]) | (static_cast<uint32_t>(at[16]) << 16);
       }
-  v4f acc[8];   // dB (s-wave) or dC (t-wave): rows own + 4 q + e, states 16 j + r
+  v4f acc[N / 16];   // dB (s-wave) or dC (t-wave): rows own + 4 q + e, states 16 j + r
   zero(acc);
   for (int i = 0; i < p.hb; ++i) {
     int64_t h = h0 + i;
@@ -1501,21 +1507,23 @@ __device__ __forceinline__ void bwd_chunk_waves(const SsdParams& p, BwdChunkLds&
     }
     park_states(dh);
     __syncthreads();
-    fetch_states(h, 1);
+    if (NG > 1) fetch_states(h, 1);
+    else if (i + 1 < p.hb) fetch_states(h + 1, 0);
     // This wave's own x (s) or dY (t) rows, terms over p in frag_col's order.
-    Frag<1> xo[2];
-    Frag<3> yo[2];
+    Frag<1> xo[PK];
+    Frag<3> yo[PK];
 #pragma unroll
-    for (int k = 0; k < 2; ++k) {
+    for (int k = 0; k < PK; ++k) {
       if (sw) xo[k] = frag_row_as_col<1>(s_X + own * kLdP + 32 * k, kLdP, kPlaneP);
       else yo[k] = frag_row_as_col<3>(s_dY + own * kLdP + 32 * k, kLdP, kPlaneP);
     }
-    v4f dxa[4], dxs[4];   // s-wave: d(dt x) from the chunk, and from the state before w
+    v4f dxa[PT], dxs[PT];   // s-wave: d(dt x) from the chunk, and from the state before w
     zero(dxa);
     zero(dxs);
     // dG of each pair of tiles (32 of the other's steps), then G, dCB = dt_s dG
     // o M and R = dCB o C B^T, whose sum over the pair's rows is this lane's
-    // column sum (s-wave) or row sum (t-wave) of R.
+    // column sum (s-wave) or row sum (t-wave) of R. Both leave out the diagonal,
+    // whose decay is 1: it would only cancel between them, and round both.
     float rpart[4] = {0.f, 0.f, 0.f, 0.f};   // per tile: short chains of additions
     {
       const float cso = s_cs[step_own], cslo = s_csl[step_own], dto = s_dt[step_own];
@@ -1528,7 +1536,7 @@ __device__ __forceinline__ void bwd_chunk_waves(const SsdParams& p, BwdChunkLds&
           const int row0 = 32 * kt + 16 * u;
           v4f dg = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-          for (int k = 0; k < 2; ++k) {
+          for (int k = 0; k < PK; ++k) {
             if (sw) dg = mma32(frag_row_as_col<3>(s_dY + row0 * kLdP + 32 * k, kLdP, kPlaneP), xo[k], dg);
             else dg = mma32(frag_row_as_col<1>(s_X + row0 * kLdP + 32 * k, kLdP, kPlaneP), yo[k], dg);
           }
@@ -1546,7 +1554,7 @@ __device__ __forceinline__ void bwd_chunk_waves(const SsdParams& p, BwdChunkLds&
             const float m = in ? fast_exp(dc) : 0.f;
             gv[u][e] = cb[2 * kt + u][e] * m;
             dv[u][e] = dg[e] * (sw ? dto : tv[e]) * m;
-            rpart[2 * kt + u] = fmaf(dv[u][e], cb[2 * kt + u][e], rpart[2 * kt + u]);
+            rpart[2 * kt + u] = fmaf(o == step_own ? 0.f : dv[u][e], cb[2 * kt + u][e], rpart[2 * kt + u]);
           }
           __builtin_amdgcn_sched_barrier(0);
         }
@@ -1554,14 +1562,14 @@ __device__ __forceinline__ void bwd_chunk_waves(const SsdParams& p, BwdChunkLds&
         if (sw) {  // d(dt x)[s][p] += sum_t G[t][s] dY[t][p]
           const Frag<3> gf = frag_acc<3>(gv[0], gv[1]);
 #pragma unroll
-          for (int j = 0; j < 4; ++j) {
+          for (int j = 0; j < PT; ++j) {
             dxa[j] = mma32(gf, frag_col<3>(s_dY + 32 * kt * kLdP + 16 * j, kLdP, kPlaneP), dxa[j]);
             if (j & 1) __builtin_amdgcn_sched_barrier(0);  // two operands at a time: registers
           }
         }
         // dB[s][n] += sum_t dCB[t][s] C[t][n], or dC[t][n] += sum_s dCB[t][s] B[s][n]
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
+        for (int j = 0; j < N / 16; ++j) {
           acc[j] = mma32(df, frag_col<1>(s_oth + 32 * kt * kLdT + 16 * j, kLdT, 0), acc[j]);
           if (j & 1) __builtin_amdgcn_sched_barrier(0);
         }
@@ -1577,9 +1585,9 @@ __device__ __forceinline__ void bwd_chunk_waves(const SsdParams& p, BwdChunkLds&
     const float4 t4 = *reinterpret_cast<const float4*>(&s_dt[own + 4 * q]);
     const float fr[4] = {f4.x, f4.y, f4.z, f4.w};   // w_s or exp(cs_t) of the rows own + 4 q + e
     const float dtr[4] = {t4.x, t4.y, t4.z, t4.w};
-    float a_grp[4][4] = {};                         // t-wave: sum_n C[t][n] exp(cs_t) (dY H)[t][n], 32 states each
+    float a_grp[N / 32][4] = {};                    // t-wave: sum_n C[t][n] exp(cs_t) (dY H)[t][n], 32 states each
 #pragma unroll
-    for (int grp = 0; grp < 2; ++grp) {
+    for (int grp = 0; grp < NG; ++grp) {
       if (grp == 1) {
         __syncthreads();  // every wave is done reading s_dH / s_H
         park_states(dh);
@@ -1593,16 +1601,17 @@ __device__ __forceinline__ void bwd_chunk_waves(const SsdParams& p, BwdChunkLds&
           // (x dH)[s][n], and (B dH^T)[s][p] of headdim tile j
 #pragma unroll
           for (int k = 0; k < 2; ++k) {
-            tv = mma32(xo[k], frag_col<3>(s_dH + 32 * k * kLdP + 16 * j, kLdP, kPlaneP), tv);
-            dxs[j] = mma32(frag_row<1>(s_own + 64 * grp + 32 * k, kLdT, 0),
-                           frag_row<3>(s_dH + 16 * j * kLdP + 32 * k, kLdP, kPlaneP), dxs[j]);
+            if (k < PK) tv = mma32(xo[k % PK], frag_col<3>(s_dH + 32 * k * kLdP + 16 * j, kLdP, kPlaneP), tv);
+            if (j < PT)
+              dxs[j % PT] = mma32(frag_row<1>(s_own + 64 * grp + 32 * k, kLdT, 0),
+                                  frag_row<3>(s_dH + 16 * j * kLdP + 32 * k, kLdP, kPlaneP), dxs[j % PT]);
           }
 #pragma unroll
           for (int e = 0; e < 4; ++e) acc[4 * grp + j][e] = fmaf(fr[e] * dtr[e], tv[e], acc[4 * grp + j][e]);
         } else {
           // (dY H)[t][n]
 #pragma unroll
-          for (int k = 0; k < 2; ++k)
+          for (int k = 0; k < PK; ++k)
             tv = mma32(yo[k], frag_col<3>(s_H + 32 * k * kLdP + 16 * j, kLdP, kPlaneP), tv);
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
@@ -1620,7 +1629,9 @@ __device__ __forceinline__ void bwd_chunk_waves(const SsdParams& p, BwdChunkLds&
     if (!sw) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const float a = row_allreduce16((a_grp[0][e] + a_grp[1][e]) + (a_grp[2][e] + a_grp[3][e]));
+        float a = a_grp[0][e] + a_grp[1][e];
+        if constexpr (NG > 1) a += a_grp[2][e] + a_grp[3][e];
+        a = row_allreduce16(a);
         if (r == e) lds.a[own + 4 * q + e] = a;
       }
     }
@@ -1629,7 +1640,7 @@ __device__ __forceinline__ void bwd_chunk_waves(const SsdParams& p, BwdChunkLds&
 #pragma unroll
       for (int e = 0; e < 4; ++e)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (int j = 0; j < PT; ++j) {
           const int at = (own + 4 * q + e) * XP + 16 * j + r;
           const float wv = fr[e] * dxs[j][e];
           s_W[at] = wv;
@@ -1659,9 +1670,9 @@ __device__ __forceinline__ void bwd_chunk_waves(const SsdParams& p, BwdChunkLds&
           dD[u] = fmaf(yv[u], xv[u], dD[u]);
           o[u] = fmaf(Dv[u], yv[u], Xv[u] * dt);
         }
-        cr = row_allreduce16(cr);
-        br = row_allreduce16(br);
-        if (r == 0) {
+        cr = lanes_allreduce<P / 4>(cr);
+        br = lanes_allreduce<P / 4>(br);
+        if (lane % (P / 4) == 0) {
           lds.c[s] = cr;
           lds.b[s] = br * dt;
         }
@@ -1673,8 +1684,9 @@ __device__ __forceinline__ void bwd_chunk_waves(const SsdParams& p, BwdChunkLds&
       for (int u = 0; u < 4; ++u) {
         dD[u] = swap_sum<32>(dD[u], dD[u]);
         dD[u] = swap_sum<16>(dD[u], dD[u]);
+        if (P == 32) dD[u] += __shfl_xor(dD[u], 8, 64);
       }
-      if (q == 0) *reinterpret_cast<float4*>(&lds.dD[wave][4 * r]) = make_float4(dD[0], dD[1], dD[2], dD[3]);
+      if (lane < P / 4) *reinterpret_cast<float4*>(&lds.dD[wave][4 * lane]) = make_float4(dD[0], dD[1], dD[2], dD[3]);
     }
     __syncthreads();
     const int64_t prt = (b * p.nchunks + c) * H + h;
@@ -1704,7 +1716,7 @@ __device__ __forceinline__ void bwd_chunk_waves(const SsdParams& p, BwdChunkLds&
         p.dA_part[prt] = wa;
         p.dbias_part[prt] = wb;
       }
-    } else if (!SW && wave == 5) {
+    } else if (!SW && wave == 5 && lane < P) {
       float v = 0.f;
 #pragma unroll
       for (int k = 0; k < 8; ++k) v += lds.dD[k][lane];
@@ -1719,13 +1731,13 @@ __device__ __forceinline__ void bwd_chunk_waves(const SsdParams& p, BwdChunkLds&
     if (t >= nvalid) continue;
     const int64_t at = ((b * L + t0 + t) * p.nhb + blockIdx.y) * N;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) part[at + 16 * j + r] = acc[j][e];
+    for (int j = 0; j < N / 16; ++j) part[at + 16 * j + r] = acc[j][e];
   }
 }
 
-template <bool HAS_Z, bool SEQ>
+template <bool HAS_Z, bool SEQ, int P, int N>
 __global__ void __launch_bounds__(kThreads3, 2) ssd_bwd_chunk_bf16_kernel(const SsdParams p) {
-  constexpr int TPB = kThreads3, N = kSsdMaxN;
+  constexpr int TPB = kThreads3;
   __shared__ BwdChunkLds lds;
   const int64_t c = blockIdx.x, b = blockIdx.z;
   const int64_t L = p.seqlen, G = p.ngroups;
@@ -1734,7 +1746,7 @@ __global__ void __launch_bounds__(kThreads3, 2) ssd_bwd_chunk_bf16_kernel(const 
   const int nvalid = chunk_steps(p, t0);
   {
     const TileMap<TPB, N, true> mn(N);
-    constexpr int VN = vec_n<TPB>();
+    constexpr int VN = Q * N / 4 / TPB;
     const int64_t off = ((b * L + t0) * G + g) * N;
     raw4<bf16> rb[VN], rc[VN];
     map_load<bf16>(rb, mn, static_cast<const bf16*>(p.B) + off, G * N, nvalid);
@@ -1742,8 +1754,8 @@ __global__ void __launch_bounds__(kThreads3, 2) ssd_bwd_chunk_bf16_kernel(const 
     map_park<bf16>(lds.B, kLdT, 0, mn, rb, nvalid);
     map_park<bf16>(lds.C, kLdT, 0, mn, rc, nvalid);
   }
-  if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) < 4) bwd_chunk_waves<HAS_Z, SEQ, true>(p, lds);
-  else bwd_chunk_waves<HAS_Z, SEQ, false>(p, lds);
+  if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) < 4) bwd_chunk_waves<HAS_Z, SEQ, P, N, true>(p, lds);
+  else bwd_chunk_waves<HAS_Z, SEQ, P, N, false>(p, lds);
 }
 
 // Per-sequence final states of packed sequences in batch row 0 (mamba_ssm's
@@ -1874,7 +1886,8 @@ template <typename Tx, bool SEQ>
 hipError_t bwd_t(const SsdParams& p, hipStream_t st) {
   const dim3 chunks(static_cast<unsigned>(p.nchunks), static_cast<unsigned>(p.nhb), static_cast<unsigned>(p.batch));
   // The bf16 chunk-gradient kernel, which forms its own dcsL.
-  const bool pieces = std::is_same_v<Tx, bf16> && exact_shape(p);
+  const bool pieces = std::is_same_v<Tx, bf16> && (p.headdim == 64 || p.headdim == 32) &&
+                      (p.dstate == 128 || p.dstate == 64);
   if (hipError_t e = state_t<Tx, SEQ, true>(p, st)) return e;
   if (!p.in_order) {
     const dim3 slices(static_cast<unsigned>(p.nslices), static_cast<unsigned>(p.nheads),
@@ -1885,8 +1898,17 @@ hipError_t bwd_t(const SsdParams& p, hipStream_t st) {
   }
   if constexpr (std::is_same_v<Tx, bf16>) {
     if (pieces) {
-      if (p.z) hipLaunchKernelGGL((ssd_bwd_chunk_bf16_kernel<true, SEQ>), chunks, dim3(kThreads3), 0, st, p);
-      else hipLaunchKernelGGL((ssd_bwd_chunk_bf16_kernel<false, SEQ>), chunks, dim3(kThreads3), 0, st, p);
+      auto go = [&](auto hd, auto ds) {
+        if (p.z)
+          hipLaunchKernelGGL((ssd_bwd_chunk_bf16_kernel<true, SEQ, hd.value, ds.value>), chunks, dim3(kThreads3), 0, st, p);
+        else
+          hipLaunchKernelGGL((ssd_bwd_chunk_bf16_kernel<false, SEQ, hd.value, ds.value>), chunks, dim3(kThreads3), 0, st, p);
+      };
+      using n32 = std::integral_constant<int, 32>;
+      using n64 = std::integral_constant<int, 64>;
+      using n128 = std::integral_constant<int, 128>;
+      if (p.headdim == 64) p.dstate == 128 ? go(n64{}, n128{}) : go(n64{}, n64{});
+      else p.dstate == 128 ? go(n32{}, n128{}) : go(n32{}, n64{});
       return hipGetLastError();
     }
   }

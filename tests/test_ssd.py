@@ -298,7 +298,7 @@ def test_opcheck_ssd_ops():
 
 
 @pytest.mark.parametrize("seqlen", [1, 17, 63, 64, 65, 128, 200])
-@pytest.mark.parametrize("headdim,dstate", [(64, 128), (64, 64), (16, 16), (48, 80), (32, 112)])
+@pytest.mark.parametrize("headdim,dstate", [(64, 128), (64, 64), (32, 128), (32, 64), (16, 16), (48, 80), (32, 112)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 def test_tile_edges_of_every_product_form(seqlen, headdim, dstate, dtype):
     """The products in bf16 pieces (one to three per operand, by storage type)
