@@ -563,9 +563,10 @@ def ssd_bytes(shape, e):
 
 def ssd_workloads(torch, dev, stream, cpu):
     """mamba_chunk_scan_combined forward and forward+backward at the Mamba-2
-    2.7B layer shape, bf16 and fp32 storage: time, matrix-core TFLOP/s against
-    the fp32 MFMA peak (the kernels multiply in fp32 for every storage type)
-    and algorithmic GB/s against HBM."""
+    2.7B layer shape, bf16 and fp32 storage: time, the algorithm's TFLOP/s
+    against the fp32 MFMA peak (the products are float32-accurate for every
+    storage type; those formed from bf16 pieces may pass that peak) and
+    algorithmic GB/s against HBM."""
     from mamba_cpu import mamba_chunk_scan_combined
     from mamba_cpu.ops.ssd_combined import ssd_flops
 

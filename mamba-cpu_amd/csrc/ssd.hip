@@ -1,8 +1,9 @@
 // Mamba-2 SSD scan (mamba_ssm's mamba_chunk_scan_combined) on gfx950, in
 // 64-step chunks with the chunk-local contractions on the matrix cores: in bf16
 // pieces at float32 accuracy (ssd_pieces.h), or, in the chunk gradients of
-// storage and shapes other than bf16 64 x 128 and the per-sequence states, on
-// v_mfma_f32_16x16x4_f32 with the storage type widened when a tile is staged.
+// float32, fp16 and headdims and dstates other than 32, 64 and 64, 128, and in
+// the per-sequence states, on v_mfma_f32_16x16x4_f32 with the storage type
+// widened when a tile is staged.
 //
 // Per batch row b and head h (group g), with a_t = dt_t A and, inside a
 // chunk, cs_t = a_0 + ... + a_t (so cs <= 0 and decays are exp of differences):
