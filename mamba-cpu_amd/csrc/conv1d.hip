@@ -759,7 +759,10 @@ __global__ void __launch_bounds__(256) conv_bwd_vt_kernel(const ConvParams p) {
 #pragma unroll
       for (int k = 0; k < W; ++k) {
         const int a = 4 + i - (W - 1) + k;
-        dwk[k] = fmaf(same(a, 4 + i) ? dp[i] : 0.f, xv[a], dwk[k]);
+        const float sum = fmaf(same(a, 4 + i) ? dp[i] : 0.f, xv[a], dwk[k]);
+        // A step past the sequence has no term at all: its taps reach the last
+        // inputs, and 0 times an infinite one is NaN.
+        dwk[k] = !RAG || i < left ? sum : dwk[k];
       }
       float acc = 0.f;
 #pragma unroll

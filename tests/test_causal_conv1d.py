@@ -516,3 +516,30 @@ def test_time_contiguous_rows_of_any_length(seqlen, dtype, kind):
     for name, got, ref in zip(("dx", "dw", "dbias", "dinit"), grads, wg):
         scale = 1.0 if name in ("dx", "dinit") else max(1.0, float(np.abs(ref).max()))
         close(got / scale, ref / scale, gtol, 1e-4 if dtype == torch.float32 else 1e-3, name)
+
+
+@pytest.mark.parametrize("width", [2, 3, 4, 5])
+@pytest.mark.parametrize("seqlen", [9, 17, 130, 1021])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_infinite_last_inputs_reach_only_their_own_taps(width, seqlen, dtype):
+    """Without an activation dweight[k] sums dout[t] x[t - (width - 1) + k] over
+    the steps t of the sequence: an infinite last input belongs to the last tap
+    alone, a NaN before it to the last two, also where a thread's steps run past
+    the sequence (its taps there reach these inputs, but there is no such step)."""
+    torch.manual_seed(seqlen + width)
+    b, d = 2, 3
+    x = torch.randn(b, d, seqlen, device=DEV).to(dtype)
+    x[0, 1, -1] = float("inf")
+    x[0, 2, -2] = float("nan")
+    x.requires_grad_()
+    w = torch.randn(d, width, device=DEV, requires_grad=True)
+    g = torch.randn(b, d, seqlen, device=DEV).to(dtype)
+    dw, = torch.autograd.grad(causal_conv1d_fn(x, w, None), w, g)
+    with np.errstate(invalid="ignore"):
+        want = O.causal_conv1d_bwd(x, w, None, dout=g)[1]
+    dw = dw.cpu().numpy().astype(np.float64)
+    assert np.isfinite(want).sum() == want.size - 3
+    np.testing.assert_array_equal(np.isnan(dw), np.isnan(want))
+    np.testing.assert_array_equal(np.isinf(dw), np.isinf(want))
+    ok = np.isfinite(want)
+    close(torch.from_numpy(dw[ok]), want[ok], 1e-4, 1e-3, "dweight")
