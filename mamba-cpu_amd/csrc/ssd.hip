@@ -206,9 +206,9 @@ template <int TPB, int NC, bool EXACT> struct TileMap {
   static constexpr int step = TPB / (NC / 4);
   int row, col;
   bool on;   // the thread's column exists
-  __device__ __forceinline__ explicit TileMap(int ncols) {
-    row = static_cast<int>(threadIdx.x) / (NC / 4);
-    col = (static_cast<int>(threadIdx.x) % (NC / 4)) * 4;
+  __device__ __forceinline__ explicit TileMap(int ncols, int tid = threadIdx.x) {
+    row = tid / (NC / 4);
+    col = (tid % (NC / 4)) * 4;
     on = EXACT || col < ncols;
   }
 };
@@ -240,7 +240,7 @@ __device__ __forceinline__ void map_load(raw4<Tx> (&x)[V], const TileMap<TPB, NC
 
 // Those entries as bf16 pieces (ssd_pieces.h) in LDS tile s; rows from nvalid
 // on, and columns that do not exist, zero.
-template <typename Tx, int V, int TPB, int NC, bool EXACT>
+template <typename Tx, bool F32 = false, int V, int TPB, int NC, bool EXACT>
 __device__ __forceinline__ void map_park(uint16_t* s, int ld, int plane, const TileMap<TPB, NC, EXACT>& m,
                                          const raw4<Tx> (&x)[V], int nvalid) {
   constexpr int NP = kPieces<Tx>;
@@ -255,7 +255,7 @@ __device__ __forceinline__ void map_park(uint16_t* s, int ld, int plane, const T
       const float4 f = widen<Tx>(v);
       const float fv[4] = {f.x, f.y, f.z, f.w};
       uint2 o[NP];
-      split4<NP>(fv, o);
+      split4<NP, F32>(fv, o);
 #pragma unroll
       for (int i = 0; i < NP; ++i) *reinterpret_cast<uint2*>(to + i * plane) = o[i];
     }
@@ -519,11 +519,19 @@ __global__ void __launch_bounds__(kThreads) ssd_chunk_decay_kernel(const SsdPara
   p.step[row + lane] = st;
 }
 
+// The thread's index for a kernel's second pass: what the compiler derives from it
+// does not wait in registers through the first.
+__device__ __forceinline__ int second_tid() {
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));
+  return tid;
+}
+
 constexpr int kLdS = 64 + 4;          // rows of the state kernel's 64-column tiles
 constexpr int kPlaneS = Q * kLdS;
 
 // Entries of map_load's mapping, times sc[k], in three pieces.
-template <int V, int TPB, int NC, bool EXACT>
+template <bool F32, int V, int TPB, int NC, bool EXACT>
 __device__ __forceinline__ void park_scaled(uint16_t* s, const TileMap<TPB, NC, EXACT>& m, const float4 (&x)[V],
                                             const float (&sc)[V]) {
   uint16_t* at = s + m.row * kLdS + m.col;
@@ -531,11 +539,17 @@ __device__ __forceinline__ void park_scaled(uint16_t* s, const TileMap<TPB, NC, 
   for (int k = 0; k < V; ++k) {
     const float fv[4] = {x[k].x * sc[k], x[k].y * sc[k], x[k].z * sc[k], x[k].w * sc[k]};
     uint2 o[3];
-    split4<3>(fv, o);
+    split4<3, F32>(fv, o);
 #pragma unroll
     for (int i = 0; i < 3; ++i) *reinterpret_cast<uint2*>(at + k * m.step * kLdS + i * kPlaneS) = o[i];
   }
 }
+
+template <typename Tx> struct StateLds {
+  __align__(16) uint16_t A[3 * kPlaneS];             // the scaled x or dY (steps x headdim)
+  __align__(16) uint16_t B[kPieces<Tx> * kPlaneS];   // B or C (steps x 64 states)
+  float part[kThreads / 64];
+};
 
 // The states' products, in both directions and both forms. Per chunk c, for 64
 // state columns of one head,
@@ -559,14 +573,17 @@ __device__ __forceinline__ void park_scaled(uint16_t* s, const TileMap<TPB, NC, 
 // Batch 4, seqlen 2048, 80 heads, bf16 with z: forward 138 us (3.7 TB/s), backward
 // 171 us (3.9 TB/s), against 195 and 254 us on float32 tiles, the latter with
 // H_c read for dcsL.
-template <typename Tx, bool HAS_Z, bool SEQ, bool BWD, bool WALK, bool EXACT>
-__global__ void __launch_bounds__(kThreads, 3) ssd_state_kernel(const SsdParams p) {
+// F32: the pass on the float32 unit, for a workgroup whose pass in pieces ended with
+// a value that is not finite (returned: 0 if there is none; none becomes finite again
+// on the way).
+template <typename Tx, bool HAS_Z, bool SEQ, bool BWD, bool WALK, bool EXACT, bool F32>
+__device__ __forceinline__ float state_pass(const SsdParams& p, StateLds<Tx>& lds) {
   constexpr int TPB = kThreads, V = vec_x(), NX = kPieces<Tx>, NT = kSsdPassCols / 16;
   constexpr bool DCS = BWD && WALK && !(EXACT && std::is_same_v<Tx, bf16>);
-  __shared__ __align__(16) uint16_t s_A[3 * kPlaneS];    // the scaled x or dY (steps x headdim)
-  __shared__ __align__(16) uint16_t s_B[NX * kPlaneS];   // B or C (steps x 64 states)
-  __shared__ float s_part[TPB / 64];
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  uint16_t* const s_A = lds.A;
+  uint16_t* const s_B = lds.B;
+  float (&s_part)[TPB / 64] = lds.part;
+  const int tid = F32 ? second_tid() : threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, q = lane >> 4;
   const int64_t L = p.seqlen, H = p.nheads, G = p.ngroups;
   const int64_t P = EXACT ? kSsdMaxP : p.headdim, N = EXACT ? kSsdMaxN : p.dstate;
@@ -577,23 +594,13 @@ __global__ void __launch_bounds__(kThreads, 3) ssd_state_kernel(const SsdParams 
   const int64_t g = h / (H / G);
   const int ncol = static_cast<int>(N - n0 < kSsdPassCols ? N - n0 : kSsdPassCols);
   const bool act = EXACT || 16 * wave < P;
-  const TileMap<TPB, kSsdMaxP, EXACT> ma(static_cast<int>(P));
-  const TileMap<TPB, kSsdPassCols, EXACT> mb(ncol);
+  const TileMap<TPB, kSsdMaxP, EXACT> ma(static_cast<int>(P), tid);
+  const TileMap<TPB, kSsdPassCols, EXACT> mb(ncol, tid);
   // Accumulator element (j, e) of this lane: state row 16 wave + 4 q + e,
   // column n0 + 16 j + r, at offset eo + e N + 16 j of a (headdim x dstate) block.
   const uint32_t eo = static_cast<uint32_t>((16 * wave + 4 * q) * N + n0 + r);
   auto on = [&](int j) { return EXACT || (act && 16 * j < ncol); };
   v4f acc[NT];
-  zero(acc);
-  const float* init = BWD ? p.dfinal : p.init;
-  if (WALK && init != nullptr) {
-    const float* src = init + (b * H + h) * P * N;
-#pragma unroll
-    for (int j = 0; j < NT; ++j)
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (on(j)) acc[j][e] = src[eo + e * N + 16 * j];
-  }
   const Tx* const Ah = static_cast<const Tx*>(BWD ? p.dout : p.x) + b * L * H * P + h * P;
   const Tx* const Zh = static_cast<const Tx*>(p.z) + b * L * H * P + h * P;
   const Tx* const Bg = static_cast<const Tx*>(BWD ? p.C : p.B) + b * L * G * N + g * N + n0;
@@ -629,11 +636,21 @@ __global__ void __launch_bounds__(kThreads, 3) ssd_state_kernel(const SsdParams 
     }
   };
   float* const dcsl = DCS ? p.dcsL + (chunk_row(p, b, h, 0) / Q) * p.nslices + blk : nullptr;
-  int64_t pend = -1;        // chunk whose dcsL share awaits the cross-wave sum
-  float pend_decay = 0.f;
   const int64_t only = WALK ? 0 : blockIdx.x / ncb;
   const int64_t count = WALK ? p.nchunks : 1;
   auto chunk_at = [&](int64_t i) { return WALK ? (BWD ? p.nchunks - 1 - i : i) : only; };
+  int64_t pend = -1;        // chunk whose dcsL share awaits the cross-wave sum
+  float pend_decay = 0.f;
+  zero(acc);
+  const float* init = BWD ? p.dfinal : p.init;
+  if (WALK && init != nullptr) {
+    const float* src = init + (b * H + h) * P * N;
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (on(j)) acc[j][e] = src[eo + e * N + 16 * j];
+  }
   fetch(chunk_at(0));
   for (int64_t i = 0; i < count; ++i) {
     const int64_t c = chunk_at(i), t0 = c * Q;
@@ -681,8 +698,8 @@ __global__ void __launch_bounds__(kThreads, 3) ssd_state_kernel(const SsdParams 
     if constexpr (DCS)
       if (pend >= 0 && tid == 0)
         dcsl[pend * p.nslices] = pend_decay * ((s_part[0] + s_part[1]) + (s_part[2] + s_part[3]));
-    park_scaled(s_A, ma, av, sc);
-    map_park<Tx>(s_B, kLdS, kPlaneS, mb, rb, nv);
+    park_scaled<F32>(s_A, ma, av, sc);
+    map_park<Tx, F32>(s_B, kLdS, kPlaneS, mb, rb, nv);
     if (i + 1 < count) fetch(chunk_at(i + 1));
     __syncthreads();
     if constexpr (DCS) {
@@ -696,7 +713,7 @@ __global__ void __launch_bounds__(kThreads, 3) ssd_state_kernel(const SsdParams 
         const Frag<3> a = frag_col<3>(s_A + 32 * k * kLdS + 16 * wave, kLdS, kPlaneS);
 #pragma unroll
         for (int j = 0; j < NT; ++j)
-          if (on(j)) acc[j] = mma32(a, frag_col<NX>(s_B + 32 * k * kLdS + 16 * j, kLdS, kPlaneS), acc[j]);
+          if (on(j)) acc[j] = mma32<F32>(a, frag_col<NX>(s_B + 32 * k * kLdS + 16 * j, kLdS, kPlaneS), acc[j]);
       }
   }
   if constexpr (DCS) {
@@ -713,6 +730,21 @@ __global__ void __launch_bounds__(kThreads, 3) ssd_state_kernel(const SsdParams 
 #pragma unroll
         for (int e = 0; e < 4; ++e) end[eo + e * N + 16 * j] = acc[j][e];
   }
+  mma_wait(acc);
+  float spoilt = 0.f;
+#pragma unroll
+  for (int j = 0; j < NT; ++j)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) spoilt = spoil(spoilt, acc[j][e]);
+  return spoilt;
+}
+
+template <typename Tx, bool HAS_Z, bool SEQ, bool BWD, bool WALK, bool EXACT>
+__global__ void __launch_bounds__(kThreads, 3) ssd_state_kernel(const SsdParams p) {
+  __shared__ StateLds<Tx> lds;
+  const float spoilt = state_pass<Tx, HAS_Z, SEQ, BWD, WALK, EXACT, false>(p, lds);
+  if (__builtin_expect(__syncthreads_or(spoilt != 0.f), 0))
+    state_pass<Tx, HAS_Z, SEQ, BWD, WALK, EXACT, true>(p, lds);
 }
 
 // F3: the chunk's outputs, Y = (C B^T o M) (dt x) + diag(exp(cs)) C H^T + D x,
@@ -731,17 +763,91 @@ __global__ void __launch_bounds__(kThreads, 3) ssd_state_kernel(const SsdParams 
 // 32 against 48 us.
 // MN: 64 or 128, at least dstate. EXACT: headdim is 64 and dstate MN (128 in
 // every Mamba-2 model); otherwise tiles are filled up with zeros.
+// In this order everything but the last pieces of H is within an LDS instruction's
+// own 64 KB offset (with H first, float32 at 64 x 128 spills 6 registers).
+template <typename Tx> struct ScanLds {
+  __align__(16) uint16_t X[kPieces<Tx> * kPlaneP];   // x
+  __align__(16) float cs[Q], csl[Q], dt[Q], D[kSsdMaxP];
+  uint8_t first[Q];                                  // first step of each step's sequence run in the chunk
+  __align__(16) uint16_t H[3 * kPlaneN];             // B (Q x N), then each head's entering state H (P x N), then Y
+};
+
+// The same outputs one element at a time in plain float32, for a block whose products
+// in pieces left one that is not finite. C B^T and G pass through LDS over H; what
+// bounds it does not matter.
+template <typename Tx, bool HAS_Z, bool SEQ>
+__device__ __forceinline__ void chunk_scan_plain(const SsdParams& p, ScanLds<Tx>& lds) {
+  constexpr int TPB = kThreads3;
+  float* const s_CB = reinterpret_cast<float*>(lds.H);   // rows t of QP floats
+  float* const s_G = s_CB + Q * QP;
+  static_assert(2 * Q * QP * 4 <= sizeof(lds.H), "C B^T and G fit over H");
+  const int tid = second_tid();
+  const int64_t c = blockIdx.x, b = blockIdx.z;
+  const int64_t L = p.seqlen, H = p.nheads, P = p.headdim, N = p.dstate, G = p.ngroups;
+  const int64_t h0 = static_cast<int64_t>(blockIdx.y) * p.hb;
+  const int64_t t0 = c * Q, bcoff = ((b * L + t0) * G + h0 / (H / G)) * N;
+  const int nvalid = chunk_steps(p, t0);
+  const bool enter = seq_of<SEQ>(p, b, t0) == seq_of<SEQ>(p, b, t0 - 1);
+  auto first = [&](int t) { return SEQ ? lds.first[t] : 0; };
+  for (int i = tid; i < Q * Q; i += TPB) {
+    const int t = i / Q, u = i % Q;
+    float v = 0.f;
+    if (u <= t && t < nvalid)
+      for (int64_t n = 0; n < N; ++n)
+        v = fmaf(ld<Tx>(p.C, bcoff + t * G * N + n), ld<Tx>(p.B, bcoff + u * G * N + n), v);
+    s_CB[t * QP + u] = v;
+  }
+  for (int64_t h = h0; h < h0 + p.hb; ++h) {
+    const int64_t row = chunk_row(p, b, h, c), xoff = ((b * L + t0) * H + h) * P;
+    const float* st = p.states + state_block(p, b, c, h);
+    __syncthreads();  // C B^T is there, and every thread is done with the previous head's G
+    if (tid < Q) {
+      lds.cs[tid] = p.cs[row + tid];
+      lds.csl[tid] = p.cs_lo[row + tid];
+      lds.dt[tid] = p.step[row + tid];
+    }
+    __syncthreads();
+    for (int i = tid; i < Q * Q; i += TPB) {
+      const int t = i / Q, u = i % Q;
+      s_G[t * QP + u] =
+          u <= t && u >= first(t) ? s_CB[t * QP + u] * seg_exp(lds.cs, lds.csl, t, u) * lds.dt[u] : 0.f;
+    }
+    __syncthreads();
+    for (int i = tid; i < nvalid * static_cast<int>(P); i += TPB) {
+      const int t = i / static_cast<int>(P), pp = i % static_cast<int>(P);
+      float y = 0.f;
+      if (enter && first(t) == 0) {
+        for (int64_t n = 0; n < N; ++n) y = fmaf(ld<Tx>(p.C, bcoff + t * G * N + n), st[pp * N + n], y);
+        y *= fast_exp(lds.cs[t] + lds.csl[t]);
+      }
+      for (int u = first(t); u <= t; ++u) y = fmaf(s_G[t * QP + u], ld<Tx>(p.x, xoff + u * H * P + pp), y);
+      const int64_t at = xoff + t * H * P + pp;
+      if (p.D) y = fmaf(p.D[h * P + pp], ld<Tx>(p.x, at), y);
+      if (HAS_Z) {
+        if (p.ysave) mcpu::st<Tx>(p.ysave, at, y);
+        const float z = ld<Tx>(p.z, at);
+        y *= z * sigmoid(z);
+      }
+      mcpu::st<Tx>(p.out, at, y);
+    }
+  }
+}
+
 template <typename Tx, bool HAS_Z, bool SEQ, int MN, bool EXACT>
 __global__ void __launch_bounds__(kThreads3, 4) ssd_chunk_scan_kernel(const SsdParams p) {
   constexpr int TPB = kThreads3, NT = kSsdMaxP / 16;
   constexpr int NX = kPieces<Tx>, NK = MN / 64;   // k-steps of a half over the states
   constexpr int VX = vec_x<TPB>(), VN = Q * MN / 4 / TPB;
-  __shared__ __align__(16) uint16_t s_H[3 * kPlaneN];   // B (Q x N), then each head's entering state H (P x N), then Y
-  __shared__ __align__(16) uint16_t s_X[NX * kPlaneP];  // x
-  __shared__ __align__(16) float s_cs[Q], s_csl[Q], s_dt[Q], s_D[kSsdMaxP];
-  __shared__ uint8_t s_first[Q];                        // first step of each step's sequence run in the chunk
+  __shared__ ScanLds<Tx> lds;
+  uint16_t* const s_H = lds.H;
+  uint16_t* const s_X = lds.X;
+  float (&s_cs)[Q] = lds.cs;
+  float (&s_csl)[Q] = lds.csl;
+  float (&s_dt)[Q] = lds.dt;
+  float (&s_D)[kSsdMaxP] = lds.D;
+  uint8_t (&s_first)[Q] = lds.first;
   float* s_Y = reinterpret_cast<float*>(s_H);           // per half (Q x P), rows of XP floats
-  static_assert(2 * Q * XP * 4 <= sizeof(s_H), "Y fits over H");
+  static_assert(2 * Q * XP * 4 <= sizeof(lds.H), "Y fits over H");
   // x and z load once the products are done where three pieces of C leave no
   // registers for them before (spills: a reload waits for every load in flight).
   constexpr bool kLate = NX == 3;
@@ -764,6 +870,7 @@ __global__ void __launch_bounds__(kThreads3, 4) ssd_chunk_scan_kernel(const SsdP
     const int t = 16 * ws + r, n = 32 * k + 8 * q;
     return frag_mem<Tx>(static_cast<const Tx*>(p.C) + bcoff + t * G * N + n, t < nvalid && n < N);
   };
+  float spoilt = 0.f;
   Frag<NX> cf[NK];
 #pragma unroll
   for (int k = 0; k < NK; ++k) cf[k] = c_frag(NK * hf + k);
@@ -902,6 +1009,8 @@ __global__ void __launch_bounds__(kThreads3, 4) ssd_chunk_scan_kernel(const SsdP
         const float4 ya = *reinterpret_cast<const float4*>(&s_Y[to * XP + pp]);
         const float4 yb = *reinterpret_cast<const float4*>(&s_Y[(Q + to) * XP + pp]);
         float o[4] = {ya.x + yb.x, ya.y + yb.y, ya.z + yb.z, ya.w + yb.w};
+#pragma unroll
+        for (int u = 0; u < 4; ++u) spoilt = spoil(spoilt, o[u]);
         if (p.D) {
           const float4 d = *reinterpret_cast<const float4*>(&s_D[pp]), x4 = pieces4<NX>(s_X + to * kLdP + pp, kPlaneP);
           o[0] = fmaf(d.x, x4.x, o[0]);
@@ -920,6 +1029,7 @@ __global__ void __launch_bounds__(kThreads3, 4) ssd_chunk_scan_kernel(const SsdP
       }
     }
   }
+  if (__builtin_expect(__syncthreads_or(spoilt != 0.f), 0)) chunk_scan_plain<Tx, HAS_Z, SEQ>(p, lds);
 }
 
 // K2: walks the chunks from the last: dH^out_c (gradient of the state leaving
@@ -973,24 +1083,48 @@ __global__ void __launch_bounds__(kThreads) ssd_bwd_pass_kernel(const SsdParams 
 // hide each other's LDS and memory latency. Row sums over columns are
 // combined across the two halves through LDS. dB and dC of the block's heads
 // stay in accumulators and are written once, as the block's partial sums.
-template <typename Tx, bool HAS_Z, bool SEQ>
-__global__ void __launch_bounds__(kThreads3, 2) ssd_bwd_chunk_kernel(const SsdParams p) {
+// In this order the tiles that rows are read from lie within an LDS instruction's own
+// 64 KB offset of each other (with B and C first, 9 to 56 registers spill).
+struct BwdF32Lds {
+  __align__(16) float colp[16][Q];    // column sums of dG o G, per (row strip, lane quarter)
+  float dD[16][kSsdMaxP];
+  float half[2][4][Q];                // per column half: sum_s R, sum_n C.., sum_n B~.., sum_p ..
+  float cs[Q], csl[Q], dt[Q], w[Q], ecs[Q], dcs[Q];
+  float tot[8], wa[8], wb[8];
+  __align__(4) uint8_t first[Q];      // first step of each step's sequence run in the chunk
+  __align__(16) float X[Q][XP], dY[Q][XP];
+  __align__(16) float U[Q][QP];       // G = C B^T o M, then dH^out (P x 64-state group)
+  __align__(16) float V[Q][QP];       // dCB, then H (P x 64-state group), then dx
+  __align__(16) float C[Q][NP], B[Q][NP];
+};
+
+// DCS: <dH^out, exp(cs_L) H_c> comes from the states' kernels as dcsL; otherwise it is
+// formed here, from the tiles that are read anyway.
+template <typename Tx, bool HAS_Z, bool SEQ, bool DCS>
+__device__ __forceinline__ void bwd_chunk_f32(const SsdParams& p, BwdF32Lds& lds) {
   constexpr int TPB = kThreads3;
   constexpr int VX = vec_x<TPB>(), VN = vec_n<TPB>();
-  __shared__ __align__(16) float s_C[Q][NP];
-  __shared__ __align__(16) float s_B[Q][NP];
-  __shared__ __align__(16) float s_X[Q][XP];      // x
-  __shared__ __align__(16) float s_dY[Q][XP];     // dY
-  __shared__ __align__(16) float s_U[Q][QP];      // G = C B^T o M, then dH^out (P x 64-state group)
-  __shared__ __align__(16) float s_V[Q][QP];      // dCB, then H (P x 64-state group), then dx
-  __shared__ float s_colp[16][Q];                 // column sums of dG o G, per (row strip, lane quarter)
-  __shared__ float s_dD[16][kSsdMaxP];
-  __shared__ float s_half[2][4][Q];               // per column half: sum_s R, sum_n C.., sum_n B~.., sum_p ..
-  __shared__ float s_cs[Q], s_csl[Q], s_dt[Q], s_w[Q], s_ecs[Q], s_dcs[Q];
-  __shared__ float s_tot[8], s_wa[8], s_wb[8];
-  __shared__ __align__(4) uint8_t s_first[Q];     // first step of each step's sequence run in the chunk
+  float (&s_C)[Q][NP] = lds.C;
+  float (&s_B)[Q][NP] = lds.B;
+  float (&s_X)[Q][XP] = lds.X;
+  float (&s_dY)[Q][XP] = lds.dY;
+  float (&s_U)[Q][QP] = lds.U;
+  float (&s_V)[Q][QP] = lds.V;
+  float (&s_colp)[16][Q] = lds.colp;
+  float (&s_dD)[16][kSsdMaxP] = lds.dD;
+  float (&s_half)[2][4][Q] = lds.half;
+  float (&s_cs)[Q] = lds.cs;
+  float (&s_csl)[Q] = lds.csl;
+  float (&s_dt)[Q] = lds.dt;
+  float (&s_w)[Q] = lds.w;
+  float (&s_ecs)[Q] = lds.ecs;
+  float (&s_dcs)[Q] = lds.dcs;
+  float (&s_tot)[8] = lds.tot;
+  float (&s_wa)[8] = lds.wa;
+  float (&s_wb)[8] = lds.wb;
+  uint8_t (&s_first)[Q] = lds.first;
   const int64_t c = blockIdx.x, b = blockIdx.z;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = DCS ? threadIdx.x : second_tid(), lane = tid & 63, wave = tid >> 6;
   const int ws = wave & 3, hf = wave >> 2;        // row strip, column half
   const int r = lane & 15, q = lane >> 4;
   const int64_t L = p.seqlen, H = p.nheads, P = p.headdim, N = p.dstate, G = p.ngroups;
@@ -1141,12 +1275,17 @@ __global__ void __launch_bounds__(kThreads3, 2) ssd_bwd_chunk_kernel(const SsdPa
     float a_row[4] = {0.f, 0.f, 0.f, 0.f};  // sum_n C[t][n] exp(cs_t) (dY H)[t][n]
     float b_row[4] = {0.f, 0.f, 0.f, 0.f};  // sum_n w_s B[s][n] ((dt x) dH)[s][n]
     const float dt_row = s_dt[16 * ws + r], w_row = s_w[16 * ws + r];
+    float dh = 0.f;                         // this thread's part of <dH^out, H_c>
 #pragma unroll
     for (int grp = 0; grp < kSsdMaxN / 64; ++grp) {
       const int n0 = 64 * grp;
       if (n0 >= N) break;
       const int nw = static_cast<int>(N - n0 < 64 ? N - n0 : 64);
       const int nt = ntw(grp);
+      if (!DCS)
+#pragma unroll
+        for (int k = 0; k < VX; ++k)
+          dh += fmaf(su[k].x, sv[k].x, su[k].y * sv[k].y) + fmaf(su[k].z, sv[k].z, su[k].w * sv[k].w);
       __syncthreads();  // every wave is done reading s_U / s_V
       tile_store<float, VX, TPB>(&s_U[0][0], QP, su, static_cast<int>(P), nw);
       tile_store<float, VX, TPB>(&s_V[0][0], QP, sv, static_cast<int>(P), nw);
@@ -1205,6 +1344,7 @@ __global__ void __launch_bounds__(kThreads3, 2) ssd_bwd_chunk_kernel(const SsdPa
 #pragma unroll
     for (int e = 0; e < 4; ++e) bsum += b_row[e];  // this quarter's 4 rows, alike in every lane of the row
     bsum = wave_total(r == 0 ? bsum : 0.f);
+    if (!DCS) bsum = fmaf(s_ecs[Q - 1], wave_total(dh), bsum);
     if (lane == 0) s_tot[wave] = bsum;
     if (r < 4) {
       float av = 0.f, bv = 0.f, cv = 0.f;
@@ -1240,8 +1380,10 @@ __global__ void __launch_bounds__(kThreads3, 2) ssd_bwd_chunk_kernel(const SsdPa
                 (s_half[0][2][lane] + s_half[1][2][lane]);
       if (lane == Q - 1) {
         float l = ((s_tot[0] + s_tot[1]) + (s_tot[2] + s_tot[3])) + ((s_tot[4] + s_tot[5]) + (s_tot[6] + s_tot[7]));
-        const float* dl = p.dcsL + (row / Q) * p.nslices;
-        for (int64_t k = 0; k < p.nslices; ++k) l += dl[k];
+        if (DCS) {
+          const float* dl = p.dcsL + (row / Q) * p.nslices;
+          for (int64_t k = 0; k < p.nslices; ++k) l += dl[k];
+        }
         v += l;
       }
       s_dcs[lane] = wave_suffix_sum(v);
@@ -1312,6 +1454,12 @@ __global__ void __launch_bounds__(kThreads3, 2) ssd_bwd_chunk_kernel(const SsdPa
   }
 }
 
+template <typename Tx, bool HAS_Z, bool SEQ>
+__global__ void __launch_bounds__(kThreads3, 2) ssd_bwd_chunk_kernel(const SsdParams p) {
+  __shared__ BwdF32Lds lds;
+  bwd_chunk_f32<Tx, HAS_Z, SEQ, true>(p, lds);
+}
+
 // K3 for bf16 storage, headdim P 32 or 64 and dstate N 64 or 128: the same
 // gradients with every product on the bf16 matrix cores in pieces
 // (ssd_pieces.h): x, B and C are one piece as stored; dY, G, dCB, dH^out and H
@@ -1336,20 +1484,23 @@ __global__ void __launch_bounds__(kThreads3, 2) ssd_bwd_chunk_kernel(const SsdPa
 // 32 x 128 745 against 1161, 32 x 64 577 against 833.
 constexpr int kLdT = kSsdMaxN + 16;   // rows of B and C here, read mostly transposed: eight rows on 64 banks
 
+// The small arrays first: with them last, beyond an LDS instruction's own 64 KB
+// offset, P 64, N 128 spills 5 registers.
 struct BwdChunkLds {
-  __align__(16) uint16_t C[Q * kLdT], B[Q * kLdT];
-  __align__(16) uint16_t X[kPlaneP], dY[3 * kPlaneP];
-  __align__(16) uint16_t st[6 * kPlaneP];   // dH^out, then H, of a 64-state group; then dX and W
   __align__(16) float cs[Q], csl[Q], dt[Q], w[Q], ecs[Q];
   float row[Q], col[Q], a[Q], b[Q], c[Q], dh[8];
   float dD[8][kSsdMaxP];
   uint8_t first[Q], last[Q];                // ends of each step's sequence run in the chunk
+  __align__(16) uint16_t X[kPlaneP], dY[3 * kPlaneP];
+  __align__(16) uint16_t st[6 * kPlaneP];   // dH^out, then H, of a 64-state group; then dX and W
+  __align__(16) uint16_t C[Q * kLdT], B[Q * kLdT];
 };
 
 // The waves of one kind, s (SW) or t: the head loop. Both kinds meet at the same
-// barriers, in the same order.
+// barriers, in the same order. Returns 0 if the sums that every factor of the block
+// enters (C B^T, dB or dC, and the decay's gradient) are finite.
 template <bool HAS_Z, bool SEQ, int P, int N, bool SW>
-__device__ __forceinline__ void bwd_chunk_waves(const SsdParams& p, BwdChunkLds& lds) {
+__device__ __forceinline__ float bwd_chunk_waves(const SsdParams& p, BwdChunkLds& lds) {
   constexpr int TPB = kThreads3, VX = Q * P / 4 / TPB;
   constexpr int PT = P / 16, PK = P / 32;                  // headdim tiles, and products' terms over it
   constexpr int NG = N / 64, VS = P * 64 / 4 / TPB;        // 64-state groups, and a thread's entries of one
@@ -1461,6 +1612,7 @@ __device__ __forceinline__ void bwd_chunk_waves(const SsdParams& p, BwdChunkLds&
         const uint16_t* at = s_own + (4 * q + e) * kLdT + 32 * j + r;
         cd[e][j] = static_cast<uint32_t>(at[0]) | (static_cast<uint32_t>(at[16]) << 16);
       }
+  float spoilt = 0.f;
   v4f acc[N / 16];   // dB (s-wave) or dC (t-wave): rows own + 4 q + e, states 16 j + r
   zero(acc);
   for (int i = 0; i < p.hb; ++i) {
@@ -1704,6 +1856,7 @@ __device__ __forceinline__ void bwd_chunk_waves(const SsdParams& p, BwdChunkLds&
       const float last = fmaf(s_ecs[Q - 1], dhs, wave_total(bv));
       if (lane == Q - 1) v = add2(v, last, lo);
       const float da = wave_suffix_sum2(v, lo);
+      spoilt = spoil(spoilt, da);
       float ddt_raw = 0.f, dA_term = 0.f;
       if (lane < nvalid) {
         float gfac;
@@ -1734,12 +1887,24 @@ __device__ __forceinline__ void bwd_chunk_waves(const SsdParams& p, BwdChunkLds&
 #pragma unroll
     for (int j = 0; j < N / 16; ++j) part[at + 16 * j + r] = acc[j][e];
   }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) spoilt = spoil(spoilt, cb[u][e]);
+#pragma unroll
+    for (int j = 0; j < N / 16; ++j) spoilt = spoil(spoilt, acc[j][e]);
+  }
+  return spoilt;
 }
 
 template <bool HAS_Z, bool SEQ, int P, int N>
 __global__ void __launch_bounds__(kThreads3, 2) ssd_bwd_chunk_bf16_kernel(const SsdParams p) {
   constexpr int TPB = kThreads3;
-  __shared__ BwdChunkLds lds;
+  __shared__ union {
+    BwdChunkLds pieces;
+    BwdF32Lds f32;
+  } shared;
+  BwdChunkLds& lds = shared.pieces;
   const int64_t c = blockIdx.x, b = blockIdx.z;
   const int64_t L = p.seqlen, G = p.ngroups;
   const int64_t g = static_cast<int64_t>(blockIdx.y) * p.hb / (p.nheads / G);
@@ -1755,8 +1920,11 @@ __global__ void __launch_bounds__(kThreads3, 2) ssd_bwd_chunk_bf16_kernel(const 
     map_park<bf16>(lds.B, kLdT, 0, mn, rb, nvalid);
     map_park<bf16>(lds.C, kLdT, 0, mn, rc, nvalid);
   }
-  if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) < 4) bwd_chunk_waves<HAS_Z, SEQ, P, N, true>(p, lds);
-  else bwd_chunk_waves<HAS_Z, SEQ, P, N, false>(p, lds);
+  float spoilt;
+  if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) < 4) spoilt = bwd_chunk_waves<HAS_Z, SEQ, P, N, true>(p, lds);
+  else spoilt = bwd_chunk_waves<HAS_Z, SEQ, P, N, false>(p, lds);
+  if (__builtin_expect(__syncthreads_or(spoilt != 0.f), 0))
+    bwd_chunk_f32<bf16, HAS_Z, SEQ, false>(p, shared.f32);
 }
 
 // Per-sequence final states of packed sequences in batch row 0 (mamba_ssm's

@@ -9,9 +9,19 @@
 // v_mfma_f32_16x16x32_bf16 replace the eight v_mfma_f32_16x16x4_f32 of a
 // float32 product over 32 terms at half the cycles each, three where one side
 // is stored in bf16, one where both are: 2.7, 5.3 and 16 times the rate.
-// An infinite float32 operand splits into inf, NaN, NaN: products of infinities
-// are NaN where the float32 unit gives inf or NaN.
+// The split is that of bf16x3 products, Henry, Tang and Heinecke, "Leveraging
+// the bfloat16 Artificial Intelligence Datatype For Higher-Precision
+// Computations", ARITH 2019.
+// The split holds a value to 2^-24 of itself, or to 2^-134 where that is more
+// (below about 2^-110 the last pieces are bf16 subnormals).
+// A product in pieces of an infinite factor is NaN: infinity times the other's
+// pieces, of which some are zero or of the other sign. So is one of a finite value
+// above the largest bf16, whose first piece is infinite. No result that such a
+// factor enters is finite, and where a workgroup ends with one that is not, it
+// does its work again in float32 (spoil).
 #pragma once
+
+#include <type_traits>
 
 #include "mcpu_common.h"
 
@@ -23,21 +33,28 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 template <typename T> constexpr int kPieces = sizeof(T) == 4 ? 3 : (std::is_same_v<T, bf16> ? 1 : 2);
 
-// Two floats into NP pairs of bf16 (element 0 in the low half).
-template <int NP> __device__ __forceinline__ void split2(float a, float b, uint32_t (&o)[NP]) {
+// Two floats into NP pairs of bf16 (element 0 in the low half). F32: of three pieces
+// the first is held to the largest bf16, so that their sum is every finite value;
+// an infinity is then that, infinity, NaN (in two pieces infinity, NaN; whole_of).
+template <int NP, bool F32 = false> __device__ __forceinline__ void split2(float a, float b, uint32_t (&o)[NP]) {
+  const float most = __builtin_bit_cast(float, 0x7f7f0000u);
 #pragma unroll
   for (int i = 0; i < NP; ++i) {
-    o[i] = pack_bf16x2(a, b);
+    if (F32 && NP == 3 && i == 0)
+      o[i] = pack_bf16x2(__builtin_amdgcn_fmed3f(a, -most, most), __builtin_amdgcn_fmed3f(b, -most, most));
+    else
+      o[i] = pack_bf16x2(a, b);
     if (i + 1 < NP) {
       a -= __builtin_bit_cast(float, o[i] << 16);
       b -= __builtin_bit_cast(float, o[i] & 0xffff0000u);
     }
   }
 }
-template <int NP> __device__ __forceinline__ void split4(const float (&v)[4], uint2 (&o)[NP]) {
+template <int NP, bool F32 = false>
+__device__ __forceinline__ void split4(const float (&v)[4], uint2 (&o)[NP]) {
   uint32_t lo[NP], hi[NP];
-  split2<NP>(v[0], v[1], lo);
-  split2<NP>(v[2], v[3], hi);
+  split2<NP, F32>(v[0], v[1], lo);
+  split2<NP, F32>(v[2], v[3], hi);
 #pragma unroll
   for (int i = 0; i < NP; ++i) o[i] = make_uint2(lo[i], hi[i]);
 }
@@ -59,20 +76,56 @@ template <int NP> __device__ __forceinline__ Frag<NP> split8(const float (&v)[8]
   return f;
 }
 
-// c + A B over 32 terms, the small products first.
-template <int NA, int NB>
+// Element e of a lane's eight, its pieces put back together (here, not ahead of a
+// loop that the pieces do not change in: registers).
+template <int NP> __device__ __forceinline__ float whole_of(const Frag<NP>& f, int e) {
+  float v = 0.f;
+#pragma unroll
+  for (int i = 0; i < NP; ++i) {
+    uint32_t u = f.u[i][e >> 1];
+    asm volatile("" : "+v"(u));
+    const float w = __builtin_bit_cast(float, e & 1 ? u & 0xffff0000u : u << 16);
+    if (i == 0) v = w;
+    else if (i + 1 < NP || w == w) v += w;   // the last piece of an infinity is NaN
+  }
+  return v;
+}
+
+// c + A B over 32 terms: in pieces, the small products first, or with F32 on the
+// float32 unit (term 4 k + q of its step e is element e of quarter q, in A and B
+// alike).
+template <bool F32 = false, int NA, int NB>
 __device__ __forceinline__ v4f mma32(const Frag<NA>& a, const Frag<NB>& b, v4f c) {
+  if constexpr (F32) {
 #pragma unroll
-  for (int order = 2; order >= 0; --order)
+    for (int e = 0; e < 8; ++e) {
+      c = __builtin_amdgcn_mfma_f32_16x16x4f32(whole_of(a, e), whole_of(b, e), c, 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);  // one term of each lane at a time: registers
+    }
+  } else {
 #pragma unroll
-    for (int i = 0; i < NA; ++i)
+    for (int order = 2; order >= 0; --order)
 #pragma unroll
-      for (int j = 0; j < NB; ++j)
-        if (i + j == order)
-          c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a.u[i]),
-                                                      __builtin_bit_cast(bf16x8, b.u[j]), c, 0, 0, 0);
+      for (int i = 0; i < NA; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+          if (i + j == order)
+            c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a.u[i]),
+                                                        __builtin_bit_cast(bf16x8, b.u[j]), c, 0, 0, 0);
+  }
   return c;
 }
+
+// Waits for the matrix cores' last results. The compiler does so by itself, but
+// where the products sit under conditions it counts along the longest way to their
+// use, and a tile whose successors were skipped would be read before it is written.
+template <int NT> __device__ __forceinline__ void mma_wait(v4f (&acc)[NT]) {
+  static_assert(NT == 4, "tiles");
+  asm volatile("s_nop 15" : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]));
+}
+
+// sum + 0 v: no longer 0 once a v was not finite.
+__device__ __forceinline__ float spoil(float sum, float v) { return fmaf(v, 0.f, sum); }
 
 // LDS tiles of bf16 pieces: piece i of element (row, col) at i * plane + row *
 // ld + col, in rows of 64 or 128 columns padded by 16 bytes, so that the 16

@@ -320,3 +320,118 @@ def test_tile_edges_of_every_product_form(seqlen, headdim, dstate, dtype):
             wg = dict(zip(NAMES, S.ssd_bwd(**c, **kw, dout=W.float(), dfinal_states=V)))
             for name, i, atol in (("dt", 1, 1e-4), ("A", 2, 1e-3), ("D", 5, 1e-3), ("dt_bias", 7, 1e-3)):
                 assert_close_report(g[i], wg[name], 1e-3, atol, f"d{name}")
+
+
+def classes_match(got, want, name, rtol, atol):
+    """Infinities of one sign and NaN where want has them, the rest within bounds."""
+    got, want = got.detach().cpu().double().numpy(), np.asarray(want, dtype=np.float64)
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(want), err_msg=name)
+    np.testing.assert_array_equal(np.where(np.isinf(got), got, 0), np.where(np.isinf(want), want, 0), err_msg=name)
+    ok = np.isfinite(want)
+    assert_close_report(got[ok], want[ok], rtol, atol, name)
+
+
+END_SHAPES = [(1, 130, 4, 64, 1, 128), (1, 130, 4, 32, 2, 64), (1, 100, 4, 48, 1, 80), (2, 130, 8, 16, 1, 16)]
+
+
+@pytest.mark.parametrize("shape", END_SHAPES, ids=lambda s: "p{}n{}".format(s[3], s[5]))
+@pytest.mark.parametrize("chunk_pass", [1, 2], ids=["two-launch", "in-order"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_infinite_values_stay_infinite(shape, chunk_pass, dtype):
+    """One infinite value, where the recurrence gives infinities of one sign and
+    nothing else: an initial state (the outputs of its row, its final state), a
+    final state's gradient (dx of its row, dB of its column), an input x or B
+    (the final states it feeds) and an output gradient (the initial state's
+    gradient of its row). Everything that the value does not reach is finite."""
+    low = dtype != torch.float32
+    inf = float("inf")
+    otol, gtol = ((2e-2, 2e-2), (2e-2, 2e-2)) if low else ((1e-4, 1e-5), (1e-3, 1e-3))
+    for where in ("initial_states", "V", "x", "B", "W"):
+        c = case(*shape, seed=3, init=True, dtype=dtype, z=where != "V")
+        c["A"] = c["A"] * 0.05   # no decay over the sequence underflows to 0
+        gen = torch.Generator().manual_seed(1)
+        W = torch.randn(c["x"].shape, generator=gen).to(dtype)
+        V = torch.randn(c["initial_states"].shape, generator=gen)
+        if where == "initial_states":
+            c[where][0, 1, 5, 7] = inf
+        elif where == "V":
+            V[0, 1, 5, 7] = inf
+        elif where == "W":
+            W[0, 70, 1, 5] = inf
+        else:
+            c[where][(0, 70, 1, 5) if where == "x" else (0, 70, 0, 5)] = inf
+        out, fin, g = run_with(c, W, V, chunk_pass)
+        with np.errstate(invalid="ignore", over="ignore"):
+            want, want_fin = S.ssd_fwd(**c, dt_softplus=True)
+            wg = dict(zip(NAMES, S.ssd_bwd(**c, dt_softplus=True, dout=W.float(), dfinal_states=V)))
+        print(where)
+        if where in ("initial_states", "V"):
+            classes_match(out, want, "out", *otol)
+            for name in ("x", "B"):
+                if where == "V" or name == "x":
+                    classes_match(g[name], wg[name], f"d{name}", *gtol)
+        if where != "W":
+            classes_match(fin, want_fin, "final_states", *((1e-4, 1e-4) if not low else otol))
+        if where in ("V", "W"):
+            classes_match(g["initial_states"], wg["initial_states"], "dinitial_states", *gtol)
+
+
+def run_with(c, W, V, chunk_pass):
+    d = {k: None if v is None else v.to(DEV) for k, v in c.items()}
+    args = tuple(d[k] for k in NAMES) + (True, 0.0, float("inf"))
+    out, fin, saved, ysave = torch.ops.mamba_cpu.ssd_fwd(*args, True, 0, chunk_pass)
+    g = torch.ops.mamba_cpu.ssd_bwd(W.to(DEV), V.to(DEV), *args, saved, ysave, 0, chunk_pass)
+    torch.cuda.synchronize()
+    return out, fin, dict(zip(NAMES, g))
+
+
+@pytest.mark.parametrize("shape", END_SHAPES, ids=lambda s: "p{}n{}".format(s[3], s[5]))
+@pytest.mark.parametrize("chunk_pass", [1, 2], ids=["two-launch", "in-order"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("scale", [1e-36, 1e-33, 1e37])
+def test_values_near_the_ends_of_the_float32_range(shape, chunk_pass, dtype, scale):
+    """The scan is linear in (x, initial states), and its gradients in (dout,
+    dfinal_states): both scaled to the ends of float32's range, at the upper end
+    with one value of each within 2^-8 of the largest, against the oracle. Bound:
+    that of the unscaled problem, plus what a value split into bf16 pieces may be
+    off at the small end, 2^-134 (ssd_pieces.h), four times."""
+    low = dtype != torch.float32
+    c = case(*shape, seed=4, init=True, dtype=dtype, z=False, D=None)
+    c["A"] = c["A"] * 0.05   # what the decays leave stays of the inputs' size
+    gen = torch.Generator().manual_seed(1)
+    W = torch.randn(c["x"].shape, generator=gen).to(dtype)
+    V = torch.randn(c["initial_states"].shape, generator=gen)
+    big = scale > 1
+    if big:   # sums of up to 128 products stay in range
+        c["B"], c["C"] = (t * 2.0**-7 for t in (c["B"], c["C"]))
+    scale = 2.0 ** round(math.log2(scale))
+    for fwd in (True, False):
+        cc, WW, VV = dict(c), W, V
+        if fwd:
+            cc["x"], cc["initial_states"] = c["x"] * scale, c["initial_states"] * scale
+            WW, VV = W * 0, V * 0
+            if big:
+                cc["initial_states"][0, 1, 5, 7] = 3.4e38
+                if not low:
+                    cc["x"][0, 70, 1, 5] = 3.4e38
+        else:
+            WW, VV = W * scale, V * scale
+            cc["x"], cc["initial_states"] = c["x"] * 2.0**-10, c["initial_states"] * 2.0**-10
+            if big:
+                VV[0, 1, 5, 7] = 3.4e38
+                if not low:
+                    WW[0, 70, 1, 5] = 3.4e38
+        out, fin, g = run_with(cc, WW, VV, chunk_pass)
+        if fwd:
+            want, want_fin = S.ssd_fwd(**cc, dt_softplus=True)
+            pairs = [("out", out, want, 2.0**-8 if low else 1e-5), ("final_states", fin, want_fin, 1e-5)]
+        else:
+            wg = dict(zip(NAMES, S.ssd_bwd(**cc, dt_softplus=True, dout=WW.float(), dfinal_states=VV)))
+            pairs = [("dx", g["x"], wg["x"], 2.0**-8 if low else 1e-5),
+                     ("dinitial_states", g["initial_states"], wg["initial_states"], 1e-5)]
+        for name, got, ref, tol in pairs:
+            got = got.double().cpu().numpy()
+            assert np.isfinite(got).all(), name
+            err = np.linalg.norm(got / scale - ref / scale) / np.linalg.norm(ref / scale)
+            print(name, scale, err)
+            assert err <= tol + 2.0**-132 / scale, (name, err)
