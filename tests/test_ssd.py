@@ -435,3 +435,40 @@ def test_values_near_the_ends_of_the_float32_range(shape, chunk_pass, dtype, sca
             err = np.linalg.norm(got / scale - ref / scale) / np.linalg.norm(ref / scale)
             print(name, scale, err)
             assert err <= tol + 2.0**-132 / scale, (name, err)
+
+
+@pytest.mark.parametrize("headdim,dstate", [(64, 128), (64, 64), (32, 128), (32, 64)])
+@pytest.mark.parametrize("z", [False, True], ids=["noz", "z"])
+@pytest.mark.parametrize("packed", [False, True])
+def test_bf16_chunk_gradients_over_head_blocks(headdim, dstate, z, packed):
+    """The chunk gradients of bf16 storage as training runs them: several heads
+    to a workgroup (the next head's tiles prefetched, the shared tiles reused, dB
+    and dC summed over the block), several chunks and a ragged tail, both ways of
+    carrying the states, single and packed sequences. Without z (whose saved y is
+    rounded to bf16) the float32 results meet the float32 bounds; each head's dx
+    and ddt do not depend on the block."""
+    seqlen = 200
+    rng = np.random.default_rng(headdim + dstate)
+    seq = np.sort(rng.integers(0, 4, (2, seqlen)), axis=1).astype(np.int32) if packed else None
+    c = case(2, seqlen, 8, headdim, 1, dstate, seed=headdim + dstate + z, init=True, dtype=torch.bfloat16, z=z)
+    want = wg = None
+    for chunk_pass in (1, 2):
+        first = None
+        for hb in (1, 2, 4, 8):
+            out, fin, g, W, V = run_ops(c, head_block=hb, chunk_pass=chunk_pass, seq=seq)
+            if want is None:
+                want = S.ssd_fwd(**c, dt_softplus=True, seq_idx=seq)
+                wg = S.ssd_bwd(**c, dt_softplus=True, seq_idx=seq, dout=W.float(), dfinal_states=V)
+            print(f" chunk_pass {chunk_pass} head_block {hb}")
+            assert_close_report(out, want[0], 2e-2, 2e-2, "out")
+            assert_close_report(fin, want[1], 1e-4, 1e-5, "final_states")
+            for name, got, w in zip(NAMES, g, wg):
+                if c[name] is None:
+                    continue
+                tol = (2e-2, 2e-2)
+                if not z and name in ("dt", "A", "D", "dt_bias", "initial_states"):
+                    tol = (1e-3, 1e-4 if name == "dt" else 1e-3)
+                assert_close_report(got, w, *tol, f"d{name}")
+            if first is None:
+                first = (g[0], g[1])
+            assert torch.equal(g[0], first[0]) and torch.equal(g[1], first[1])
