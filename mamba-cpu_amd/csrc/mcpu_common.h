@@ -195,6 +195,7 @@ template <int CTRL> __device__ __forceinline__ float dpp(float x) {
 // lane 63 (resp. 0), whose source is outside the wave, reads 0.
 constexpr int kWaveShl1 = 0x130;
 constexpr int kWaveShr1 = 0x138;
+constexpr int kRowRor4 = 0x124;   // lane j of a row of 16 takes lane j - 4 (mod 16)
 constexpr int kRowMirror = 0x140;
 constexpr int kRowHalfMirror = 0x141;
 constexpr int kQuadXor3 = 0x1B;   // quad_perm [3,2,1,0]

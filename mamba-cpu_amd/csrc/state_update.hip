@@ -9,11 +9,13 @@
 // once the batch fills the GPU: 2 * 4 bytes per float32 state against a few
 // instructions. Two kernels:
 //   - dstate 16, 32, 64, 128 or 256 (every model's): LPR lanes per row, each
-//     moving VPL vectors of four neighbouring states, so a wave's loads and
-//     stores are whole 1 KB runs, and the <state, C> sum a DPP sum over LPR
-//     lanes. Vectors need no more than their element's alignment, so any base
-//     and strides run here.
-//     (64, 80, 64, 128) float32 states with bf16 x, B and C: 72 us, 4.7 TB/s,
+//     moving VPL vectors of four neighbouring states. 8 lanes from 32 states
+//     on: whole 128-byte lines, twice the rows to a wave that 16 lanes have for
+//     what is done once per row (128 states 70 against 75 us, 64 states 38
+//     against 52), and half the registers of 4 lanes (74 us); 256 states take
+//     16 lanes for their registers. Vectors need no more than their element's
+//     alignment, so any base and strides run here.
+//     (64, 80, 64, 128) float32 states with bf16 x, B and C: 70 us, 4.8 TB/s,
 //     against 90 us with one state per lane and load and B and C cast to
 //     float32 by two launches; (64, 5120, 16): 13.7 against 40.8 us.
 //   - any other dstate: 16 lanes per row, lane j owning states j, j + 16, ...
@@ -24,21 +26,38 @@
 
 namespace mcpu {
 
-// Sum over groups of LPR lanes (4, 8 or 16), in every lane of the group.
-template <int LPR> __device__ __forceinline__ float lanes_sum(float x) {
-  x += dpp<kQuadXor1>(x);
-  x += dpp<kQuadXor2>(x);
-  if constexpr (LPR >= 8) x += dpp<kRowHalfMirror>(x);
-  if constexpr (LPR >= 16) x += dpp<kRowMirror>(x);
-  return x;
+// The vector (of LPR in a row) that lane j moves: vector j, but with 8 lanes the upper
+// quad's in the other order, for chains_sum.
+template <int LPR> __device__ __forceinline__ int vector_of(int j) { return LPR == 8 && j >= 4 ? 11 - j : j; }
+
+// <state, C> of a row whose lane j of LPR holds states 4 (vector_of(j) + LPR v) + i, in
+// the last quad's lanes. The sum is that of one state per lane (VPL = 0 below, and the
+// fused decode steps'), so that all give the same bits: 16 chains over the states m,
+// m + 16, ..., then a tree over m. States 16 k .. 16 k + 16 are in quad k % (LPR / 4)
+// of the row, so the chains pass from quad to quad, by a mirror where the row has two;
+// what the other quads add meanwhile is not used.
+template <int LPR, int VPL>
+__device__ __forceinline__ float chains_sum(const float (&v)[4 * VPL], const float (&c)[4 * VPL]) {
+  constexpr int kNextQuad = LPR == 8 ? kRowHalfMirror : kRowRor4;
+  float acc[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int k = 0; k < VPL * LPR / 4; ++k)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int at = 4 * (4 * k / LPR) + i;
+      acc[i] = fmaf(v[at], c[at], k == 0 ? 0.f : dpp<kNextQuad>(acc[i]));
+    }
+  float sum = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+  sum += dpp<kQuadXor1>(sum);
+  return sum + dpp<kQuadXor2>(sum);
 }
 
-// VPL > 0: dstate = 4 LPR VPL, lane j of a row owning states 4 (j + LPR v) + i.
+// VPL > 0: dstate = 4 LPR VPL, lane j of a row owning states 4 (vector_of(j) + LPR v) + i.
 // VPL = 0: any dstate up to 16 SPL, LPR = 16, lane j owning states j + 16 s.
 template <typename Tx, typename Ts, typename Tb, int LPR, int VPL, int SPL>
 __global__ void __launch_bounds__(256) state_update_kernel(const StateUpdateParams p) {
   constexpr int NS = VPL > 0 ? 4 * VPL : SPL;  // states of a lane
-  const int j = threadIdx.x & (LPR - 1);
+  const int j = threadIdx.x & (LPR - 1), jv = vector_of<LPR>(j);
   const uint32_t hp = blockIdx.x * (256u / LPR) + threadIdx.x / LPR;  // row within (nheads, headdim)
   // Whole rows share every branch, so the DPP reduction below never mixes
   // live and retired lanes of one row.
@@ -66,10 +85,10 @@ __global__ void __launch_bounds__(256) state_update_kernel(const StateUpdatePara
     float sv[NS], av[NS], bv[NS], cv[NS];
     if constexpr (VPL > 0) {
 #pragma unroll
-      for (int v = 0; v < VPL; ++v) ld4_elem<Ts>(p.state, sbase + 4 * (j + LPR * v), sv + 4 * v);
+      for (int v = 0; v < VPL; ++v) ld4_elem<Ts>(p.state, sbase + 4 * (jv + LPR * v), sv + 4 * v);
 #pragma unroll
       for (int v = 0; v < VPL; ++v) {
-        const int n = 4 * (j + LPR * v);
+        const int n = 4 * (jv + LPR * v);
         ld4_elem<Tb>(p.B, Boff + n, bv + 4 * v);
         ld4_elem<Tb>(p.C, Coff + n, cv + 4 * v);
         if (p.sA[2] == 1) {
@@ -100,9 +119,7 @@ __global__ void __launch_bounds__(256) state_update_kernel(const StateUpdatePara
 #pragma unroll
       for (int i = 0; i < NS; ++i) sv[i] = fmaf(sv[i], fast_exp(dt * av[i]), dtx * bv[i]);
 #pragma unroll
-      for (int v = 0; v < VPL; ++v) st4_elem<Ts>(p.state, sbase + 4 * (j + LPR * v), sv + 4 * v);
-#pragma unroll
-      for (int i = 0; i < NS; ++i) acc = fmaf(sv[i], cv[i], acc);
+      for (int v = 0; v < VPL; ++v) st4_elem<Ts>(p.state, sbase + 4 * (jv + LPR * v), sv + 4 * v);
     } else {
 #pragma unroll
       for (int s = 0; s < NS; ++s) {
@@ -114,8 +131,10 @@ __global__ void __launch_bounds__(256) state_update_kernel(const StateUpdatePara
         }
       }
     }
-    float y = lanes_sum<LPR>(acc);
-    if (j == 0) {
+    float y;
+    if constexpr (VPL > 0) y = chains_sum<LPR, VPL>(sv, cv);
+    else y = row_allreduce16(acc);
+    if (j == (VPL > 0 ? LPR - 4 : 0)) {
       if (p.D != nullptr) y = fmaf(x, p.D[h * p.sD[0] + pp * p.sD[1]], y);
       if (p.z != nullptr) {
         const float zz = ld<Tx>(p.z, b * p.sz[0] + h * p.sz[1] + pp * p.sz[2]);
@@ -139,8 +158,8 @@ static hipError_t launch_su_types(const StateUpdateParams& p, hipStream_t st) {
   const int64_t n = p.dstate;
   if (n == 16) launch_su_one<Tx, Ts, Tb, 4, 1, 0>(p, st);
   else if (n == 32) launch_su_one<Tx, Ts, Tb, 8, 1, 0>(p, st);
-  else if (n == 64) launch_su_one<Tx, Ts, Tb, 16, 1, 0>(p, st);
-  else if (n == 128) launch_su_one<Tx, Ts, Tb, 16, 2, 0>(p, st);
+  else if (n == 64) launch_su_one<Tx, Ts, Tb, 8, 2, 0>(p, st);
+  else if (n == 128) launch_su_one<Tx, Ts, Tb, 8, 4, 0>(p, st);
   else if (n == 256) launch_su_one<Tx, Ts, Tb, 16, 4, 0>(p, st);
   else if (n < 16) launch_su_one<Tx, Ts, Tb, 16, 0, 1>(p, st);
   else if (n < 64) launch_su_one<Tx, Ts, Tb, 16, 0, 4>(p, st);

@@ -164,3 +164,27 @@ def test_state_sizes_types_and_unaligned_views(n, sdt, bcdt):
         close(out, want, 2e-5 if xdt == torch.float32 else 2.0**-8, 2e-5, "out")
         tol = 1e-5 if sdt == torch.float32 else 2.0**-8
         close(state, want_state, tol, 1e-5, "state")
+
+
+@pytest.mark.parametrize("n,rows_n", [(16, 17), (32, 33), (64, 65), (128, 129), (256, 200)])
+@pytest.mark.parametrize("xdt,sdt", [(torch.float32, torch.float32), (torch.bfloat16, torch.float32),
+                                     (torch.bfloat16, torch.bfloat16)])
+def test_vector_and_row_layouts_sum_alike(n, rows_n, xdt, sdt):
+    """<state, C> is one sum whatever layout the size takes: 16 chains over the
+    states j, j + 16, ..., added as a tree (what the fused decode steps compute,
+    so that their tokens are the unfused model's). Each vector size against a
+    neighbouring size of the one-state-per-lane layout, the extra states all
+    zero: outputs and states bitwise equal."""
+    torch.manual_seed(n)
+    b, h, p, m = 3, 4, 21, min(n, rows_n)
+    state = torch.randn(b, h, p, m, device=DEV).to(sdt)
+    x, dt, z = (f(b, h, p, device=DEV).to(xdt) for f in (torch.randn, torch.rand, torch.randn))
+    A = -torch.rand(h, p, m, device=DEV) - 0.5
+    B, C = (torch.randn(b, 2, m, device=DEV).to(xdt) for _ in range(2))
+    D, dtb = torch.randn(h, p, device=DEV), torch.rand(h, p, device=DEV) * 0.1
+    got = []
+    for size in (n, rows_n):
+        s, a, bb, c = (torch.nn.functional.pad(t, (0, size - m)) for t in (state, A, B, C))
+        out = selective_state_update(s, x, dt, a, bb, c, D, z, dtb, True)
+        got.append((out, s[..., :m]))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
