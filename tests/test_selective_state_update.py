@@ -188,3 +188,26 @@ def test_vector_and_row_layouts_sum_alike(n, rows_n, xdt, sdt):
         out = selective_state_update(s, x, dt, a, bb, c, D, z, dtb, True)
         got.append((out, s[..., :m]))
     assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
+@pytest.mark.parametrize("n", [16, 24, 64, 100, 128])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("groups", [1, 3])
+def test_float32_state_with_16_bit_inputs(n, dtype, groups):
+    """16-bit x, dt, z, B and C beside a float32 state (a 16-bit model's decode):
+    B and C are read as stored, one row per group of heads, so the state keeps the
+    float32 bound against the oracle on the same rounded inputs; the output
+    carries one rounding of its storage type."""
+    torch.manual_seed(n + groups)
+    b, h, p = 3, 6, 19
+    state = torch.randn(b, h, p, n, device=DEV)
+    x, dt, z = (f(b, h, p, device=DEV).to(dtype) for f in (torch.randn, torch.rand, torch.randn))
+    B, C = (torch.randn(b, n, groups, device=DEV).to(dtype).transpose(1, 2) for _ in range(2))
+    A = -torch.rand(h, p, n, device=DEV) - 0.5
+    D, dtb = torch.randn(h, p, device=DEV), torch.rand(h, p, device=DEV) * 0.1
+    for Bc, Cc in ((B, C), (B.contiguous(), C.contiguous())):
+        s = state.clone()
+        want, want_state = O.selective_state_update(s, x, dt, A, Bc, Cc, D, z, dtb, True)
+        out = selective_state_update(s, x, dt, A, Bc, Cc, D, z, dtb, True)
+        close(out, want, 2.0**-8 if dtype == torch.bfloat16 else 2.0**-11, 2e-5, "out")
+        close(s, want_state, 1e-5, 1e-5, "state")
