@@ -162,6 +162,7 @@ static hipError_t launch_su_types(const StateUpdateParams& p, hipStream_t st) {
   else if (n == 128) launch_su_one<Tx, Ts, Tb, 8, 4, 0>(p, st);
   else if (n == 256) launch_su_one<Tx, Ts, Tb, 16, 4, 0>(p, st);
   else if (n < 16) launch_su_one<Tx, Ts, Tb, 16, 0, 1>(p, st);
+  else if (n < 32) launch_su_one<Tx, Ts, Tb, 16, 0, 2>(p, st);
   else if (n < 64) launch_su_one<Tx, Ts, Tb, 16, 0, 4>(p, st);
   else if (n < 128) launch_su_one<Tx, Ts, Tb, 16, 0, 8>(p, st);
   else launch_su_one<Tx, Ts, Tb, 16, 0, 16>(p, st);
