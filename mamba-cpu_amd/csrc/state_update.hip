@@ -9,12 +9,12 @@
 // once the batch fills the GPU: 2 * 4 bytes per float32 state against a few
 // instructions. Two kernels:
 //   - dstate 16, 32, 64, 128 or 256 (every model's): LPR lanes per row, each
-//     moving VPL vectors of four neighbouring states. 8 lanes from 32 states
-//     on: whole 128-byte lines, twice the rows to a wave that 16 lanes have for
-//     what is done once per row (128 states 70 against 75 us, 64 states 38
-//     against 52), and half the registers of 4 lanes (74 us); 256 states take
-//     16 lanes for their registers. Vectors need no more than their element's
-//     alignment, so any base and strides run here.
+//     moving VPL vectors of four neighbouring states. The fewer lanes to a row,
+//     the more rows to a wave for what is done once per row; 4 lanes up to 64
+//     states (64 states 37 us, 8 lanes 39, 16 lanes 52; 32 states 17 against 23),
+//     8 for 128 (70 us; 16 lanes 75; 4 lanes 74, of 222 registers), 16 for 256,
+//     for their registers. Vectors need no more than their element's alignment,
+//     so any base and strides run here.
 //     (64, 80, 64, 128) float32 states with bf16 x, B and C: 70 us, 4.8 TB/s,
 //     against 90 us with one state per lane and load and B and C cast to
 //     float32 by two launches; (64, 5120, 16): 13.7 against 40.8 us.
@@ -34,18 +34,21 @@ template <int LPR> __device__ __forceinline__ int vector_of(int j) { return LPR 
 // the last quad's lanes. The sum is that of one state per lane (VPL = 0 below, and the
 // fused decode steps'), so that all give the same bits: 16 chains over the states m,
 // m + 16, ..., then a tree over m. States 16 k .. 16 k + 16 are in quad k % (LPR / 4)
-// of the row, so the chains pass from quad to quad, by a mirror where the row has two;
-// what the other quads add meanwhile is not used.
+// of the row, so the chains pass from quad to quad where the row has more than one, by
+// a mirror where it has two; what the other quads add meanwhile is not used.
 template <int LPR, int VPL>
 __device__ __forceinline__ float chains_sum(const float (&v)[4 * VPL], const float (&c)[4 * VPL]) {
-  constexpr int kNextQuad = LPR == 8 ? kRowHalfMirror : kRowRor4;
+  auto from_quad = [](float x) {
+    if constexpr (LPR == 4) return x;
+    else return dpp<LPR == 8 ? kRowHalfMirror : kRowRor4>(x);
+  };
   float acc[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int k = 0; k < VPL * LPR / 4; ++k)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int at = 4 * (4 * k / LPR) + i;
-      acc[i] = fmaf(v[at], c[at], k == 0 ? 0.f : dpp<kNextQuad>(acc[i]));
+      acc[i] = fmaf(v[at], c[at], k == 0 ? 0.f : from_quad(acc[i]));
     }
   float sum = (acc[0] + acc[1]) + (acc[2] + acc[3]);
   sum += dpp<kQuadXor1>(sum);
@@ -157,8 +160,8 @@ template <typename Tx, typename Ts, typename Tb>
 static hipError_t launch_su_types(const StateUpdateParams& p, hipStream_t st) {
   const int64_t n = p.dstate;
   if (n == 16) launch_su_one<Tx, Ts, Tb, 4, 1, 0>(p, st);
-  else if (n == 32) launch_su_one<Tx, Ts, Tb, 8, 1, 0>(p, st);
-  else if (n == 64) launch_su_one<Tx, Ts, Tb, 8, 2, 0>(p, st);
+  else if (n == 32) launch_su_one<Tx, Ts, Tb, 4, 2, 0>(p, st);
+  else if (n == 64) launch_su_one<Tx, Ts, Tb, 4, 4, 0>(p, st);
   else if (n == 128) launch_su_one<Tx, Ts, Tb, 8, 4, 0>(p, st);
   else if (n == 256) launch_su_one<Tx, Ts, Tb, 16, 4, 0>(p, st);
   else if (n < 16) launch_su_one<Tx, Ts, Tb, 16, 0, 1>(p, st);
