@@ -284,8 +284,8 @@ typedef struct mcpu_state_update_args {
   const void* x;           /* (batch, nheads, headdim), dtype */
   const void* dt;          /* (batch, nheads, headdim), dtype */
   const float* A;          /* (nheads, headdim, dstate) contiguous */
-  const void* B;           /* (batch, ngroups, dstate), bc_dtype, unit dstate stride */
-  const void* C;           /* (batch, ngroups, dstate), bc_dtype, unit dstate stride */
+  const void* B;           /* (batch, ngroups, dstate), float32 (..._bc: bc_dtype), unit dstate stride */
+  const void* C;           /* (batch, ngroups, dstate), float32 (..._bc: bc_dtype), unit dstate stride */
   const float* D;          /* (nheads, headdim), optional */
   const void* z;           /* (batch, nheads, headdim), dtype, optional */
   const float* dt_bias;    /* (nheads, headdim), optional */
@@ -294,7 +294,7 @@ typedef struct mcpu_state_update_args {
   int32_t dt_softplus;
   int32_t dtype;           /* storage type of x, dt, z, out */
   int32_t state_dtype;     /* storage type of state */
-  int32_t bc_dtype;        /* storage type of B and C: MCPU_F32 (0) or dtype */
+  int32_t _pad;
   int64_t state_stride[3]; /* over (batch, head, headdim) */
   int64_t x_stride[3];
   int64_t dt_stride[3];
@@ -322,6 +322,9 @@ typedef struct mcpu_state_update_args {
 } mcpu_state_update_args;
 
 int mcpu_selective_state_update(const mcpu_state_update_args* a, void* stream);
+
+/* The same with B and C stored as bc_dtype: MCPU_F32 or the value of dtype. */
+int mcpu_selective_state_update_bc(const mcpu_state_update_args* a, int32_t bc_dtype, void* stream);
 
 /* ------------------------------------------------------------------------ */
 /* Mamba-2 SSD scan.                                                         */

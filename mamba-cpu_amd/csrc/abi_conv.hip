@@ -264,6 +264,10 @@ extern "C" int mcpu_causal_conv1d_update(const mcpu_conv_update_args* a, void* s
 }
 
 extern "C" int mcpu_selective_state_update(const mcpu_state_update_args* a, void* stream) {
+  return mcpu_selective_state_update_bc(a, MCPU_F32, stream);
+}
+
+extern "C" int mcpu_selective_state_update_bc(const mcpu_state_update_args* a, int32_t bc_dtype, void* stream) {
   clear_error();
   if (a == nullptr) return fail(MCPU_ERR_INVALID, "selective_state_update: null argument block");
   if (a->batch < 0 || a->nheads < 0 || a->headdim < 0)
@@ -277,7 +281,7 @@ extern "C" int mcpu_selective_state_update(const mcpu_state_update_args* a, void
     return fail(MCPU_ERR_UNSUPPORTED, "selective_state_update: dstate must be in [1, 256]");
   if (a->ngroups < 1 || (a->nheads > 0 && a->nheads % a->ngroups != 0))
     return fail(MCPU_ERR_INVALID, "selective_state_update: nheads must be divisible by ngroups");
-  if (!valid_dtype(a->dtype) || !valid_dtype(a->state_dtype) || (a->bc_dtype != MCPU_F32 && a->bc_dtype != a->dtype))
+  if (!valid_dtype(a->dtype) || !valid_dtype(a->state_dtype) || (bc_dtype != MCPU_F32 && bc_dtype != a->dtype))
     return fail(MCPU_ERR_INVALID, "selective_state_update: bad dtype");
   if (a->nheads * a->headdim > 0xffff0000ll)
     return fail(MCPU_ERR_UNSUPPORTED, "selective_state_update: nheads * headdim too large");
@@ -301,7 +305,7 @@ extern "C" int mcpu_selective_state_update(const mcpu_state_update_args* a, void
   p.headdim = a->headdim;
   p.dstate = a->dstate;
   p.ngroups = a->ngroups;
-  p.bc_dtype = a->bc_dtype;
+  p.bc_dtype = bc_dtype;
   for (int i = 0; i < 3; ++i) {
     p.sst[i] = a->state_stride[i];
     p.sx[i] = a->x_stride[i];

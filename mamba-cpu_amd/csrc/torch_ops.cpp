@@ -1008,7 +1008,6 @@ Tensor selective_state_update(Tensor& state, const Tensor& x, const Tensor& dt, 
   a.A = static_cast<const float*>(A.data_ptr());
   a.B = B.data_ptr();
   a.C = C.data_ptr();
-  a.bc_dtype = dtype_tag(B.scalar_type());
   a.D = fptr(D);
   a.z = ptr(z);
   a.dt_bias = fptr(dt_bias);
@@ -1049,7 +1048,7 @@ Tensor selective_state_update(Tensor& state, const Tensor& x, const Tensor& dt, 
   };
   s2(a.D_stride, D);
   s2(a.dt_bias_stride, dt_bias);
-  check_rc(mcpu_selective_state_update(&a, stream_of(x)), name);
+  check_rc(mcpu_selective_state_update_bc(&a, dtype_tag(B.scalar_type()), stream_of(x)), name);
   return out;
 }
 

@@ -94,7 +94,7 @@ class StateUpdateArgs(ctypes.Structure):
         ("state", _P), ("x", _P), ("dt", _P), ("A", _P), ("B", _P), ("C", _P), ("D", _P),
         ("z", _P), ("dt_bias", _P), ("out", _P),
         ("batch", _I64), ("nheads", _I64), ("headdim", _I64), ("dstate", _I64), ("ngroups", _I64),
-        ("dt_softplus", _I32), ("dtype", _I32), ("state_dtype", _I32), ("bc_dtype", _I32),
+        ("dt_softplus", _I32), ("dtype", _I32), ("state_dtype", _I32), ("_pad", _I32),
         ("state_stride", _S3), ("x_stride", _S3), ("dt_stride", _S3), ("z_stride", _S3),
         ("B_stride", _S2), ("C_stride", _S2),
         ("state_batch_indices", _P), ("state_batch", _I64),
@@ -183,6 +183,8 @@ lib.mcpu_causal_conv1d_update.argtypes = [_ARGP["conv_update"], _P]
 lib.mcpu_causal_conv1d_update.restype = ctypes.c_int
 lib.mcpu_selective_state_update.argtypes = [_ARGP["state_update"], _P]
 lib.mcpu_selective_state_update.restype = ctypes.c_int
+lib.mcpu_selective_state_update_bc.argtypes = [_ARGP["state_update"], _I32, _P]
+lib.mcpu_selective_state_update_bc.restype = ctypes.c_int
 lib.mcpu_ssd_saved_size.argtypes = [_ARGP["ssd"]]
 lib.mcpu_ssd_saved_size.restype = ctypes.c_size_t
 lib.mcpu_ssd_fwd.argtypes = [_ARGP["ssd"], _P, ctypes.c_size_t, _P]

@@ -710,3 +710,19 @@ def test_fused_step_lds_rule_is_the_librarys():
             assert dec._fused_lds_fits(batch, dm, di, gated=True) == takes, ("mamba2", batch, dm)
     assert seen == {True, False}
     assert dec._fused_lds_fits(8, 2048, 4096) and not dec._fused_lds_fits(5, 2560, 5120)
+
+
+def test_state_update_ignores_its_padding():
+    """A caller that leaves the padding of mcpu_state_update_args unset reads B
+    and C as float32 all the same (an empty batch: no device work)."""
+    from mamba_cpu import _C
+
+    s = _C.StateUpdateArgs()
+    s.nheads, s.headdim, s.dstate, s.ngroups = 2, 4, 16, 1
+    s.dtype = _C.MCPU_BF16
+    s._pad = 0x55AA55AA
+    rc, msg = _rc(_C.lib.mcpu_selective_state_update, ctypes.byref(s), None)
+    assert rc != _C.MCPU_ERR_INVALID, msg
+    for bc, ok in ((_C.MCPU_F32, True), (_C.MCPU_BF16, True), (_C.MCPU_F16, False), (7, False)):
+        rc, msg = _rc(_C.lib.mcpu_selective_state_update_bc, ctypes.byref(s), bc, None)
+        assert (rc != _C.MCPU_ERR_INVALID) == ok, (bc, msg)
