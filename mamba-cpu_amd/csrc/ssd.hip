@@ -1803,8 +1803,8 @@ __device__ __forceinline__ float bwd_chunk_waves(const SsdParams& p, BwdChunkLds
     // dx = dt dX + D dY; c = <x, dX>, b = dt <x, W> per row; dD over the rows
     {
       float dD[4] = {0.f, 0.f, 0.f, 0.f};
-      const float4 D4 = p.D ? *reinterpret_cast<const float4*>(p.D + h * P + mp.col) : make_float4(0.f, 0.f, 0.f, 0.f);
-      const float Dv[4] = {D4.x, D4.y, D4.z, D4.w};
+      float Dv[4] = {0.f, 0.f, 0.f, 0.f};
+      if (p.D) ld4_elem<float>(p.D, h * P + mp.col, Dv);   // D may start at any element
 #pragma unroll
       for (int k = 0; k < VX; ++k) {
         const int s = mp.row + k * mp.step;

@@ -472,3 +472,24 @@ def test_bf16_chunk_gradients_over_head_blocks(headdim, dstate, z, packed):
             if first is None:
                 first = (g[0], g[1])
             assert torch.equal(g[0], first[0]) and torch.equal(g[1], first[1])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("headdim,dstate", [(64, 128), (32, 64), (48, 80)])
+def test_parameters_may_start_at_any_element(dtype, headdim, dstate):
+    """A, D and dt_bias one element into their buffers give what aligned ones give,
+    bit for bit."""
+    c = case(1, 130, 4, headdim, 1, dstate, seed=headdim, dtype=dtype)
+    gen = torch.Generator().manual_seed(1)
+    W = torch.randn(c["x"].shape, generator=gen).to(dtype)
+    V = torch.randn(1, 4, headdim, dstate, generator=gen)
+    off = dict(c)
+    for k in ("A", "D", "dt_bias"):
+        buf = torch.zeros(c[k].numel() + 1, device=DEV)
+        off[k] = buf[1:].view(c[k].shape)
+        off[k].copy_(c[k])
+        assert off[k].data_ptr() % 16 == 4
+    (out, fin, g), (out1, fin1, g1) = run_with(c, W, V, 1), run_with(off, W, V, 1)
+    assert torch.equal(out, out1) and torch.equal(fin, fin1)
+    for k, v in g.items():
+        assert (v is None and g1[k] is None) or torch.equal(v, g1[k]), k
