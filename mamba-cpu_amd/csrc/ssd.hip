@@ -567,8 +567,8 @@ template <typename Tx> struct StateLds {
 //     running decays. Grid (nchunks x column blocks, nheads, batch).
 // EXACT: headdim 64, dstate 128; otherwise tiles are filled up with zeros. The
 // next chunk's tiles load while the current products run.
-// DCS (backward walk): also <X, exp(cs_L) H_c> over its columns to dcsL, which the
-// bf16 chunk-gradient kernel (EXACT, bf16) forms itself from tiles it reads anyway.
+// DCS (backward walk): also <X, exp(cs_L) H_c> over its columns to dcsL, for the
+// float32 chunk gradients; the bf16 ones form it from tiles they read anyway.
 // What bounds it is memory: x (or dout and z) once per column block, X out.
 // Batch 4, seqlen 2048, 80 heads, bf16 with z: forward 138 us (3.7 TB/s), backward
 // 171 us (3.9 TB/s), against 195 and 254 us on float32 tiles, the latter with
@@ -576,10 +576,10 @@ template <typename Tx> struct StateLds {
 // F32: the pass on the float32 unit, for a workgroup whose pass in pieces ended with
 // a value that is not finite (returned: 0 if there is none; none becomes finite again
 // on the way).
-template <typename Tx, bool HAS_Z, bool SEQ, bool BWD, bool WALK, bool EXACT, bool F32>
+template <typename Tx, bool HAS_Z, bool SEQ, bool BWD, bool WALK, bool EXACT, bool DCS, bool F32>
 __device__ __forceinline__ float state_pass(const SsdParams& p, StateLds<Tx>& lds) {
   constexpr int TPB = kThreads, V = vec_x(), NX = kPieces<Tx>, NT = kSsdPassCols / 16;
-  constexpr bool DCS = BWD && WALK && !(EXACT && std::is_same_v<Tx, bf16>);
+  static_assert(!DCS || (BWD && WALK), "dcsL belongs to the backward walk");
   uint16_t* const s_A = lds.A;
   uint16_t* const s_B = lds.B;
   float (&s_part)[TPB / 64] = lds.part;
@@ -739,12 +739,12 @@ __device__ __forceinline__ float state_pass(const SsdParams& p, StateLds<Tx>& ld
   return spoilt;
 }
 
-template <typename Tx, bool HAS_Z, bool SEQ, bool BWD, bool WALK, bool EXACT>
+template <typename Tx, bool HAS_Z, bool SEQ, bool BWD, bool WALK, bool EXACT, bool DCS>
 __global__ void __launch_bounds__(kThreads, 3) ssd_state_kernel(const SsdParams p) {
   __shared__ StateLds<Tx> lds;
-  const float spoilt = state_pass<Tx, HAS_Z, SEQ, BWD, WALK, EXACT, false>(p, lds);
+  const float spoilt = state_pass<Tx, HAS_Z, SEQ, BWD, WALK, EXACT, DCS, false>(p, lds);
   if (__builtin_expect(__syncthreads_or(spoilt != 0.f), 0))
-    state_pass<Tx, HAS_Z, SEQ, BWD, WALK, EXACT, true>(p, lds);
+    state_pass<Tx, HAS_Z, SEQ, BWD, WALK, EXACT, DCS, true>(p, lds);
 }
 
 // F3: the chunk's outputs, Y = (C B^T o M) (dt x) + diag(exp(cs)) C H^T + D x,
@@ -1997,6 +1997,11 @@ __global__ void __launch_bounds__(kThreads) ssd_varlen_state_kernel(const SsdPar
 
 namespace {
 
+// Whether the chunk gradients run in bf16 pieces (and form their own dcsL).
+template <typename Tx> bool bwd_in_pieces(const SsdParams& p) {
+  return std::is_same_v<Tx, bf16> && (p.headdim == 64 || p.headdim == 32) && (p.dstate == 128 || p.dstate == 64);
+}
+
 bool exact_shape(const SsdParams& p) { return p.headdim == kSsdMaxP && p.dstate == kSsdMaxN; }
 
 // The states' products of one direction: walking the chunks (in order), or per
@@ -2006,13 +2011,21 @@ hipError_t state_t(const SsdParams& p, hipStream_t st) {
   const int64_t ncb = (p.dstate + kSsdPassCols - 1) / kSsdPassCols;
   const dim3 grid(static_cast<unsigned>(p.in_order ? ncb : ncb * p.nchunks), static_cast<unsigned>(p.nheads),
                   static_cast<unsigned>(p.batch));
-  auto go = [&](auto z, auto walk, auto exact) {
-    hipLaunchKernelGGL((ssd_state_kernel<Tx, z.value, SEQ, BWD, walk.value, exact.value>), grid, dim3(kThreads), 0,
-                       st, p);
+  auto go = [&](auto z, auto walk, auto exact, auto dcs) {
+    hipLaunchKernelGGL((ssd_state_kernel<Tx, z.value, SEQ, BWD, walk.value, exact.value, dcs.value>), grid,
+                       dim3(kThreads), 0, st, p);
+  };
+  auto shape = [&](auto z, auto walk, auto dcs) {
+    constexpr bool never = std::is_same_v<Tx, bf16> && dcs.value;   // 64 x 128 runs in pieces
+    if (!exact_shape(p)) go(z, walk, std::false_type{}, dcs);
+    else if constexpr (!never) go(z, walk, std::true_type{}, dcs);
   };
   auto form = [&](auto z, auto walk) {
-    if (exact_shape(p)) go(z, walk, std::true_type{});
-    else go(z, walk, std::false_type{});
+    if constexpr (BWD && walk.value) {
+      if (!bwd_in_pieces<Tx>(p)) return shape(z, walk, std::true_type{});
+      if constexpr (!std::is_same_v<Tx, bf16>) return;
+    }
+    shape(z, walk, std::false_type{});
   };
   auto gate = [&](auto z) {
     if (p.in_order) form(z, std::true_type{});
@@ -2054,9 +2067,7 @@ hipError_t fwd_t(const SsdParams& p, hipStream_t st) {
 template <typename Tx, bool SEQ>
 hipError_t bwd_t(const SsdParams& p, hipStream_t st) {
   const dim3 chunks(static_cast<unsigned>(p.nchunks), static_cast<unsigned>(p.nhb), static_cast<unsigned>(p.batch));
-  // The bf16 chunk-gradient kernel, which forms its own dcsL.
-  const bool pieces = std::is_same_v<Tx, bf16> && (p.headdim == 64 || p.headdim == 32) &&
-                      (p.dstate == 128 || p.dstate == 64);
+  const bool pieces = bwd_in_pieces<Tx>(p);
   if (hipError_t e = state_t<Tx, SEQ, true>(p, st)) return e;
   if (!p.in_order) {
     const dim3 slices(static_cast<unsigned>(p.nslices), static_cast<unsigned>(p.nheads),
