@@ -562,7 +562,8 @@ __global__ void __launch_bounds__(kThreads) gemv_kernel(const MixerParams p, con
 // softplus + selective state update + D skip + silu(z) gate. 16 lanes per
 // channel (state n = lane + 16 s), 64 channels per workgroup; grid
 // (ceil(d_inner / 64), batch). The arithmetic of each channel is the
-// selective state update kernel's.
+// selective state update kernel's, its sums included (chains_sum), so that both give
+// the same bits.
 template <typename T, typename Ts, int SPL, bool FUSED>
 __global__ void __launch_bounds__(kSsmThreads) block_ssm_kernel(const MixerParams p) {
   __shared__ float s_red[kSsmThreads];
@@ -669,8 +670,8 @@ __global__ void __launch_bounds__(kSsmThreads) block_ssm_kernel(const MixerParam
 }
 
 // Mamba-2 step, launch 2: the selective state update of every (head,
-// channel) row, in the state update kernel's layout and arithmetic (16 lanes
-// per row, states n = lane + 16 s, the same fixed-order sums):
+// channel) row, in the state update kernel's arithmetic and fixed-order sums
+// (chains_sum there; here 16 lanes per row, states n = lane + 16 s):
 //   dt = softplus(dt_raw[h] + dt_bias[h]),
 //   state = state exp(dt A[h]) + dt x B_g,   y = <state, C_g> + D[h] x,
 // y rounded to T. x, B and C are the conv outputs (xc: x | B | C of every

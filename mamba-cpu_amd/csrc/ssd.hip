@@ -282,26 +282,25 @@ __device__ __forceinline__ void stage(float* s, int ld, const Tx* src, int64_t r
   tile_store<Tx, V, TPB>(s, ld, x, nrows, ncols, scale);
 }
 
-// The dout, z and ysave tiles of one head's chunk (x layout from `off`, z and
-// ysave only when HAS_Z and, for ysave, want_y), for a workgroup of TPB threads.
+// The dout tile of one head's chunk, and with HAS_Z its z and ysave (x layout from
+// `off`), for a workgroup of TPB threads.
 template <typename Tx, bool HAS_Z, int TPB = kThreads>
 struct DyTiles {
   static constexpr int V = vec_x<TPB>();
   raw4<Tx> go[V], zz[V], yy[V];
 
-  __device__ __forceinline__ void load(const SsdParams& p, int64_t off, int64_t rs, int nvalid, int ncols,
-                                       bool want_y) {
+  __device__ __forceinline__ void load(const SsdParams& p, int64_t off, int64_t rs, int nvalid, int ncols) {
     tile_load<Tx, V, TPB>(go, static_cast<const Tx*>(p.dout) + off, rs, Q, nvalid, ncols);
     if (HAS_Z) {
       tile_load<Tx, V, TPB>(zz, static_cast<const Tx*>(p.z) + off, rs, Q, nvalid, ncols);
-      if (want_y) tile_load<Tx, V, TPB>(yy, static_cast<const Tx*>(p.ysave) + off, rs, Q, nvalid, ncols);
+      tile_load<Tx, V, TPB>(yy, static_cast<const Tx*>(p.ysave) + off, rs, Q, nvalid, ncols);
     }
   }
 
-  // LDS tile of dY = dout silu(z) (dout without z); dz = dout y silu'(z)
-  // written to rows below nvalid when write_dz.
+  // LDS tile of dY = dout silu(z) (dout without z); dz = dout y silu'(z) to rows
+  // below nvalid.
   __device__ __forceinline__ void store(float* s, int ld, const SsdParams& p, int64_t off, int64_t rs, int nvalid,
-                                        int ncols, bool write_dz) const {
+                                        int ncols) const {
     const int nv = ncols >> 2, total = Q * nv;
     const float inv = 1.0f / static_cast<float>(nv);
 #pragma unroll
@@ -311,14 +310,14 @@ struct DyTiles {
       const int r = tile_row(v, inv);
       const int c = (v - r * nv) << 2;
       float4 dz = make_float4(0.f, 0.f, 0.f, 0.f);
-      const float4 dy = dy_of(k, write_dz ? &dz : nullptr);
-      if (HAS_Z && write_dz && r < nvalid) st4<Tx>(static_cast<Tx*>(p.dz) + off + r * rs + c, dz);
+      const float4 dy = dy_of(k, dz);
+      if (HAS_Z && r < nvalid) st4<Tx>(static_cast<Tx*>(p.dz) + off + r * rs + c, dz);
       *reinterpret_cast<float4*>(s + r * ld + c) = dy;
     }
   }
 
-  // dY of float4 number k, and dz into *dzp when given (HAS_Z).
-  __device__ __forceinline__ float4 dy_of(int k, float4* dzp) const {
+  // dY of float4 number k, and with HAS_Z its dz.
+  __device__ __forceinline__ float4 dy_of(int k, float4& dz) const {
     const float4 g4 = widen<Tx>(go[k]);
     if (!HAS_Z) return g4;
     const float4 z4 = widen<Tx>(zz[k]);
@@ -329,14 +328,12 @@ struct DyTiles {
       sg[u] = sigmoid(zx[u]);
       d[u] = gx[u] * zx[u] * sg[u];
     }
-    if (dzp) {
-      const float4 y4 = widen<Tx>(yy[k]);
-      const float yv[4] = {y4.x, y4.y, y4.z, y4.w};
-      float dzv[4];
+    const float4 y4 = widen<Tx>(yy[k]);
+    const float yv[4] = {y4.x, y4.y, y4.z, y4.w};
+    float dzv[4];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) dzv[u] = gx[u] * yv[u] * sg[u] * (1.f + zx[u] * (1.f - sg[u]));
-      *dzp = make_float4(dzv[0], dzv[1], dzv[2], dzv[3]);
-    }
+    for (int u = 0; u < 4; ++u) dzv[u] = gx[u] * yv[u] * sg[u] * (1.f + zx[u] * (1.f - sg[u]));
+    dz = make_float4(dzv[0], dzv[1], dzv[2], dzv[3]);
     return make_float4(d[0], d[1], d[2], d[3]);
   }
 };
@@ -1185,7 +1182,7 @@ __device__ __forceinline__ void bwd_chunk_f32(const SsdParams& p, BwdF32Lds& lds
       rcslL = p.cs_lo[row + Q - 1];
     }
     tile_load<Tx, VX, TPB>(rx, static_cast<const Tx*>(p.x) + xoff, H * P, Q, nvalid, static_cast<int>(P));
-    rdy.load(p, xoff, H * P, nvalid, static_cast<int>(P), true);
+    rdy.load(p, xoff, H * P, nvalid, static_cast<int>(P));
   };
   fetch(h0);
   for (int i = 0; i < p.hb; ++i) {
@@ -1202,7 +1199,7 @@ __device__ __forceinline__ void bwd_chunk_f32(const SsdParams& p, BwdF32Lds& lds
       s_ecs[tid] = from ? fast_exp(rcs + rcsl) : 0.f;
     }
     tile_store<Tx, VX, TPB>(&s_X[0][0], XP, rx, Q, static_cast<int>(P));
-    rdy.store(&s_dY[0][0], XP, p, xoff, H * P, nvalid, static_cast<int>(P), true);
+    rdy.store(&s_dY[0][0], XP, p, xoff, H * P, nvalid, static_cast<int>(P));
     __syncthreads();
     if (i + 1 < p.hb) fetch(h + 1);
     // dGraw = dY x^T (rows t of this strip, this half's columns s); with M and
@@ -1496,8 +1493,10 @@ struct BwdChunkLds {
   __align__(16) uint16_t C[Q * kLdT], B[Q * kLdT];
 };
 
-// The waves of one kind, s (SW) or t: the head loop. Both kinds meet at the same
-// barriers, in the same order. Returns 0 if the sums that every factor of the block
+// The waves of one kind, s (SW) or t: the head loop. The two kinds reach their
+// barriers at different places in the code: the hardware counts arrivals, so both must
+// pass the same number of them, in the same order, and nothing here may leave the loop
+// early or skip one. Returns 0 if the sums that every factor of the block
 // enters (C B^T, dB or dC, and the decay's gradient) are finite.
 template <bool HAS_Z, bool SEQ, int P, int N, bool SW>
 __device__ __forceinline__ float bwd_chunk_waves(const SsdParams& p, BwdChunkLds& lds) {
