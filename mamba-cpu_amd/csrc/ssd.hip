@@ -1477,8 +1477,8 @@ __global__ void __launch_bounds__(kThreads3, 2) ssd_bwd_chunk_kernel(const SsdPa
 // prefetched tiles stay in registers (run-time bounds spill them, and a reload
 // waits for every load in flight). Batch 4, seqlen 2048, 80 heads with z, forward
 // and backward, these products against the float32 ones below: P 64, N 128 K3
-// alone 462 against 971 us, 64 x 64 750 against 1073,
-// 32 x 128 745 against 1161, 32 x 64 577 against 833.
+// alone 485 against 971 us; the whole call at 64 x 64 724 against 1073,
+// 32 x 128 715 against 1161, 32 x 64 541 against 833.
 constexpr int kLdT = kSsdMaxN + 16;   // rows of B and C here, read mostly transposed: eight rows on 64 banks
 
 // The small arrays first: with them last, beyond an LDS instruction's own 64 KB

@@ -130,6 +130,11 @@ def mamba_chunk_scan_combined(x, dt, A, B, C, chunk_size, D=None, z=None, dt_bia
     nseqs + 1 offsets of the packed sequences, seq_idx marking the same
     sequences): the state after each sequence's last step, zeros for an empty
     sequence, without gradient.
+
+    Every product has float32's accuracy in any storage type, for operands
+    (inputs, states and gradients) above about 8e-34 in magnitude; below, each is
+    off by at most 2**-134. Infinities and values up to float32's largest give
+    what float32 products give.
     """
     if x.device.type != "cuda":
         raise ValueError(f"mamba_cpu (MI355X build) runs on ROCm GPU tensors, got device {x.device}")
