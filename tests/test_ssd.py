@@ -493,3 +493,37 @@ def test_parameters_may_start_at_any_element(dtype, headdim, dstate):
     assert torch.equal(out, out1) and torch.equal(fin, fin1)
     for k, v in g.items():
         assert (v is None and g1[k] is None) or torch.equal(v, g1[k]), k
+
+
+@pytest.mark.parametrize("headdim,dstate", [(64, 128), (32, 64), (48, 80)])
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("chunk_pass", [1, 2], ids=["two-launch", "in-order"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_an_infinite_input_leaves_the_rest_of_its_workgroup(headdim, dstate, packed, chunk_pass, dtype):
+    """The last x of one head infinite, four heads to a workgroup: that workgroup does
+    its work again in float32, and whatever the value does not enter (the other
+    heads' outputs and gradients, its own head's earlier outputs) is the oracle's
+    for a finite x, within the bounds of the storage type."""
+    seqlen, low = 200, dtype != torch.float32
+    rng = np.random.default_rng(headdim)
+    seq = np.sort(rng.integers(0, 4, (1, seqlen)), axis=1).astype(np.int32) if packed else None
+    c = case(1, seqlen, 4, headdim, 1, dstate, seed=headdim, init=True, dtype=dtype)
+    bad = dict(c, x=c["x"].clone())
+    bad["x"][0, -1, 1, 5] = float("inf")
+    out, fin, g, W, V = run_ops(bad, head_block=4, chunk_pass=chunk_pass, seq=seq)
+    want, want_fin = S.ssd_fwd(**c, dt_softplus=True, seq_idx=seq)
+    wg = dict(zip(NAMES, S.ssd_bwd(**c, dt_softplus=True, seq_idx=seq, dout=W.float(), dfinal_states=V)))
+    tol = (2e-2, 2e-2) if low else (1e-4, 1e-5)
+    assert not torch.isfinite(out[0, -1, 1, 5]) and torch.isinf(fin[0, 1, 5]).all()
+    out, fin = out.float().cpu().numpy(), fin.float().cpu().numpy()
+    out[0, -1, 1, 5], fin[0, 1, 5] = want[0, -1, 1, 5], want_fin[0, 1, 5]
+    assert_close_report(out, want, *tol, "out")
+    assert_close_report(fin, want_fin, *tol, "final_states")
+    rest = [0, 2, 3]
+    for name in ("x", "dt", "z"):
+        got = dict(zip(NAMES, g))[name].float().cpu().numpy()[:, :, rest]
+        assert_close_report(got, wg[name][:, :, rest], *((2e-2, 2e-2) if low else (1e-3, 1e-4)), f"d{name}")
+    for name, atol in (("A", 1e-3), ("D", 1e-3), ("dt_bias", 1e-3), ("initial_states", 1e-3)):
+        got, ref = dict(zip(NAMES, g))[name].float().cpu().numpy(), wg[name]
+        got, ref = (got[:, rest], ref[:, rest]) if name == "initial_states" else (got[rest], ref[rest])
+        assert_close_report(got, ref, *((2e-2, 2e-2) if low else (1e-3, atol)), f"d{name}")
