@@ -342,7 +342,11 @@ int mcpu_selective_state_update_bc(const mcpu_state_update_args* a, int32_t bc_d
  * of 16 up to 128. The forward fills a caller-owned "saved" buffer of
  * mcpu_ssd_saved_size() bytes (per-chunk decays and states) that the backward
  * reads; the chunking is internal (64 steps) and does not change the result
- * beyond float32 rounding. */
+ * beyond float32 rounding. Outputs may take the place of inputs of the same
+ * type and shape (out that of x or z, final_states that of initial_states, dx
+ * and dz that of dout, x, z or ysave, ddt that of dt, dinitial_states that of
+ * dfinal_states). With out, ysave, dx, dz or ddt so placed, a chunk that an
+ * infinite value enters may hold NaN where separate buffers hold infinities. */
 typedef struct mcpu_ssd_args {
   const void* x;                /* (batch, seqlen, nheads, headdim), dtype */
   const float* dt;              /* (batch, seqlen, nheads), before dt_bias and softplus */

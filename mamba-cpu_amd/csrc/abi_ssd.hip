@@ -1,8 +1,10 @@
 // C-ABI entry points of the Mamba-2 SSD scan: argument checks, the layout of
 // the saved buffer and of the backward's workspace, and kernel sequencing.
 // Nothing is allocated here.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <initializer_list>
 
 #include "abi_util.h"
 #include "scan_common.h"
@@ -169,6 +171,12 @@ void bind_saved(SsdParams& p, const void* saved) {
   p.states = reinterpret_cast<float*>(s + w.states);
 }
 
+// Whether an output takes the place of one of the inputs. (Buffers that overlap in
+// any other way race between workgroups.)
+bool over(const void* out, std::initializer_list<const void*> inputs) {
+  return out != nullptr && std::find(inputs.begin(), inputs.end(), out) != inputs.end();
+}
+
 }  // namespace
 }  // namespace mcpu
 
@@ -207,6 +215,7 @@ extern "C" int mcpu_ssd_fwd(const mcpu_ssd_args* a, void* saved, size_t saved_by
   p.out = a->out;
   p.final_states = a->final_states;
   p.ysave = a->ysave;
+  p.apart = !over(a->out, {a->x, a->z}) && !over(a->ysave, {a->x, a->z});
   return hip_status(ssd_fwd_launch(p, a->dtype, static_cast<hipStream_t>(stream)), "ssd_fwd launch");
 }
 
@@ -292,6 +301,8 @@ extern "C" int mcpu_ssd_bwd(const mcpu_ssd_args* a, const void* saved, size_t sa
   p.ddt = a->ddt;
   p.dz = a->dz;
   p.dinit = a->dinitial_states;
+  p.apart = !over(a->dx, {a->x, a->z, a->dout, a->ysave}) && !over(a->dz, {a->x, a->z, a->dout, a->ysave}) &&
+            !over(a->ddt, {a->dt});
   p.dstates = reinterpret_cast<float*>(ws + w.dstates);
   p.dB_part = reinterpret_cast<float*>(ws + w.dB);
   p.dC_part = reinterpret_cast<float*>(ws + w.dC);

@@ -639,9 +639,12 @@ __device__ __forceinline__ float state_pass(const SsdParams& p, StateLds<Tx>& ld
   int64_t pend = -1;        // chunk whose dcsL share awaits the cross-wave sum
   float pend_decay = 0.f;
   zero(acc);
-  const float* init = BWD ? p.dfinal : p.init;
+  // The state the walk starts from. The second pass reads it back from where the first
+  // put it, element by element in the same threads: the first has also written the
+  // walk's end, which may lie over it.
+  const float* init = F32 ? (BWD ? p.dstates : p.states) : BWD ? p.dfinal : p.init;
   if (WALK && init != nullptr) {
-    const float* src = init + (b * H + h) * P * N;
+    const float* src = init + (F32 ? state_block(p, b, chunk_at(0), h) : (b * H + h) * P * N);
 #pragma unroll
     for (int j = 0; j < NT; ++j)
 #pragma unroll
@@ -1026,7 +1029,7 @@ __global__ void __launch_bounds__(kThreads3, 4) ssd_chunk_scan_kernel(const SsdP
       }
     }
   }
-  if (__builtin_expect(__syncthreads_or(spoilt != 0.f), 0)) chunk_scan_plain<Tx, HAS_Z, SEQ>(p, lds);
+  if (__builtin_expect(__syncthreads_or(spoilt != 0.f), 0) && p.apart) chunk_scan_plain<Tx, HAS_Z, SEQ>(p, lds);
 }
 
 // K2: walks the chunks from the last: dH^out_c (gradient of the state leaving
@@ -1922,7 +1925,7 @@ __global__ void __launch_bounds__(kThreads3, 2) ssd_bwd_chunk_bf16_kernel(const 
   float spoilt;
   if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) < 4) spoilt = bwd_chunk_waves<HAS_Z, SEQ, P, N, true>(p, lds);
   else spoilt = bwd_chunk_waves<HAS_Z, SEQ, P, N, false>(p, lds);
-  if (__builtin_expect(__syncthreads_or(spoilt != 0.f), 0))
+  if (__builtin_expect(__syncthreads_or(spoilt != 0.f), 0) && p.apart)
     bwd_chunk_f32<bf16, HAS_Z, SEQ, false>(p, shared.f32);
 }
 

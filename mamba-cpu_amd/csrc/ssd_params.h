@@ -64,6 +64,8 @@ struct SsdParams {
   int hb, nhb;              // heads per block, blocks over the heads
   int in_order;             // chunk states carried by the in-order kernels (one launch per
                             // direction, no chunk-end states stored) instead of two launches
+  int apart;                // no output lies over an input of the same kernel, which may then read
+                            // its inputs a second time
   int softplus;
   float dt_lo, dt_hi;       // the step is clamped to [dt_lo, dt_hi]
 };

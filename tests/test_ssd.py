@@ -527,3 +527,67 @@ def test_an_infinite_input_leaves_the_rest_of_its_workgroup(headdim, dstate, pac
         got, ref = dict(zip(NAMES, g))[name].float().cpu().numpy(), wg[name]
         got, ref = (got[:, rest], ref[:, rest]) if name == "initial_states" else (got[rest], ref[rest])
         assert_close_report(got, ref, *((2e-2, 2e-2) if low else (1e-3, atol)), f"d{name}")
+
+
+@pytest.mark.parametrize("headdim,dstate", [(64, 128), (48, 80)])
+@pytest.mark.parametrize("chunk_pass", [1, 2], ids=["two-launch", "in-order"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_outputs_over_inputs_with_an_infinite_value(headdim, dstate, chunk_pass, dtype):
+    """The C calls with every output over the input of its shape (out over x, the
+    final states over the initial ones, dx over dout, dz over z, ddt over dt, dinit
+    over dfinal), one x infinite, four heads to a workgroup: the other heads'
+    results are those of separate buffers, and no workgroup does its work twice on
+    what it has written. Bound: the storage type's, as the workgroups that do their
+    work again add up in another order."""
+    import ctypes
+
+    from mamba_cpu import _C
+
+    shape = (1, 200, 4, headdim, 1, dstate)
+    low = dtype != torch.float32
+    c = case(*shape, seed=headdim, init=True, dtype=dtype, z=True)
+    c["x"][0, -1, 1, 5] = float("inf")
+    gen = torch.Generator().manual_seed(1)
+    W = torch.randn(c["x"].shape, generator=gen).to(dtype)
+    V = torch.randn(c["initial_states"].shape, generator=gen)
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def call(over):
+        d = {k: v.to(DEV).contiguous() for k, v in c.items()}
+        dout, dfin = W.to(DEV), V.to(DEV)
+        a = _C.SsdArgs()
+        for n in NAMES:
+            setattr(a, n, d[n].data_ptr())
+        a.batch, a.seqlen, a.nheads, a.headdim, a.ngroups, a.dstate = shape
+        a.dtype = _C.MCPU_BF16 if low else _C.MCPU_F32
+        a.dt_softplus, a.dt_limit_hi, a.head_block, a.chunk_pass = 1, float("inf"), 4, chunk_pass
+        place = lambda t: t if over else torch.empty_like(t)  # noqa: E731
+        saved = torch.empty(_C.lib.mcpu_ssd_saved_size(ctypes.byref(a)), dtype=torch.uint8, device=DEV)
+        out, fin, y = place(d["x"]), place(d["initial_states"]), torch.empty_like(d["x"])
+        a.out, a.final_states, a.ysave = out.data_ptr(), fin.data_ptr(), y.data_ptr()
+        assert _C.lib.mcpu_ssd_fwd(ctypes.byref(a), saved.data_ptr(), saved.numel(), stream) == _C.MCPU_OK
+        res = {"out": out.clone(), "final_states": fin.clone()}
+        d["x"].copy_(c["x"])
+        d["initial_states"].copy_(c["initial_states"])
+        f32 = dict(dtype=torch.float32, device=DEV)
+        g = {"dx": place(dout), "ddt": place(d["dt"]), "dz": place(d["z"]), "dinitial_states": place(dfin)}
+        rest = {"dA": torch.empty(4, **f32), "dB": torch.empty(d["B"].shape, **f32),
+                "dC": torch.empty(d["C"].shape, **f32), "dD": torch.empty(4, headdim, **f32),
+                "ddt_bias": torch.empty(4, **f32)}
+        a.dout, a.dfinal_states = dout.data_ptr(), dfin.data_ptr()
+        for n, t in {**g, **rest}.items():
+            setattr(a, n, t.data_ptr())
+        ws = torch.empty(_C.lib.mcpu_ssd_bwd_workspace_size(ctypes.byref(a)), dtype=torch.uint8, device=DEV)
+        assert _C.lib.mcpu_ssd_bwd(ctypes.byref(a), saved.data_ptr(), saved.numel(), ws.data_ptr(), ws.numel(),
+                                   stream) == _C.MCPU_OK
+        torch.cuda.synchronize()
+        return {**res, **g}
+
+    want, got = call(False), call(True)
+    assert torch.isinf(want["final_states"][0, 1, 5]).all() and torch.isinf(got["final_states"][0, 1, 5]).all()
+    rest = [0, 2, 3]
+    for name, w in want.items():
+        heads = (lambda t: t[:, rest]) if "states" in name else (lambda t: t[:, :, rest])
+        assert torch.isfinite(heads(w)).all(), name
+        assert_close_report(heads(got[name]).float(), heads(w).float().cpu().numpy(),
+                            *((2e-2, 2e-2) if low else (1e-3, 1e-4)), name)
