@@ -12,12 +12,13 @@
 //     moving VPL vectors of four neighbouring states. The fewer lanes to a row,
 //     the more rows to a wave for what is done once per row; 4 lanes up to 64
 //     states (64 states 37 us, 8 lanes 39, 16 lanes 52; 32 states 17 against 23),
-//     8 for 128 (70 us; 16 lanes 75; 4 lanes 74, of 222 registers), 16 for 256,
-//     for their registers. Vectors need no more than their element's alignment,
-//     so any base and strides run here.
+//     8 for 128 (70 us; 16 lanes 75; 4 lanes 74, of 222 registers), 16 for 256
+//     (120 us, 117 of them without chains_sum's order; 8 lanes 135, for their
+//     registers). Vectors need no more than their element's alignment, so any
+//     base and strides run here.
 //     (64, 80, 64, 128) float32 states with bf16 x, B and C: 70 us, 4.8 TB/s,
 //     against 90 us with one state per lane and load and B and C cast to
-//     float32 by two launches; (64, 5120, 16): 13.7 against 40.8 us.
+//     float32 by two launches; (64, 5120, 16): 12.8 against 40.8 us.
 //   - any other dstate: 16 lanes per row, lane j owning states j, j + 16, ...
 // Both run row tiles of the (nheads, headdim) rows x batch, so the row decode is
 // one 32-bit division. B and C are float32 or of x's type (Tb).
