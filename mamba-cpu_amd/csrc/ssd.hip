@@ -772,34 +772,57 @@ template <typename Tx> struct ScanLds {
   __align__(16) uint16_t H[3 * kPlaneN];             // B (Q x N), then each head's entering state H (P x N), then Y
 };
 
-// The same outputs one element at a time in plain float32, for a block whose products
-// in pieces left one that is not finite. C B^T and G pass through LDS over H; what
-// bounds it does not matter.
+// The same outputs in float32, for a block whose products in pieces left one that is
+// not finite. C B^T and C H^T, whose terms all belong to their element, run on the
+// float32 matrix unit with operands straight from memory; G x adds the steps that an
+// output has, and no others (0 times an infinite x is NaN), a lane's four rows per x.
+// C B^T and G pass through LDS over H. Batch 4, seqlen 2048, 80 heads, bf16 with z, x
+// all NaN: the forward takes 1.8 ms (11.4 one element at a time; 0.33 with finite x).
 template <typename Tx, bool HAS_Z, bool SEQ>
 __device__ __forceinline__ void chunk_scan_plain(const SsdParams& p, ScanLds<Tx>& lds) {
   constexpr int TPB = kThreads3;
   float* const s_CB = reinterpret_cast<float*>(lds.H);   // rows t of QP floats
   float* const s_G = s_CB + Q * QP;
   static_assert(2 * Q * QP * 4 <= sizeof(lds.H), "C B^T and G fit over H");
-  const int tid = second_tid();
+  const int tid = second_tid(), lane = tid & 63, wave = tid >> 6;
+  const int ws = wave & 3, hf = wave >> 2;        // row strip, tiles 2 hf and 2 hf + 1 of 16 columns
+  const int r = lane & 15, q = lane >> 4;
   const int64_t c = blockIdx.x, b = blockIdx.z;
   const int64_t L = p.seqlen, H = p.nheads, P = p.headdim, N = p.dstate, G = p.ngroups;
   const int64_t h0 = static_cast<int64_t>(blockIdx.y) * p.hb;
   const int64_t t0 = c * Q, bcoff = ((b * L + t0) * G + h0 / (H / G)) * N;
   const int nvalid = chunk_steps(p, t0);
   const bool enter = seq_of<SEQ>(p, b, t0) == seq_of<SEQ>(p, b, t0 - 1);
-  auto first = [&](int t) { return SEQ ? lds.first[t] : 0; };
-  for (int i = tid; i < Q * Q; i += TPB) {
-    const int t = i / Q, u = i % Q;
-    float v = 0.f;
-    if (u <= t && t < nvalid)
-      for (int64_t n = 0; n < N; ++n)
-        v = fmaf(ld<Tx>(p.C, bcoff + t * G * N + n), ld<Tx>(p.B, bcoff + u * G * N + n), v);
-    s_CB[t * QP + u] = v;
+  // Rows and columns that do not exist repeat the last one and are not stored.
+  const int64_t crow = bcoff + static_cast<int64_t>(min(16 * ws + r, nvalid - 1)) * G * N + q;
+  int col[2], first[4];
+  v4f acc[2];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) first[e] = SEQ ? lds.first[16 * ws + 4 * q + e] : 0;
+  int64_t brow[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int u = 32 * hf + 16 * j + r;
+    col[j] = min(u, static_cast<int>(P) - 1);
+    brow[j] = bcoff + static_cast<int64_t>(min(u, nvalid - 1)) * G * N + q;
+    acc[j] = v4f{0.f, 0.f, 0.f, 0.f};
   }
+  int64_t n = 0;
+  do {   // dstate is at least 16
+    const float a = ld<Tx>(p.C, crow + n);
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+      acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, ld<Tx>(p.B, brow[j] + n), acc[j], 0, 0, 0);
+    n += 4;
+  } while (n < N);
+  mma_wait(acc);
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) s_CB[(16 * ws + 4 * q + e) * QP + 32 * hf + 16 * j + r] = acc[j][e];
   for (int64_t h = h0; h < h0 + p.hb; ++h) {
     const int64_t row = chunk_row(p, b, h, c), xoff = ((b * L + t0) * H + h) * P;
-    const float* st = p.states + state_block(p, b, c, h);
+    const float* st = p.states + state_block(p, b, c, h) + q;
     __syncthreads();  // C B^T is there, and every thread is done with the previous head's G
     if (tid < Q) {
       lds.cs[tid] = p.cs[row + tid];
@@ -809,27 +832,54 @@ __device__ __forceinline__ void chunk_scan_plain(const SsdParams& p, ScanLds<Tx>
     __syncthreads();
     for (int i = tid; i < Q * Q; i += TPB) {
       const int t = i / Q, u = i % Q;
-      s_G[t * QP + u] =
-          u <= t && u >= first(t) ? s_CB[t * QP + u] * seg_exp(lds.cs, lds.csl, t, u) * lds.dt[u] : 0.f;
+      s_G[t * QP + u] = u <= t ? s_CB[t * QP + u] * seg_exp(lds.cs, lds.csl, t, u) * lds.dt[u] : 0.f;
     }
     __syncthreads();
-    for (int i = tid; i < nvalid * static_cast<int>(P); i += TPB) {
-      const int t = i / static_cast<int>(P), pp = i % static_cast<int>(P);
-      float y = 0.f;
-      if (enter && first(t) == 0) {
-        for (int64_t n = 0; n < N; ++n) y = fmaf(ld<Tx>(p.C, bcoff + t * G * N + n), st[pp * N + n], y);
-        y *= fast_exp(lds.cs[t] + lds.csl[t]);
-      }
-      for (int u = first(t); u <= t; ++u) y = fmaf(s_G[t * QP + u], ld<Tx>(p.x, xoff + u * H * P + pp), y);
-      const int64_t at = xoff + t * H * P + pp;
-      if (p.D) y = fmaf(p.D[h * P + pp], ld<Tx>(p.x, at), y);
-      if (HAS_Z) {
-        if (p.ysave) mcpu::st<Tx>(p.ysave, at, y);
-        const float z = ld<Tx>(p.z, at);
-        y *= z * sigmoid(z);
-      }
-      mcpu::st<Tx>(p.out, at, y);
+    acc[0] = acc[1] = v4f{0.f, 0.f, 0.f, 0.f};
+    n = 0;
+    do {
+      const float a = ld<Tx>(p.C, crow + n);
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, st[col[j] * N + n], acc[j], 0, 0, 0);
+      n += 4;
+    } while (n < N);
+    mma_wait(acc);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int te = 16 * ws + 4 * q + e;
+      const float ecs = fast_exp(lds.cs[te] + lds.csl[te]);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) acc[j][e] = enter && first[e] == 0 ? acc[j][e] * ecs : 0.f;
     }
+    for (int s = 0; s < min(16 * ws + 16, nvalid); ++s) {
+      float x[2];
+#pragma unroll
+      for (int j = 0; j < 2; ++j) x[j] = ld<Tx>(p.x, xoff + s * H * P + col[j]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int te = 16 * ws + 4 * q + e;
+        const float g = s_G[te * QP + s];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[j][e] = s <= te && s >= first[e] ? fmaf(g, x[j], acc[j][e]) : acc[j][e];
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int te = 16 * ws + 4 * q + e, pp = 32 * hf + 16 * j + r;
+        if (te >= nvalid || pp >= P) continue;
+        const int64_t at = xoff + te * H * P + pp;
+        float y = acc[j][e];
+        if (p.D) y = fmaf(p.D[h * P + pp], ld<Tx>(p.x, at), y);
+        if (HAS_Z) {
+          if (p.ysave) mcpu::st<Tx>(p.ysave, at, y);
+          const float z = ld<Tx>(p.z, at);
+          y *= z * sigmoid(z);
+        }
+        mcpu::st<Tx>(p.out, at, y);
+      }
   }
 }
 

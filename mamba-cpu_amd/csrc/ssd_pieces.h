@@ -120,8 +120,9 @@ __device__ __forceinline__ v4f mma32(const Frag<NA>& a, const Frag<NB>& b, v4f c
 // where the products sit under conditions it counts along the longest way to their
 // use, and a tile whose successors were skipped would be read before it is written.
 template <int NT> __device__ __forceinline__ void mma_wait(v4f (&acc)[NT]) {
-  static_assert(NT == 4, "tiles");
-  asm volatile("s_nop 15" : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]));
+  static_assert(NT == 4 || NT == 2, "tiles");
+  if constexpr (NT == 4) asm volatile("s_nop 15" : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]));
+  else asm volatile("s_nop 15" : "+v"(acc[0]), "+v"(acc[1]));
 }
 
 // sum + 0 v: no longer 0 once a v was not finite.
