@@ -605,6 +605,9 @@ def ssd_workloads(torch, dev, stream, cpu):
                 "achieved_fwd": round(tf_f, 2), "frac_fwd": round(tf_f / MFMA_F32_PEAK_TFS, 4),
                 "achieved": round(tf_fb, 2), "frac": round(tf_fb / MFMA_F32_PEAK_TFS, 4),
                 "matrix_flops": {"fwd": int(ff), "fwd_bwd": int(fbf)},
+                "note": "peak is that of float32 products; the kernels form float32-accurate products of bf16 "
+                        "pieces (but for the float32 chunk gradients), and their traffic, chunk states "
+                        "included, takes more of the time than the matrix cores do",
                 "hbm_GBps": round(fb_bytes / (fb_ms * 1e-3) / 1e9, 1),
                 "hbm_frac": round(fb_bytes / (fb_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
                 "algorithmic_bytes_fwd_bwd": int(fb_bytes),
